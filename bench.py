@@ -101,8 +101,8 @@ KERNEL_KEYS = [
     ("cwa::b2d::k2_density<", "batched", "density"), ("cwa::b2d::k2_force<", "batched", "force"),
     ("cwa::b2d::k2_hash(", "batched", "hash"), ("cwa::b2d::k2_scatter(", "batched", "scatter"),
     ("cwa::b2d::k2_reorder(", "batched", "reorder"), ("cwa::b2d::k2_wave(", "batched", "wave"),
-    ("cwa::k_density(", "plain", "density"), ("cwa::k_force_integrate(", "plain", "force_integrate"),
-    ("cwa::k_hash_count(", "plain", "hash"), ("cwa::k_scatter_runs(", "plain", "scatter"),
+    ("cwa::k_density(", "plain", "density"), ("cwa::k_force_integrate<", "plain", "force_integrate"),
+    ("cwa::k_hash_count<", "plain", "hash"), ("cwa::k_link_runs(", "plain", "scatter"),
     ("cwa::k_stable_reorder(", "plain", "reorder"), ("cwa::k_wave4(", "plain", "wave"),
 ]
 

@@ -5,13 +5,13 @@
 //   particles  SoA float4 pos / vel / force + int id, in cell-sorted order;
 //              two copies (A = state, B = this step's reorder target)
 //   work       rho_w (float), pw (float2: pressure, 1/rho), flux (float)
-//   grid       key, trank (int per particle), count (int per cell),
-//              offset (int per cell + 1), tmp / list (int per particle)
+//   grid       key (int per particle), count and head (int per cell), link
+//              (int2 per run), offset (int per cell + 1), list (int per particle)
 //   wave       three W*H fp32 fields (newest, previous, write)
 //
 // Reference kernels replaced (paths relative to the reference root):
 //   ugrid_particles_cs.glsl (hash / count / insert)  -> k_hash_count,
-//       k_scatter_tmp, k_stable_reorder
+//       k_stable_reorder
 //   prefix_sum_cs.glsl + ParallelScan.cpp            -> k_scan_*
 //   rho_pres_comp.glsl                               -> k_density
 //   force_comp.glsl + integrate_comp.glsl            -> k_force_integrate
@@ -38,6 +38,19 @@ long long set_lane_split_limit(long long max_n) { return g_lane_split.exchange(m
 __global__ void k_fill_i32(int* __restrict__ p, int n, int v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+}
+
+// Zeroes up to five int arrays of n (the first: n + 1) in one launch.
+struct ClearList {
+    int* p[5];
+};
+__global__ void __launch_bounds__(256) k_clear_cells(ClearList l, int n) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0 && l.p[0]) l.p[0][n] = 0;
+    if (i >= n) return;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        if (l.p[k]) l.p[k][i] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -126,7 +139,8 @@ __device__ __forceinline__ int block_excl_scan(int v, int& total) {
 __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int* __restrict__ in, int n,
                                                              const int* __restrict__ tile_prefix,
                                                              int* __restrict__ out,
-                                                             int* __restrict__ zero_out) {
+                                                             int* __restrict__ zero_out,
+                                                             int* __restrict__ zero_out2) {
     const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
     int v[kScanItems];
     load_items(in, base, n, v);
@@ -142,10 +156,9 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int* __restri
         run += v[k];
     }
     store_items(out, base, n, o);
-    if (zero_out) {
-        const int z[kScanItems] = {0, 0, 0, 0, 0, 0, 0, 0};
-        store_items(zero_out, base, n, z);
-    }
+    const int z[kScanItems] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (zero_out) store_items(zero_out, base, n, z);
+    if (zero_out2) store_items(zero_out2, base, n, z);
 }
 
 __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int* __restrict__ in, int n,
@@ -170,13 +183,15 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int* __restr
 // Exclusive scan of one tile per block.  The tile's prefix is the sum of
 // the tile sums before it (part[0 .. blockIdx.x), summed by the block
 // itself; null part: single tile).  total_out (optional) receives the grand
-// total, written by the last block.  zero_out (optional) is cleared over
-// the same index range (the other half of a double-buffered counter).
+// total, written by the last block.  zero_out and zero_out2 (optional) are
+// cleared over the same index range (the other halves of the double-buffered
+// cell counters and run-list heads).
 __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int* __restrict__ in, int n,
                                                             const int* __restrict__ part,
                                                             int* __restrict__ out,
                                                             int* __restrict__ total_out,
-                                                            int* __restrict__ zero_out) {
+                                                            int* __restrict__ zero_out,
+                                                            int* __restrict__ zero_out2) {
     int prefix = 0;
     if (part) {
         int s = 0;
@@ -200,10 +215,9 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int* __restric
         run += v[k];
     }
     store_items(out, base, n, o);
-    if (zero_out) {
-        const int z[kScanItems] = {0, 0, 0, 0, 0, 0, 0, 0};
-        store_items(zero_out, base, n, z);
-    }
+    const int z[kScanItems] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (zero_out) store_items(zero_out, base, n, z);
+    if (zero_out2) store_items(zero_out2, base, n, z);
     if (total_out && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *total_out = total + prefix;
 }
 
@@ -228,26 +242,29 @@ size_t scan_workspace_ints(int n) {
 // Up to kScanDirectTiles tiles the tile prefixes are summed inside
 // k_scan_down (two launches); larger inputs recurse on the tile sums.
 hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
-                       int* zero_out) {
+                       int* zero_out, int* zero_out2) {
     if (n <= 0) {
         k_fill_i32<<<1, 64, 0, st>>>(out, 1, 0);
         return hipGetLastError();
     }
     const int tiles = (n + kScanTile - 1) / kScanTile;
     if (tiles == 1) {
-        k_scan_down<<<1, kScanThreads, 0, st>>>(in, n, nullptr, out, out + n, zero_out);
+        k_scan_down<<<1, kScanThreads, 0, st>>>(in, n, nullptr, out, out + n, zero_out,
+                                                    zero_out2);
         return hipGetLastError();
     }
     int* part = ws;
     k_scan_reduce<<<tiles, kScanThreads, 0, st>>>(in, n, part);
     if (tiles <= kScanDirectTiles) {
-        k_scan_down<<<tiles, kScanThreads, 0, st>>>(in, n, part, out, out + n, zero_out);
+        k_scan_down<<<tiles, kScanThreads, 0, st>>>(in, n, part, out, out + n, zero_out,
+                                                    zero_out2);
         return hipGetLastError();
     }
     int* part_ex = ws + tiles;  // tiles + 1 entries
-    hipError_t e = launch_scan(part, part_ex, tiles, ws + 2 * (size_t)tiles + 1, st, nullptr);
+    hipError_t e = launch_scan(part, part_ex, tiles, ws + 2 * (size_t)tiles + 1, st, nullptr,
+                               nullptr);
     if (e != hipSuccess) return e;
-    k_scan_apply<<<tiles, kScanThreads, 0, st>>>(in, n, part_ex, out, zero_out);
+    k_scan_apply<<<tiles, kScanThreads, 0, st>>>(in, n, part_ex, out, zero_out, zero_out2);
     k_scan_total<<<1, 64, 0, st>>>(part_ex + tiles, out + n);
     return hipGetLastError();
 }
@@ -259,32 +276,41 @@ hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
 // deterministic) with the UniformGrid2D::Build order (UniformGrid2D.cpp:
 // 75-91: items ascending within each cell):
 //   count    one atomicAdd per run of equal keys in a wave (lane order),
-//            issued by the run's first lane, its result unused (the wave
-//            does not wait for it)
+//            issued by the run's first lane, its result unused.  The same lane
+//            pushes the run on its cell's run list: head[c] (first item + 1 of
+//            the newest run, 0 for an empty list) is exchanged, and link[first
+//            item] records (the older head, the run's length)
 //   scan     exclusive scan of the counts -> offsets
-//   scatter  each run head takes a provisional place in its cell's segment
-//            from a fill counter and writes (first item, length) there; the
-//            runs tile the segment
-//   reorder  the run head walks its cell's run records (one per run, not one
+//   reorder  the run head walks its cell's run list (one link per run, not one
 //            per item) and counts the items of the runs that start before
 //            its own; the lanes of the run take that rank plus their
 //            distance to the head.  The particle positions and ids move to
-//            their sorted slots in the same pass, which also clears the
-//            fill counters for the next build.
+//            their sorted slots in the same pass.
 // The wave layout (blocks of 256 over the same item range) is identical in
-// the three item passes, so every pass sees the same runs.
+// both item passes, so both see the same runs.  The lists need no offsets, so
+// whoever counts the keys can also list the runs; builds of up to
+// kFuseLinksMax particles do.  In larger ones k_link_runs lists them
+// (kFuseLinksMax gives both sides' times).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void count_runs(int c, bool valid, int* __restrict__ count) {
+template <bool kCount, bool kLink>
+__device__ __forceinline__ void push_runs(int c, bool valid, int i, const CellRuns& r) {
     const int lane = threadIdx.x & 63;
-    const RunInfo r = wave_runs(c);
-    if (r.head && valid) atomicAdd(&count[c], r.run_end - lane);
+    const RunInfo w = wave_runs(c);
+    if (w.head && valid) {
+        const int len = w.run_end - lane;
+        int older = 0;
+        if (kLink) older = atomicExch(&r.head[c], i + 1);
+        if (kCount) atomicAdd(&r.count[c], len);
+        if (kLink) r.link[i] = make_int2(older, len);
+    }
 }
 
 // Cell hash + count of particle slots (ComputeCellIndex / Index / ComputeCounts,
 // ugrid_particles_cs.glsl:90-108, with the y-fastest linearisation).
+template <bool kLink>
 __global__ void __launch_bounds__(256) k_hash_count(const float4* __restrict__ pos, int n,
                                                     GridDesc g, int* __restrict__ key,
-                                                    int* __restrict__ count) {
+                                                    CellRuns runs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
     int c = -1;
@@ -296,63 +322,55 @@ __global__ void __launch_bounds__(256) k_hash_count(const float4* __restrict__ p
         c = lin_cell(g.dims, ix, iy, iz);
         key[i] = c;
     }
-    count_runs(c, valid, count);
+    push_runs<true, kLink>(c, valid, i, runs);
 }
 
-// Count of items whose keys are already known.
+// Count and runs of items whose keys are already known.
 __global__ void __launch_bounds__(256) k_key_count(const int* __restrict__ key, int n,
-                                                   int* __restrict__ count) {
+                                                   CellRuns runs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
-    count_runs(valid ? key[i] : -1, valid, count);
+    push_runs<true, true>(valid ? key[i] : -1, valid, i, runs);
 }
 
-// Run records: (first item, length) at a provisional place in the cell's
-// segment (fill: zero on entry).
-__global__ void __launch_bounds__(256) k_scatter_runs(const int* __restrict__ key,
-                                                      const int* __restrict__ offset,
-                                                      int* __restrict__ fill, int n,
-                                                      int2* __restrict__ runs) {
+// Runs of items that are already counted.
+__global__ void __launch_bounds__(256) k_link_runs(const int* __restrict__ key, int n,
+                                                   int* __restrict__ head,
+                                                   int2* __restrict__ link) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
     const bool valid = i < n;
-    const int c = valid ? key[i] : -1;
-    const RunInfo r = wave_runs(c);
-    if (valid && r.head) {
-        const int len = r.run_end - lane;
-        runs[offset[c] + atomicAdd(&fill[c], len)] = make_int2(i, len);
-    }
+    push_runs<false, true>(valid ? key[i] : -1, valid, i, CellRuns{nullptr, head, link});
 }
 
 // Stable destination of every item; list[d] = item_of[item] (or the item
 // itself), and the particle positions and ids move to their sorted slots
 // when pos_out is set (the passes that follow read velocities and forces in
-// their pre-sort slots through list).  Threads below nfill clear fill.
+// their pre-sort slots through list).  The walk ends with the cell's count,
+// whatever the links hold.
 __global__ void __launch_bounds__(256) k_stable_reorder(
-    const int* __restrict__ key, const int* __restrict__ offset,
-    const int2* __restrict__ runs, int n, const int* __restrict__ item_of,
+    const int* __restrict__ key, const int* __restrict__ offset, const int* __restrict__ head,
+    const int2* __restrict__ link, int n, const int* __restrict__ item_of,
     int* __restrict__ list, const float4* __restrict__ pos_in,
-    const int* __restrict__ id_in, float4* __restrict__ pos_out, int* __restrict__ id_out,
-    int* __restrict__ fill, int nfill) {
+    const int* __restrict__ id_in, float4* __restrict__ pos_out, int* __restrict__ id_out) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    if (s < nfill) fill[s] = 0;
     const bool valid = s < n;
     const int c = valid ? key[s] : -1;
     const RunInfo r = wave_runs(c);
-    int rank = 0, b = 0;
+    int rank = 0;
     if (valid && r.head) {
-        b = offset[c];
-        const int e = offset[c + 1];
-        for (int p = b; p < e;) {
-            const int2 u = runs[p];
-            if (u.x < s) rank += u.y;
-            p += max(u.y, 1);
+        const int b = offset[c];
+        int left = offset[c + 1] - b;
+        for (int q = head[c]; q > 0 && left > 0;) {
+            const int2 u = link[q - 1];
+            if (q - 1 < s) rank += u.y;
+            left -= max(u.y, 1);
+            q = u.x;
         }
         rank += b;
     }
     const int d = __shfl(rank, r.my_head, 64) + (lane - r.my_head);
-    if (!valid || d < 0 || d >= n) return;  // out of range only on inconsistent run records
+    if (!valid || d < 0 || d >= n) return;  // out of range only on inconsistent run lists
     list[d] = item_of ? item_of[s] : s;
     if (pos_out) {
         // read once (nt): the previous force pass's output leaves the L2 to the
@@ -684,12 +702,13 @@ __device__ __forceinline__ void column_flux_sum(const int* __restrict__ offset,
 // velocity), its id from the sorted copy and its previous force from the
 // state in its pre-sort slot (list[i]); writes the next state in the sorted
 // slot order.  When `next` is set it also hashes the new position into the
-// next step's grid (cell key, run record and count, ComputeCounts of
+// next step's grid (cell key, count and run lists, ComputeCounts of
 // ugrid_particles_cs.glsl:90-95), so that step needs no hash pass of its own.
 // Blocks nfb.. of the grid sum the particle flux per column instead (one
 // wave per column; they read only the density pass's output and run in
 // the force blocks' tail).
 // ---------------------------------------------------------------------------
+template <bool kLink>
 __global__ void __launch_bounds__(256) k_force_integrate(
     const DevParams* __restrict__ Pd, float dt, const float4* __restrict__ bpos,
     const int* __restrict__ bid, const float* __restrict__ vpad,
@@ -850,7 +869,7 @@ __global__ void __launch_bounds__(256) k_force_integrate(
             next.key[i] = cell;
         }
     }  // valid
-    if (next.key) count_runs(cell, valid, next.count);
+    if (next.key) push_runs<true, kLink>(cell, valid, i, next.runs);
 }
 
 // ---------------------------------------------------------------------------
@@ -1042,35 +1061,43 @@ hipError_t launch_fill_i32(int* p, int n, int v, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* key, int* count,
-                             hipStream_t st) {
-    if (n <= 0) return hipSuccess;
-    k_hash_count<<<blocks_for(n, 256), 256, 0, st>>>(pos, n, g, key, count);
+hipError_t launch_clear_cells(int* offset, int* a, int* b, int* c, int* d, int n,
+                              hipStream_t st) {
+    if (n < 0) return hipErrorInvalidValue;
+    k_clear_cells<<<blocks_for(std::max(n, 1), 256), 256, 0, st>>>(ClearList{{offset, a, b, c, d}},
+                                                                   n);
     return hipGetLastError();
 }
 
-hipError_t launch_key_count(const int* key, int n, int* count, hipStream_t st) {
+hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* key,
+                             const CellRuns& runs, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    k_key_count<<<blocks_for(n, 256), 256, 0, st>>>(key, n, count);
+    if (runs.head)
+        k_hash_count<true><<<blocks_for(n, 256), 256, 0, st>>>(pos, n, g, key, runs);
+    else
+        k_hash_count<false><<<blocks_for(n, 256), 256, 0, st>>>(pos, n, g, key, runs);
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_runs(const int* key, const int* offset, int* fill, int n, int2* runs,
-                               hipStream_t st) {
+hipError_t launch_key_count(const int* key, int n, const CellRuns& runs, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    k_scatter_runs<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, fill, n, runs);
+    k_key_count<<<blocks_for(n, 256), 256, 0, st>>>(key, n, runs);
     return hipGetLastError();
 }
 
-hipError_t launch_stable_reorder(const int* key, const int* offset, const int2* runs, int n,
-                                 const int* item_of, int* list, const float4* pos_in,
-                                 const int* id_in, float4* pos_out, int* id_out, int* fill,
-                                 int nfill, hipStream_t st) {
-    const int m = std::max(n, nfill);
-    if (m <= 0) return hipSuccess;
-    k_stable_reorder<<<blocks_for(m, 256), 256, 0, st>>>(key, offset, runs, n, item_of, list,
-                                                         pos_in, id_in, pos_out, id_out, fill,
-                                                         nfill);
+hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    k_link_runs<<<blocks_for(n, 256), 256, 0, st>>>(key, n, head, link);
+    return hipGetLastError();
+}
+
+hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,
+                                 const int2* link, int n, const int* item_of, int* list,
+                                 const float4* pos_in, const int* id_in, float4* pos_out,
+                                 int* id_out, hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    k_stable_reorder<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, head, link, n, item_of, list,
+                                                         pos_in, id_in, pos_out, id_out);
     return hipGetLastError();
 }
 
@@ -1134,10 +1161,10 @@ hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bp
     const int nfb = blocks_for(n, 256);
     const long long ncol = colflux ? (long long)P.dims[0] * P.dims[2] : 0;
     const int ncb = blocks_for(ncol * 64, 256);
-    k_force_integrate<<<nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list,
-                                                 offset, n, rho_w, nbw, nrec, H0, N.pos, N.vel,
-                                                 N.force, N.id, rho, prs, fpre, nfb, flux,
-                                                 colflux, next);
+    const auto kernel = next.runs.head ? k_force_integrate<true> : k_force_integrate<false>;
+    kernel<<<nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list, offset, n, rho_w,
+                                      nbw, nrec, H0, N.pos, N.vel, N.force, N.id, rho, prs, fpre,
+                                      nfb, flux, colflux, next);
     return hipGetLastError();
 }
 

@@ -24,25 +24,41 @@ struct ParticleArrays {
 };
 
 size_t scan_workspace_ints(int n);
-// zero_out (optional, n ints) is cleared in the same pass.
+// zero_out and zero_out2 (optional, n ints each) are cleared in the same pass.
 hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
-                       int* zero_out = nullptr);
+                       int* zero_out = nullptr, int* zero_out2 = nullptr);
 hipError_t launch_fill_i32(int* p, int n, int v, hipStream_t st);
+// Zeroes offset[0..n] and a, b, c, d[0..n) (each may be null).
+hipError_t launch_clear_cells(int* offset, int* a, int* b, int* c, int* d, int n,
+                              hipStream_t st);
+// Where the items of a build are counted and their runs listed: count and head
+// per cell (both zero on entry), link per item.  With head null the hash and
+// force passes only count the items.
+struct CellRuns {
+    int* count;
+    int* head;
+    int2* link;
+};
 // Stable counting sort of keyed items: count (keys of particle positions, or
-// given keys) into a zeroed counter, scan, scatter of run records (runs: n
-// int2; fill: num_cells ints, zero on entry), reorder (clears fill[0 ..
-// nfill) for the next build).
-hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* key, int* count,
-                             hipStream_t st);
-hipError_t launch_key_count(const int* key, int n, int* count, hipStream_t st);
-hipError_t launch_scatter_runs(const int* key, const int* offset, int* fill, int n, int2* runs,
-                               hipStream_t st);
+// given keys) with the cells' run lists, scan, reorder.
+hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* key,
+                             const CellRuns& runs, hipStream_t st);
+hipError_t launch_key_count(const int* key, int n, const CellRuns& runs, hipStream_t st);
+hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStream_t st);
+// Builds of up to this many particles list their runs in the pass that counts
+// the keys, larger ones in a pass of their own: each run's push waits for its
+// exchange, at the end of waves that hold the force pass's LDS.  A launch less
+// pays where launches count (MI355X, step without the pass against with it,
+// three scenes in flight: 4 096 particles 17.7 / 18.3 us, 65 536 25.9 /
+// 27.2 us, 300 007 71.0 / 71.1 us, 1 048 576 285 / 276 us; the first step's
+// hash pass at 1 048 576 particles 51 / 32 us).
+constexpr int kFuseLinksMax = 1 << 18;
 // list[d] = item_of ? item_of[s] : s at each item's stable destination d;
 // with pos_out set, pos_out[d] = pos_in[s] and id_out[d] = id_in[s].
-hipError_t launch_stable_reorder(const int* key, const int* offset, const int2* runs, int n,
-                                 const int* item_of, int* list, const float4* pos_in,
-                                 const int* id_in, float4* pos_out, int* id_out, int* fill,
-                                 int nfill, hipStream_t st);
+hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,
+                                 const int2* link, int n, const int* item_of, int* list,
+                                 const float4* pos_in, const int* id_in, float4* pos_out,
+                                 int* id_out, hipStream_t st);
 // Boxes: cells covered per box (ncov, n ints), then the (box, cell) pairs at
 // first[i] = exclusive scan of ncov (pkey: cell, pbox: box index).
 hipError_t launch_box_cover(const float4* x, const float4* hw, int n, const float gmin[3],
@@ -71,11 +87,11 @@ hipError_t launch_density(const DevParams& P, const float4* bpos, const float4* 
                           const int* list, const int* offset, int n, const float* H0,
                           float* rho_w, float2* pw, float* flux, uint2* nbw, float4* nrec,
                           float* rho_raw, float4* vel_out, float* vpad, hipStream_t st);
-// Where the force pass hashes the next step's grid (key, count; the counter
-// zero on entry), or key == null for no fused hash.
+// Where the force pass hashes the next step's grid, or key == null for no
+// fused hash.
 struct NextKeys {
     int* key;
-    int* count;
+    CellRuns runs;
 };
 // Forces + integration: own record from nrec, id from bid and the velocity
 // pad from vpad (sorted), previous force from the state S in its pre-sort

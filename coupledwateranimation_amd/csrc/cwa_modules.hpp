@@ -131,7 +131,11 @@ class UniformGrid3D {
                    hipEvent_t* ev = nullptr, int* list_out = nullptr,
                    int* offset_out = nullptr);
     // Where the force pass of this step hashes the next step's keys.
-    NextKeys FusedNext() const { return NextKeys{key_[kc_ ^ 1].get(), count_[cur_].get()}; }
+    NextKeys FusedNext() const {
+        return NextKeys{key_[kc_ ^ 1].get(),
+                        CellRuns{count_[cur_].get(), fuse_links_ ? head_[cur_].get() : nullptr,
+                                 link_.get()}};
+    }
     // The force pass has written the next step's keys and counts.
     void KeysFused() {
         kc_ ^= 1;
@@ -147,8 +151,9 @@ class UniformGrid3D {
     int* count() const { return count_[last_].get(); }
     int* offset() const { return offset_.get(); }
     int* list() const { return list_.get(); }
-    // Zero both counters (the counter of the next build must start at zero;
-    // each build's scan clears the other one); drops keys hashed ahead.
+    // Zero both counters and list heads (those of the next build must start
+    // at zero; each build's scan clears the other ones); drops keys hashed
+    // ahead.
     void ClearCounters(hipStream_t st);
     struct Parity {
         int cur, last, kc, last_kc, keys_ready;
@@ -165,10 +170,11 @@ class UniformGrid3D {
 
    private:
     GridDesc g_{};
-    DeviceBuffer<int> key_[2], count_[2], fill_, list_, offset_, ws_;
-    DeviceBuffer<int2> runs_;
-    int cur_ = 0, last_ = 0;       // counter double buffer
+    DeviceBuffer<int> key_[2], count_[2], head_[2], list_, offset_, ws_;
+    DeviceBuffer<int2> link_;      // run lists; written and read between two scans
+    int cur_ = 0, last_ = 0;       // counter and list head double buffer
     int kc_ = 0, last_kc_ = 0;     // key double buffer
+    bool fuse_links_ = true;       // the counting passes list the runs too (kFuseLinksMax)
     bool keys_ready_ = false;      // key_[kc_] / count_[cur_] hold the next build's hash
 };
 

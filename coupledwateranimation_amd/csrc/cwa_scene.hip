@@ -65,9 +65,10 @@ void UniformGrid3D::Init(const GridDesc& g, int max_particles) {
     for (int k = 0; k < 2; ++k) {
         key_[k].resize(np);
         count_[k].resize(nc);
+        head_[k].resize(nc);
     }
-    fill_.resize(nc);
-    runs_.resize(np);
+    link_.resize(np);
+    fuse_links_ = max_particles <= kFuseLinksMax;
     list_.resize(np);
     offset_.resize(nc + 1);
     ws_.resize(scan_workspace_ints((int)nc));
@@ -77,9 +78,9 @@ void UniformGrid3D::Init(const GridDesc& g, int max_particles) {
 }
 
 void UniformGrid3D::ClearCounters(hipStream_t st) {
-    for (auto& c : count_) hip_check(launch_fill_i32(c.get(), num_cells(), 0, st), "clear counts");
-    hip_check(launch_fill_i32(fill_.get(), num_cells(), 0, st), "clear fill");
-    hip_check(launch_fill_i32(offset_.get(), num_cells() + 1, 0, st), "clear offsets");
+    hip_check(launch_clear_cells(offset_.get(), count_[0].get(), count_[1].get(), head_[0].get(),
+                                 head_[1].get(), num_cells(), st),
+              "clear counters");
     keys_ready_ = false;
 }
 
@@ -91,25 +92,29 @@ void UniformGrid3D::BuildGrid(const ParticleArrays& A, int n, float4* bpos, int*
     auto mark = [&](int slot, int which) {
         if (ev) hip_check(hipEventRecord(ev[2 * slot + which], st), "event");
     };
-    int* cnt = count_[cur_].get();  // zero: cleared by the previous build's scan
+    // zero before they are filled: cleared by the previous build's scan
+    int* head = head_[cur_].get();
+    const CellRuns runs{count_[cur_].get(), fuse_links_ ? head : nullptr, link_.get()};
     int* key = key_[kc_].get();
     mark(K_HASH, 0);
     if (!keys_ready_)  // else the last force pass hashed these positions
-        hip_check(launch_hash_count(A.pos, n, g_, key, cnt, st), "hash");
+        hip_check(launch_hash_count(A.pos, n, g_, key, runs, st), "hash");
     mark(K_HASH, 1);
     keys_ready_ = false;
     mark(K_SCAN, 0);
-    hip_check(launch_scan(cnt, off, nc, ws_.get(), st, count_[cur_ ^ 1].get()), "scan");
+    hip_check(launch_scan(runs.count, off, nc, ws_.get(), st, count_[cur_ ^ 1].get(),
+                          head_[cur_ ^ 1].get()),
+              "scan");
     mark(K_SCAN, 1);
     last_ = cur_;
     cur_ ^= 1;
     last_kc_ = kc_;
     mark(K_SCATTER, 0);
-    hip_check(launch_scatter_runs(key, off, fill_.get(), n, runs_.get(), st), "scatter");
+    if (!fuse_links_) hip_check(launch_link_runs(key, n, head, runs.link, st), "link runs");
     mark(K_SCATTER, 1);
     mark(K_REORDER, 0);
-    hip_check(launch_stable_reorder(key, off, runs_.get(), n, nullptr, lst, A.pos, A.id, bpos, bid,
-                                    fill_.get(), nc, st),
+    hip_check(launch_stable_reorder(key, off, head, runs.link, n, nullptr, lst, A.pos, A.id, bpos,
+                                    bid, st),
               "reorder");
     mark(K_REORDER, 1);
 }
@@ -673,7 +678,7 @@ void CoupledScene::Readback(cwa_host_state* h) {
 
 // ===========================================================================
 // Scratch of the allocation-free grid build (cwa_grid_build_static): run
-// records for up to kStaticMaxItems items, fill counters for up to
+// links for up to kStaticMaxItems items, run-list heads for up to
 // kStaticMaxCells cells and the cell scan's workspace, in one file-scope
 // device array that every GPU running the library holds until the process
 // ends (32 MB).  Host code never passes the array's name to a kernel: its
@@ -682,13 +687,13 @@ void CoupledScene::Readback(cwa_host_state* h) {
 namespace cwa {
 constexpr int kStaticMaxItems = 1 << 21;
 constexpr int kStaticMaxCells = 1 << 22;
-constexpr size_t kStaticRunsBytes = (size_t)kStaticMaxItems * sizeof(int2);
-constexpr size_t kStaticFillBytes = (size_t)kStaticMaxCells * sizeof(int);
+constexpr size_t kStaticLinkBytes = (size_t)kStaticMaxItems * sizeof(int2);
+constexpr size_t kStaticHeadBytes = (size_t)kStaticMaxCells * sizeof(int);
 constexpr size_t kStaticWsInts = 8192;  // scan_workspace_ints(kStaticMaxCells) is 4099
 }  // namespace cwa
 
-static __device__ __align__(256) unsigned char scratch[cwa::kStaticRunsBytes +
-                                                       cwa::kStaticFillBytes +
+static __device__ __align__(256) unsigned char scratch[cwa::kStaticLinkBytes +
+                                                       cwa::kStaticHeadBytes +
                                                        cwa::kStaticWsInts * sizeof(int)];
 
 namespace cwa {
@@ -1087,17 +1092,19 @@ int cwa_grid_build(const float* d_pos4, int n, const float grid_min[3], float ce
         g.cell = cell_size;
         g.cell_y = cell_size;
         const int nc = dims[0] * dims[1] * dims[2];
-        DeviceBuffer<int> fill(nc), ws(scan_workspace_ints(nc));
-        DeviceBuffer<int2> runs((size_t)std::max(n, 1));
-        hip_check(launch_fill_i32(d_count, nc, 0, st), "clear");
-        hip_check(launch_fill_i32(fill.get(), nc, 0, st), "clear fill");
-        hip_check(launch_hash_count(reinterpret_cast<const float4*>(d_pos4), n, g, d_key, d_count,
+        DeviceBuffer<int> head(nc), ws(scan_workspace_ints(nc));
+        DeviceBuffer<int2> link((size_t)std::max(n, 1));
+        const bool fuse = n <= kFuseLinksMax;
+        const CellRuns runs{d_count, fuse ? head.get() : nullptr, link.get()};
+        hip_check(launch_clear_cells(nullptr, d_count, head.get(), nullptr, nullptr, nc, st),
+                  "clear");
+        hip_check(launch_hash_count(reinterpret_cast<const float4*>(d_pos4), n, g, d_key, runs,
                                     st),
                   "hash");
         hip_check(launch_scan(d_count, d_offset, nc, ws.get(), st), "scan");
-        hip_check(launch_scatter_runs(d_key, d_offset, fill.get(), n, runs.get(), st), "scatter");
-        hip_check(launch_stable_reorder(d_key, d_offset, runs.get(), n, nullptr, d_list, nullptr,
-                                        nullptr, nullptr, nullptr, nullptr, 0, st),
+        if (!fuse) hip_check(launch_link_runs(d_key, n, head.get(), link.get(), st), "link runs");
+        hip_check(launch_stable_reorder(d_key, d_offset, head.get(), link.get(), n, nullptr,
+                                        d_list, nullptr, nullptr, nullptr, nullptr, st),
                   "stable insert");
         hip_check(hipStreamSynchronize(st), "grid sync");
     });
@@ -1127,19 +1134,20 @@ int cwa_grid_build_static(const float* d_pos4, int n, const float grid_min[3], f
         g.cell = cell_size;
         g.cell_y = cell_size;
         unsigned char* base = static_scratch();
-        int2* runs = reinterpret_cast<int2*>(base);
-        int* fill = reinterpret_cast<int*>(base + kStaticRunsBytes);
-        int* ws = reinterpret_cast<int*>(base + kStaticRunsBytes + kStaticFillBytes);
+        int2* link = reinterpret_cast<int2*>(base);
+        int* head = reinterpret_cast<int*>(base + kStaticLinkBytes);
+        int* ws = reinterpret_cast<int*>(base + kStaticLinkBytes + kStaticHeadBytes);
         // the array keeps the last call's contents: clear what must start at zero
-        hip_check(launch_fill_i32(d_count, nc, 0, st), "clear");
-        hip_check(launch_fill_i32(fill, nc, 0, st), "clear fill");
-        hip_check(launch_hash_count(reinterpret_cast<const float4*>(d_pos4), n, g, d_key, d_count,
+        const bool fuse = n <= kFuseLinksMax;
+        const CellRuns runs{d_count, fuse ? head : nullptr, link};
+        hip_check(launch_clear_cells(nullptr, d_count, head, nullptr, nullptr, nc, st), "clear");
+        hip_check(launch_hash_count(reinterpret_cast<const float4*>(d_pos4), n, g, d_key, runs,
                                     st),
                   "hash");
         hip_check(launch_scan(d_count, d_offset, nc, ws, st), "scan");
-        hip_check(launch_scatter_runs(d_key, d_offset, fill, n, runs, st), "scatter");
-        hip_check(launch_stable_reorder(d_key, d_offset, runs, n, nullptr, d_list, nullptr,
-                                        nullptr, nullptr, nullptr, nullptr, 0, st),
+        if (!fuse) hip_check(launch_link_runs(d_key, n, head, link, st), "link runs");
+        hip_check(launch_stable_reorder(d_key, d_offset, head, link, n, nullptr, d_list, nullptr,
+                                        nullptr, nullptr, nullptr, st),
                   "stable insert");
     });
 }
@@ -1185,19 +1193,18 @@ int cwa_grid_build_boxes(const float* d_centre4, const float* d_halfw4, int n,
         const int npairs = (int)npairs64;
         hip_check(launch_scan(ncov.get(), first.get(), n, ws.get(), st), "cover scan");
         const size_t np = (size_t)std::max(npairs, 1);
-        DeviceBuffer<int> pkey(np), pbox(np), fill(nc);
-        DeviceBuffer<int2> runs(np);
+        DeviceBuffer<int> pkey(np), pbox(np), head(nc);
+        DeviceBuffer<int2> link(np);
+        const CellRuns runs{d_count, head.get(), link.get()};
         hip_check(launch_box_pairs(x, hw, n, grid_min, cell_size, dims, first.get(), pkey.get(),
                                    pbox.get(), st),
                   "pairs");
-        hip_check(launch_fill_i32(d_count, nc, 0, st), "clear");
-        hip_check(launch_fill_i32(fill.get(), nc, 0, st), "clear fill");
-        hip_check(launch_key_count(pkey.get(), npairs, d_count, st), "count");
+        hip_check(launch_clear_cells(nullptr, d_count, head.get(), nullptr, nullptr, nc, st),
+                  "clear");
+        hip_check(launch_key_count(pkey.get(), npairs, runs, st), "count");
         hip_check(launch_scan(d_count, d_offset, nc, ws.get(), st), "scan");
-        hip_check(launch_scatter_runs(pkey.get(), d_offset, fill.get(), npairs, runs.get(), st),
-                  "scatter");
-        hip_check(launch_stable_reorder(pkey.get(), d_offset, runs.get(), npairs, pbox.get(),
-                                        d_list, nullptr, nullptr, nullptr, nullptr, nullptr, 0,
+        hip_check(launch_stable_reorder(pkey.get(), d_offset, head.get(), link.get(), npairs,
+                                        pbox.get(), d_list, nullptr, nullptr, nullptr, nullptr,
                                         st),
                   "stable insert");
         hip_check(hipStreamSynchronize(st), "box grid sync");
