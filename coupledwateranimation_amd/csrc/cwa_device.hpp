@@ -292,27 +292,49 @@ __device__ __forceinline__ float fetch_clamped(const float* __restrict__ img, in
     return img[(size_t)j * (size_t)w + (size_t)i];
 }
 
-__device__ __forceinline__ float bilerp(const float* __restrict__ img, int w, int h, float x,
-                                        float y) {
+// The four texels of a bilinear sample and its weights: taken apart so that a
+// kernel can have the loads in flight long before it needs the value.
+struct TexTaps {
+    float a, b, t00, t10, t01, t11;
+    __device__ __forceinline__ float value() const {
 #pragma clang fp contract(off)  // each product and sum rounded, as the oracle's sampler
+        const float r0 = (1.0f - a) * t00 + a * t10;
+        const float r1 = (1.0f - a) * t01 + a * t11;
+        return (1.0f - b) * r0 + b * r1;
+    }
+};
+
+__device__ __forceinline__ TexTaps bilerp_taps(const float* __restrict__ img, int w, int h,
+                                               float x, float y) {
+#pragma clang fp contract(off)
     float fx = floorf(x), fy = floorf(y);
-    const float a = x - fx, b = y - fy;
+    TexTaps t;
+    t.a = x - fx;
+    t.b = y - fy;
     fx = fminf(fmaxf(fx, -2.0f), (float)(w + 1));
     fy = fminf(fmaxf(fy, -2.0f), (float)(h + 1));
     const int i0 = (int)fx, j0 = (int)fy;
-    const float t00 = fetch_clamped(img, w, h, i0, j0);
-    const float t10 = fetch_clamped(img, w, h, i0 + 1, j0);
-    const float t01 = fetch_clamped(img, w, h, i0, j0 + 1);
-    const float t11 = fetch_clamped(img, w, h, i0 + 1, j0 + 1);
-    const float r0 = (1.0f - a) * t00 + a * t10;
-    const float r1 = (1.0f - a) * t01 + a * t11;
-    return (1.0f - b) * r0 + b * r1;
+    t.t00 = fetch_clamped(img, w, h, i0, j0);
+    t.t10 = fetch_clamped(img, w, h, i0 + 1, j0);
+    t.t01 = fetch_clamped(img, w, h, i0, j0 + 1);
+    t.t11 = fetch_clamped(img, w, h, i0 + 1, j0 + 1);
+    return t;
+}
+
+__device__ __forceinline__ TexTaps tex_taps(const float* __restrict__ img, int w, int h, float u,
+                                            float v) {
+#pragma clang fp contract(off)
+    return bilerp_taps(img, w, h, u * (float)w - 0.5f, v * (float)h - 0.5f);
+}
+
+__device__ __forceinline__ float bilerp(const float* __restrict__ img, int w, int h, float x,
+                                        float y) {
+    return bilerp_taps(img, w, h, x, y).value();
 }
 
 __device__ __forceinline__ float tex_sample(const float* __restrict__ img, int w, int h, float u,
                                             float v) {
-#pragma clang fp contract(off)
-    return bilerp(img, w, h, u * (float)w - 0.5f, v * (float)h - 0.5f);
+    return tex_taps(img, w, h, u, v).value();
 }
 
 // Runs of equal keys among the 64 lanes of a wave (lane order): whether the
