@@ -63,15 +63,16 @@ void UniformGrid3D::Init(const GridDesc& g, int max_particles) {
     const size_t nc = (size_t)g.dims[0] * g.dims[1] * g.dims[2];
     const size_t np = (size_t)std::max(max_particles, 1);
     for (int k = 0; k < 2; ++k) {
-        key_[k].resize(np);
-        count_[k].resize(nc);
-        head_[k].resize(nc);
+        slab_.add(key_[k], np);
+        slab_.add(count_[k], nc);
+        slab_.add(head_[k], nc);
     }
-    link_.resize(np);
+    slab_.add(link_, np);
     fuse_links_ = max_particles <= kFuseLinksMax;
-    list_.resize(np);
-    offset_.resize(nc + 1);
-    ws_.resize(scan_workspace_ints((int)nc));
+    slab_.add(list_, np);
+    slab_.add(offset_, nc + 1);
+    slab_.add(ws_, scan_workspace_ints((int)nc));
+    slab_.commit();
     cur_ = last_ = 0;
     kc_ = last_kc_ = 0;
     keys_ready_ = false;
@@ -125,7 +126,8 @@ void UniformGrid3D::BuildGrid(const ParticleArrays& A, int n, float4* bpos, int*
 void HeightField2DTripleBuffered::Allocate(int w, int h) {
     w_ = w;
     h_ = h;
-    for (auto& b : img_) b.resize((size_t)w * h);
+    for (auto& b : img_) slab_.add(b, (size_t)w * h);
+    slab_.commit();
     read_[0] = 0;
     read_[1] = 1;
     write_ = 2;
@@ -195,20 +197,21 @@ void SphParticles3D::Allocate(int n) {
     n_ = n;
     const size_t m = (size_t)std::max(n, 1);
     for (int k = 0; k < 2; ++k) {
-        pos_[k].resize(m);
-        vel_[k].resize(m);
-        force_[k].resize(m);
-        id_[k].resize(m);
+        slab_.add(pos_[k], m);
+        slab_.add(vel_[k], m);
+        slab_.add(force_[k], m);
+        slab_.add(id_[k], m);
     }
-    bpos_.resize(m);
-    bid_.resize(m);
-    rho_.resize(m);
-    prs_.resize(m);
-    rho_w_.resize(m);
-    flux_.resize(m);
-    vpad_.resize(m);
-    nbw_.resize(nb_buffer_uint2(m));
-    nrec_.resize(2 * m);
+    slab_.add(bpos_, m);
+    slab_.add(bid_, m);
+    slab_.add(rho_, m);
+    slab_.add(prs_, m);
+    slab_.add(rho_w_, m);
+    slab_.add(flux_, m);
+    slab_.add(vpad_, m);
+    slab_.add(nbw_, nb_buffer_uint2(m));
+    slab_.add(nrec_, 2 * m);
+    slab_.commit();
     A = ParticleArrays{pos_[0].get(), vel_[0].get(), force_[0].get(), id_[0].get()};
     N = ParticleArrays{pos_[1].get(), vel_[1].get(), force_[1].get(), id_[1].get()};
     parity_ = 0;

@@ -65,7 +65,7 @@ class Tape {
         const float* h0 = nullptr;
         const float* h1 = nullptr;
     };
-    void alloc_step_tape(StepTape& t);
+    void plan_step_tape(StepTape& t);
     void release_pipeline();
     void save(Ckpt& c);
     void restore(const Ckpt& c, bool heights = true);
@@ -94,6 +94,7 @@ class Tape {
     int group_ = 1;  // lanes per particle of the pair adjoint, fixed at creation
     float dt_ = 0.0f;
     bool forward_done_ = false;
+    DeviceSlab slab_;  // every buffer below
     std::vector<Ckpt> ck_;
     std::vector<StepTape> tp_, tp2_;  // tp2_: the eager Backward's second tape
     hipStream_t ast_ = nullptr;       // the eager Backward's adjoint stream
@@ -120,35 +121,36 @@ Tape::Tape(CoupledScene& s, int nsteps, int every, bool pipelined)
     const size_t n = (size_t)std::max(n_, 1), tex = (size_t)W_ * H_;
     ck_.resize(nseg_ + 1);
     for (auto& c : ck_) {
-        c.pos.resize(n);
-        c.vel.resize(n);
-        c.force.resize(n);
-        c.id.resize(n);
-        c.rho.resize(n);
-        c.prs.resize(n);
-        c.h0.resize(tex);
-        c.h1.resize(tex);
+        slab_.add(c.pos, n);
+        slab_.add(c.vel, n);
+        slab_.add(c.force, n);
+        slab_.add(c.id, n);
+        slab_.add(c.rho, n);
+        slab_.add(c.prs, n);
+        slab_.add(c.h0, tex);
+        slab_.add(c.h1, tex);
     }
     tp_.resize(std::min(every, nsteps));
-    for (auto& t : tp_) alloc_step_tape(t);
-    // the stream and events are created last, so an allocation failure
-    // above leaves nothing behind (the buffers free themselves); the
-    // constructor body after them releases them if it throws
-    for (auto* b : {&xb_, &vb_, &xb2_, &vb2_, &xl_, &vl_}) b->resize(n);
-    adjrec_.resize(2 * n);
-    for (auto* b : {&G0_, &G1_, &G0n_, &G1n_}) b->resize(tex);
-    rhob_.resize(n);
-    rtb_.resize(n);
-    Sbar_.resize(ncol_);
-    pgrad_.resize(GRAD_NUM);
-    acc_wave_.resize((size_t)adj_wave_blocks(s.devparams()) * 5);
+    for (auto& t : tp_) plan_step_tape(t);
+    for (auto* b : {&xb_, &vb_, &xb2_, &vb2_, &xl_, &vl_}) slab_.add(*b, n);
+    slab_.add(adjrec_, 2 * n);
+    for (auto* b : {&G0_, &G1_, &G0n_, &G1n_}) slab_.add(*b, tex);
+    slab_.add(rhob_, n);
+    slab_.add(rtb_, n);
+    slab_.add(Sbar_, ncol_);
+    slab_.add(pgrad_, GRAD_NUM);
+    slab_.add(acc_wave_, (size_t)adj_wave_blocks(s.devparams()) * 5);
     group_ = adj_pair_group(n_);
-    acc_pair_.resize((size_t)adj_pair_blocks(std::max(n_, 1), group_) * 3);
+    slab_.add(acc_pair_, (size_t)adj_pair_blocks(std::max(n_, 1), group_) * 3);
+    if (pipelined && nseg_ > 1) {
+        tp2_.resize(tp_.size());
+        for (auto& t : tp2_) plan_step_tape(t);
+    }
+    slab_.commit();
+    // the stream and events are created last, so an allocation failure
+    // above leaves nothing behind (the slab frees itself); the constructor
+    // body after them releases them if it throws
     if (pipelined) {
-        if (nseg_ > 1) {
-            tp2_.resize(tp_.size());
-            for (auto& t : tp2_) alloc_step_tape(t);
-        }
         try {
             hip_check(hipStreamCreateWithFlags(&ast_, hipStreamNonBlocking), "adjoint stream");
             for (hipEvent_t& e : ev_)
@@ -175,20 +177,20 @@ void Tape::release_pipeline() {
         }
 }
 
-void Tape::alloc_step_tape(StepTape& t) {
+void Tape::plan_step_tape(StepTape& t) {
     const size_t n = (size_t)std::max(n_, 1), tex = (size_t)W_ * H_;
-    t.pos.resize(n);
-    t.vel.resize(n);
-    t.nrec.resize(2 * n);
-    t.fpre.resize(n);
-    t.list.resize(n);
-    t.offset.resize((size_t)ncell_ + 1);
-    t.nbw.resize(nb_buffer_uint2(n));
-    t.rho.resize(n);
-    t.rho_raw.resize(n);
-    t.pw.resize(n);
-    t.hout.resize(tex);
-    t.colflux.resize(ncol_);
+    slab_.add(t.pos, n);
+    slab_.add(t.vel, n);
+    slab_.add(t.nrec, 2 * n);
+    slab_.add(t.fpre, n);
+    slab_.add(t.list, n);
+    slab_.add(t.offset, (size_t)ncell_ + 1);
+    slab_.add(t.nbw, nb_buffer_uint2(n));
+    slab_.add(t.rho, n);
+    slab_.add(t.rho_raw, n);
+    slab_.add(t.pw, n);
+    slab_.add(t.hout, tex);
+    slab_.add(t.colflux, ncol_);
 }
 
 void Tape::save(Ckpt& c) {
