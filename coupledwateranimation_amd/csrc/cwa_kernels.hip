@@ -22,6 +22,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 
 #include "cwa_device.hpp"
 #include "cwa_kernels.hpp"
@@ -758,11 +759,151 @@ __device__ __forceinline__ void force_pair(float h, float4 pi, float4 vi, float 
 }
 
 // ---------------------------------------------------------------------------
+// Texels of the wave EVOLVE (wave_comp.glsl:171-206; the kernels are further
+// down).  Arithmetic is not contracted, so every kernel gives the oracle's
+// result bit for bit.  The column flux is read through cf(ix, iz), indices
+// inside the column grid.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ float wave_texel(const DevParams& P, float C0, float C1, float nn,
+                                            float ss, float ee, float ww, int i, bool flux,
+                                            float S, float dt) {
+#pragma clang fp contract(off)
+    float o = P.wc0 * C0 + P.lx * (ee + ww) + P.lz * (nn + ss) - P.wc1 * C1;
+    o *= P.atten;
+    if (flux) o += P.kappa * dt * (S * P.inv_area);
+    if (P.wake && o > P.wake_thr && i == P.W / 2) o += P.wake_amt;
+    return o;
+}
+
+// Column coordinates of texel i / row j, and the floor()ed coordinate as the
+// sampler clamps it.
+__device__ __forceinline__ float column_x(const DevParams& P, int i) {
+#pragma clang fp contract(off)
+    return P.ax * (float)i + P.bx;
+}
+__device__ __forceinline__ float column_z(const DevParams& P, int j) {
+#pragma clang fp contract(off)
+    return P.az * (float)j + P.bz;
+}
+__device__ __forceinline__ int floor_index(float g, int n) {
+    return (int)fminf(fmaxf(floorf(g), -2.0f), (float)(n + 1));
+}
+
+// bilerp() of the column grid at (gx, gz).
+template <class Col>
+__device__ __forceinline__ float colflux_at(const DevParams& P, const Col& cf, float gx, float gz) {
+#pragma clang fp contract(off)
+    const int w = P.dims[0], h = P.dims[2];
+    TexTaps t;
+    t.a = gx - floorf(gx);
+    t.b = gz - floorf(gz);
+    const int i0 = floor_index(gx, w), j0 = floor_index(gz, h);
+    const int ia = min(max(i0, 0), w - 1), ib = min(max(i0 + 1, 0), w - 1);
+    const int ja = min(max(j0, 0), h - 1), jb = min(max(j0 + 1, 0), h - 1);
+    t.t00 = cf(ia, ja);
+    t.t10 = cf(ib, ja);
+    t.t01 = cf(ia, jb);
+    t.t11 = cf(ib, jb);
+    return t.value();
+}
+
+// Column-flux source of texels i0..i0+3 of row j: bilerp of the column grid
+// at each texel's (gx, gz), with the same values and arithmetic as bilerp.
+// The four samples share gz and, when they fall in at most two adjacent x
+// cells (the column grid is much coarser than the texels), also their six
+// grid values, loaded once.
+template <class Col>
+__device__ __forceinline__ void colflux_quad(const DevParams& P, const Col& cf, int i0, int j,
+                                             float S[4]) {
+#pragma clang fp contract(off)
+    const int w = P.dims[0], h = P.dims[2];
+    const float gz = column_z(P, j);
+    float a[4];
+    int ix[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float gx = column_x(P, i0 + t);
+        a[t] = gx - floorf(gx);
+        ix[t] = floor_index(gx, w);
+    }
+    if (ix[3] - ix[0] > 1 || ix[3] < ix[0]) {  // a grid finer than the texels, or mirrored
+#pragma unroll
+        for (int t = 0; t < 4; ++t) S[t] = colflux_at(P, cf, column_x(P, i0 + t), gz);
+        return;
+    }
+    const float b = gz - floorf(gz);
+    const int j0 = floor_index(gz, h);
+    const int ra = min(max(j0, 0), h - 1), rb = min(max(j0 + 1, 0), h - 1);
+    float r0[3], r1[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int ik = min(max(ix[0] + k, 0), w - 1);
+        r0[k] = cf(ik, ra);
+        r1[k] = cf(ik, rb);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const bool d = ix[t] != ix[0];
+        const float t00 = d ? r0[1] : r0[0], t10 = d ? r0[2] : r0[1];
+        const float t01 = d ? r1[1] : r1[0], t11 = d ? r1[2] : r1[1];
+        const float q0 = (1.0f - a[t]) * t00 + a[t] * t10;
+        const float q1 = (1.0f - a[t]) * t01 + a[t] * t11;
+        S[t] = (1.0f - b) * q0 + b * q1;
+    }
+}
+
+// One texel, and four texels along u (W % 4 == 0, i0 % 4 == 0).
+template <class Col>
+__device__ __forceinline__ void wave_single(const DevParams& P, const float* __restrict__ h0,
+                                            const float* __restrict__ h1, float* __restrict__ out,
+                                            int i, int j, bool flux, const Col& cf, float dt) {
+    const int W = P.W, H = P.H;
+    const size_t c = (size_t)j * W + i;
+    const float C0 = h0[c];
+    const float C1 = h1[c];
+    const float nn = h0[(size_t)min(j + 1, H - 1) * W + i];
+    const float ss = h0[(size_t)max(j - 1, 0) * W + i];
+    const float ee = h0[(size_t)j * W + min(i + 1, W - 1)];
+    const float ww = h0[(size_t)j * W + max(i - 1, 0)];
+    const float S = flux ? colflux_at(P, cf, column_x(P, i), column_z(P, j)) : 0.0f;
+    out[c] = wave_texel(P, C0, C1, nn, ss, ee, ww, i, flux, S, dt);
+}
+
+template <class Col>
+__device__ __forceinline__ void wave_quad(const DevParams& P, const float* __restrict__ h0,
+                                          const float* __restrict__ h1, float* __restrict__ out,
+                                          int i0, int j, bool flux, const Col& cf, float dt) {
+    const int W = P.W, H = P.H;
+    const size_t row = (size_t)j * W;
+    const float4 c0 = *reinterpret_cast<const float4*>(h0 + row + i0);
+    // the older level is read once, here (nt; A/B on one box: step -0.75 %)
+    const float4 c1 = load_once(reinterpret_cast<const float4*>(h1 + row + i0));
+    const float4 nn = *reinterpret_cast<const float4*>(h0 + (size_t)min(j + 1, H - 1) * W + i0);
+    const float4 ss = *reinterpret_cast<const float4*>(h0 + (size_t)max(j - 1, 0) * W + i0);
+    const float west = h0[row + max(i0 - 1, 0)];
+    const float east = h0[row + min(i0 + 4, W - 1)];
+    float S[4] = {0.f, 0.f, 0.f, 0.f};
+    if (flux) colflux_quad(P, cf, i0, j, S);
+    float4 o;
+    o.x = wave_texel(P, c0.x, c1.x, nn.x, ss.x, c0.y, west, i0, flux, S[0], dt);
+    o.y = wave_texel(P, c0.y, c1.y, nn.y, ss.y, c0.z, c0.x, i0 + 1, flux, S[1], dt);
+    o.z = wave_texel(P, c0.z, c1.z, nn.z, ss.z, c0.w, c0.y, i0 + 2, flux, S[2], dt);
+    o.w = wave_texel(P, c0.w, c1.w, nn.w, ss.w, east, c0.z, i0 + 3, flux, S[3], dt);
+    *reinterpret_cast<float4*>(out + row + i0) = o;
+}
+
+// ---------------------------------------------------------------------------
 // Particle -> wave flux per vertical column of grid cells.  Each column is
 // one contiguous sorted range; one wave64 sums memory column `wave`
 // (lane-strided partial sums, then a fixed xor tree: deterministic) and
 // stores it at [iz*nx + ix] of its (ix, iz).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ float wave_sum_f32(float s) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
+}
+
 __device__ __forceinline__ void column_flux_sum(const int* __restrict__ offset,
                                                 const float* __restrict__ flux, int nx, int ny,
                                                 int nz, float* __restrict__ colflux, int wave,
@@ -771,14 +912,87 @@ __device__ __forceinline__ void column_flux_sum(const int* __restrict__ offset,
     const int b = offset[wave * ny], e = offset[(wave + 1) * ny];
     float s = 0.0f;
     for (int k = b + lane; k < e; k += 64) s += flux[k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    s = wave_sum_f32(s);
     if (lane == 0) {
         const int dims[3] = {nx, ny, nz};
         int ix, iz;
         grid_column_xz(dims, wave, ix, iz);
         colflux[iz * nx + ix] = s;
     }
+}
+
+// ---------------------------------------------------------------------------
+// The wave EVOLVE as blocks of the force launch (both read only the density
+// pass's output and the heightfields): a block of 256 threads advances one
+// tile of the heightfield.  It first sums the flux of the columns its texels
+// sample (column_flux_sum's order, so the same bits) into LDS, kTileColBatch
+// columns of a wave at a time; tiles are small enough that this takes a few
+// rounds (wave_tiles_for gives the rule).
+// ---------------------------------------------------------------------------
+constexpr int kTileColBatch = 4;
+
+__device__ __forceinline__ void wave_tile(const DevParams& P, const WaveTiles& w, int tile,
+                                          const int* __restrict__ offset,
+                                          const float* __restrict__ pflux, float dt,
+                                          float* __restrict__ s_col) {
+    const int tx = tile % w.nx, ty = tile / w.nx;
+    const int i_lo = tx * w.side, j_lo = ty * w.side;
+    const int i_hi = min(i_lo + w.side, P.W) - 1, j_hi = min(j_lo + w.side, P.H) - 1;
+    if (j_lo >= P.H) return;  // padding blocks
+    const int nx = P.dims[0], ny = P.dims[1], nz = P.dims[2];
+    int x0 = 0, z0 = 0, ncx = 0;
+    const bool flux = pflux != nullptr;
+    if (flux) {
+        // column coordinates are monotone in the texel index, so the tile's
+        // first and last texels bound what it samples
+        const int xa = floor_index(column_x(P, i_lo), nx), xb = floor_index(column_x(P, i_hi), nx);
+        const int za = floor_index(column_z(P, j_lo), nz), zb = floor_index(column_z(P, j_hi), nz);
+        x0 = min(max(min(xa, xb), 0), nx - 1);
+        z0 = min(max(min(za, zb), 0), nz - 1);
+        ncx = min(max(max(xa, xb) + 1, 0), nx - 1) - x0 + 1;
+        const int ncz = min(max(max(za, zb) + 1, 0), nz - 1) - z0 + 1;
+        const int nc = min(ncx * ncz, kWaveTileColumns);  // wave_tiles_for's bound
+        const int lane = threadIdx.x & 63;
+        for (int q0 = ((int)threadIdx.x >> 6) * kTileColBatch; q0 < nc; q0 += 4 * kTileColBatch) {
+            int k[kTileColBatch], e[kTileColBatch], longest = 0;
+            float s[kTileColBatch];
+#pragma unroll
+            for (int u = 0; u < kTileColBatch; ++u) {
+                s[u] = 0.0f;
+                k[u] = e[u] = 0;
+                if (q0 + u < nc) {
+                    const int c = grid_column(P.dims, x0 + (q0 + u) % ncx, z0 + (q0 + u) / ncx);
+                    k[u] = offset[c * ny];
+                    e[u] = offset[(c + 1) * ny];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kTileColBatch; ++u) {
+                longest = max(longest, e[u] - k[u]);
+                k[u] += lane;
+            }
+            for (; longest > 0; longest -= 64) {
+#pragma unroll
+                for (int u = 0; u < kTileColBatch; ++u) {
+                    if (k[u] < e[u]) s[u] += pflux[k[u]];
+                    k[u] += 64;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kTileColBatch; ++u) {
+                s[u] = wave_sum_f32(s[u]);
+                if (lane == 0 && q0 + u < nc) s_col[q0 + u] = s[u];
+            }
+        }
+        __syncthreads();
+    }
+    const auto cf = [&](int ix, int iz) { return s_col[(iz - z0) * ncx + (ix - x0)]; };
+    const int per = P.W % 4 == 0 ? 4 : 1;  // texels per thread along u
+    const int across = w.side / per;       // across * side <= 256 threads
+    const int i = i_lo + (int)threadIdx.x % across * per, j = j_lo + (int)threadIdx.x / across;
+    if (i > i_hi || j > j_hi) return;
+    if (per == 4) wave_quad(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
+    else wave_single(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
 }
 
 // ---------------------------------------------------------------------------
@@ -791,11 +1005,14 @@ __device__ __forceinline__ void column_flux_sum(const int* __restrict__ offset,
 // slot order.  When `next` is set it also hashes the new position into the
 // next step's grid (cell key, count and run lists, ComputeCounts of
 // ugrid_particles_cs.glsl:90-95), so that step needs no hash pass of its own.
-// Blocks nfb.. of the grid sum the particle flux per column instead (one
-// wave per column; they read only the density pass's output and run in
-// the force blocks' tail).
+// The grid's last blocks, from nfb on, sum the particle flux per column (one
+// wave per column; they read only the density pass's output and run in the
+// force blocks' tail).  With kWave the first wt.nblk blocks advance the
+// heightfield (wave_tile), which small scenes would otherwise wait on a launch
+// for (wave_tiles_for gives the rule and both sides); their number is a
+// multiple of eight, so the force blocks keep the density pass's XCDs.
 // ---------------------------------------------------------------------------
-template <bool kLink>
+template <bool kLink, bool kWave>
 __global__ void __launch_bounds__(256) k_force_integrate(
     const DevParams* __restrict__ Pd, float dt, const float4* __restrict__ bpos,
     const int* __restrict__ bid, const float* __restrict__ vpad,
@@ -805,18 +1022,25 @@ __global__ void __launch_bounds__(256) k_force_integrate(
     const float* __restrict__ H0, float4* __restrict__ pos_o,
     float4* __restrict__ vel_o, float4* __restrict__ force_o, int* __restrict__ id_o,
     float* __restrict__ rho_o, float* __restrict__ prs_o, float4* __restrict__ fpre, int nfb,
-    const float* __restrict__ pflux, float* __restrict__ colflux, NextKeys next) {
+    const float* __restrict__ pflux, float* __restrict__ colflux, NextKeys next, WaveTiles wt) {
     const DevParams& P = *Pd;
-    if ((int)blockIdx.x >= nfb) {
+    __shared__ uint2 s_nb[kNbStage][256];
+    static_assert(sizeof(s_nb) >= kWaveTileColumns * sizeof(float), "a tile's column sums");
+    if (kWave && (int)blockIdx.x < wt.nblk) {
+        wave_tile(P, wt, blockIdx.x, offset, colflux ? pflux : nullptr, dt,
+                  reinterpret_cast<float*>(&s_nb[0][0]));
+        return;
+    }
+    const int blk = (int)blockIdx.x - (kWave ? wt.nblk : 0);
+    if (blk >= nfb) {
         column_flux_sum(offset, pflux, P.dims[0], P.dims[1], P.dims[2], colflux,
-                        (((int)blockIdx.x - nfb) * (int)blockDim.x + (int)threadIdx.x) >> 6,
+                        ((blk - nfb) * (int)blockDim.x + (int)threadIdx.x) >> 6,
                         threadIdx.x & 63);
         return;
     }
-    const int i = xcd_block(blockIdx.x, nfb) * blockDim.x + threadIdx.x;
+    const int i = xcd_block(blk, nfb) * blockDim.x + threadIdx.x;
     const bool valid = i < n;
     int cell = -1;
-    __shared__ uint2 s_nb[kNbStage][256];
     if (valid) {
         const float4 own_a = nrec[2 * (size_t)i];      // (x, y, z, p)
         const float4 own_b = nrec[2 * (size_t)i + 1];  // (vx, vy, vz, 1/rho)
@@ -986,101 +1210,23 @@ __global__ void __launch_bounds__(256) k_neighbour_counts(const DevParams* __res
 
 // ---------------------------------------------------------------------------
 // Wave EVOLVE (wave_comp.glsl:171-206), lambda split per axis, clamped
-// neighbours, optional particle flux source, wake line.  Arithmetic is not
-// contracted so the result matches the oracle bit for bit.
+// neighbours, optional particle flux source, wake line, as a launch of its
+// own (steps without particles, grids too fine for wave_tile, profiled steps).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) k_wave(const DevParams* __restrict__ Pd, const float* __restrict__ h0,
                                               const float* __restrict__ h1,
                                               float* __restrict__ out,
                                               const float* __restrict__ colflux, float dt) {
-#pragma clang fp contract(off)
     const DevParams& P = *Pd;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int W = P.W, H = P.H;
-    if (i >= W || j >= H) return;
-    const size_t c = (size_t)j * W + i;
-    const float C0 = h0[c];
-    const float C1 = h1[c];
-    const float nn = h0[(size_t)min(j + 1, H - 1) * W + i];
-    const float ss = h0[(size_t)max(j - 1, 0) * W + i];
-    const float ee = h0[(size_t)j * W + min(i + 1, W - 1)];
-    const float ww = h0[(size_t)j * W + max(i - 1, 0)];
-    float o = P.wc0 * C0 + P.lx * (ee + ww) + P.lz * (nn + ss) - P.wc1 * C1;
-    o *= P.atten;
-    if (colflux) {
-        const float gx = P.ax * (float)i + P.bx, gz = P.az * (float)j + P.bz;
-        const float S = bilerp(colflux, P.dims[0], P.dims[2], gx, gz);
-        o += P.kappa * dt * (S * P.inv_area);
-    }
-    if (P.wake && o > P.wake_thr && i == W / 2) o += P.wake_amt;
-    out[c] = o;
+    if (i >= P.W || j >= P.H) return;
+    const int nx = P.dims[0];
+    const auto cf = [&](int ix, int iz) { return colflux[(size_t)iz * nx + ix]; };
+    wave_single(P, h0, h1, out, i, j, colflux != nullptr, cf, dt);
 }
 
-// The same EVOLVE, four texels per thread along u (W % 4 == 0): float4
-// loads of the centre, north and south rows and of h^(n-1), scalar loads of
-// the west / east neighbours of the quad.  Per texel the arithmetic is that
-// of k_wave, so both give identical results.
-__device__ __forceinline__ float wave_texel(const DevParams& P, float C0, float C1, float nn,
-                                            float ss, float ee, float ww, int i, bool flux,
-                                            float S, float dt) {
-#pragma clang fp contract(off)
-    float o = P.wc0 * C0 + P.lx * (ee + ww) + P.lz * (nn + ss) - P.wc1 * C1;
-    o *= P.atten;
-    if (flux) o += P.kappa * dt * (S * P.inv_area);
-    if (P.wake && o > P.wake_thr && i == P.W / 2) o += P.wake_amt;
-    return o;
-}
-
-// Column-flux source of texels i0..i0+3 of row j: bilerp of the column grid
-// at each texel's (gx, gz), with the same values and arithmetic as bilerp.
-// The four samples share gz and, when they fall in at most two adjacent x
-// cells (the column grid is much coarser than the texels), also their six
-// grid values, loaded once.
-__device__ __forceinline__ void colflux_quad(const DevParams& P, const float* __restrict__ cf,
-                                             int i0, int j, float S[4]) {
-#pragma clang fp contract(off)
-    const int w = P.dims[0], h = P.dims[2];
-    const float gz = P.az * (float)j + P.bz;
-    float a[4];
-    int ix[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const float gx = P.ax * (float)(i0 + t) + P.bx;
-        float fx = floorf(gx);
-        a[t] = gx - fx;
-        fx = fminf(fmaxf(fx, -2.0f), (float)(w + 1));
-        ix[t] = (int)fx;
-    }
-    if (ix[3] - ix[0] > 1) {  // a grid finer than the texels: sample one by one
-#pragma unroll
-        for (int t = 0; t < 4; ++t) S[t] = bilerp(cf, w, h, P.ax * (float)(i0 + t) + P.bx, gz);
-        return;
-    }
-    float fy = floorf(gz);
-    const float b = gz - fy;
-    fy = fminf(fmaxf(fy, -2.0f), (float)(h + 1));
-    const int j0 = (int)fy;
-    const size_t ra = (size_t)min(max(j0, 0), h - 1) * w;
-    const size_t rb = (size_t)min(max(j0 + 1, 0), h - 1) * w;
-    float r0[3], r1[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int ik = min(max(ix[0] + k, 0), w - 1);
-        r0[k] = cf[ra + ik];
-        r1[k] = cf[rb + ik];
-    }
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const bool d = ix[t] != ix[0];
-        const float t00 = d ? r0[1] : r0[0], t10 = d ? r0[2] : r0[1];
-        const float t01 = d ? r1[1] : r1[0], t11 = d ? r1[2] : r1[1];
-        const float q0 = (1.0f - a[t]) * t00 + a[t] * t10;
-        const float q1 = (1.0f - a[t]) * t01 + a[t] * t11;
-        S[t] = (1.0f - b) * q0 + b * q1;
-    }
-}
-
+// The same EVOLVE, four texels per thread along u (W % 4 == 0).
 __global__ void __launch_bounds__(256) k_wave4(const DevParams* __restrict__ Pd, const float* __restrict__ h0,
                                                const float* __restrict__ h1,
                                                float* __restrict__ out,
@@ -1088,25 +1234,10 @@ __global__ void __launch_bounds__(256) k_wave4(const DevParams* __restrict__ Pd,
     const DevParams& P = *Pd;
     const int i0 = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
     const int j = blockIdx.y * blockDim.y + threadIdx.y;
-    const int W = P.W, H = P.H;
-    if (i0 >= W || j >= H) return;
-    const size_t row = (size_t)j * W;
-    const float4 c0 = *reinterpret_cast<const float4*>(h0 + row + i0);
-    // the older level is read once, here (nt; A/B on one box: step -0.75 %)
-    const float4 c1 = load_once(reinterpret_cast<const float4*>(h1 + row + i0));
-    const float4 nn = *reinterpret_cast<const float4*>(h0 + (size_t)min(j + 1, H - 1) * W + i0);
-    const float4 ss = *reinterpret_cast<const float4*>(h0 + (size_t)max(j - 1, 0) * W + i0);
-    const float west = h0[row + max(i0 - 1, 0)];
-    const float east = h0[row + min(i0 + 4, W - 1)];
-    const bool flux = colflux != nullptr;
-    float S[4] = {0.f, 0.f, 0.f, 0.f};
-    if (flux) colflux_quad(P, colflux, i0, j, S);
-    float4 o;
-    o.x = wave_texel(P, c0.x, c1.x, nn.x, ss.x, c0.y, west, i0, flux, S[0], dt);
-    o.y = wave_texel(P, c0.y, c1.y, nn.y, ss.y, c0.z, c0.x, i0 + 1, flux, S[1], dt);
-    o.z = wave_texel(P, c0.z, c1.z, nn.z, ss.z, c0.w, c0.y, i0 + 2, flux, S[2], dt);
-    o.w = wave_texel(P, c0.w, c1.w, nn.w, ss.w, east, c0.z, i0 + 3, flux, S[3], dt);
-    *reinterpret_cast<float4*>(out + row + i0) = o;
+    if (i0 >= P.W || j >= P.H) return;
+    const int nx = P.dims[0];
+    const auto cf = [&](int ix, int iz) { return colflux[(size_t)iz * nx + ix]; };
+    wave_quad(P, h0, h1, out, i0, j, colflux != nullptr, cf, dt);
 }
 
 // InitWave (wave_comp.glsl:82-140): peak * smoothstep(5, 0, d), d = distance
@@ -1243,16 +1374,56 @@ hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bp
                                   const float4* nrec, const float* H0, ParticleArrays& N,
                                   float* rho, float* prs, float4* fpre, const float* flux,
                                   float* colflux, const float* vpad, const NextKeys& next,
-                                  hipStream_t st) {
+                                  const WaveTiles& wt, hipStream_t st) {
     if (n <= 0) return hipSuccess;
     const int nfb = blocks_for(n, 256);
     const long long ncol = colflux ? (long long)P.dims[0] * P.dims[2] : 0;
     const int ncb = blocks_for(ncol * 64, 256);
-    const auto kernel = next.runs.head ? k_force_integrate<true> : k_force_integrate<false>;
-    kernel<<<nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list, offset, n, rho_w,
-                                      nbw, nrec, H0, N.pos, N.vel, N.force, N.id, rho, prs, fpre,
-                                      nfb, flux, colflux, next);
+    const bool link = next.runs.head != nullptr;
+    if (wt.nblk && !link) return hipErrorInvalidValue;  // kFuseWaveParticles <= kFuseLinksMax
+    const auto kernel = wt.nblk ? k_force_integrate<true, true>
+                        : link  ? k_force_integrate<true, false>
+                                : k_force_integrate<false, false>;
+    kernel<<<wt.nblk + nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list, offset,
+                                                n, rho_w, nbw, nrec, H0, N.pos, N.vel, N.force,
+                                                N.id, rho, prs, fpre, nfb, flux, colflux, next,
+                                                wt);
     return hipGetLastError();
+}
+
+// Tiles of 32 texels a side (four a thread; 16 and one where W % 4 != 0 or the
+// grid is fine) whose samples touch at most kWaveTileColumns columns, up to
+// kFuseWaveTiles of them, for scenes of up to kFuseWaveParticles particles;
+// none (nblk 0) otherwise.  There the step is bound by its launches, and the
+// tiles end before the force blocks do (MI355X, three scenes in flight / alone,
+// launch of its own -> blocks of the force launch: 4 096 particles and 128^2
+// texels 14.9 / 42.9 -> 14.0 / 40.0 us a step, 5 000 and 100^2 16.9 / 39.1 ->
+// 15.2 / 36.1, 50 000 and 512^2 19.4 / 47.3 -> 19.1 / 44.7).  Larger fields
+// stream better at the occupancy of the wave's own kernel (40 000 and 1000^2
+// 19.6 -> 24.0 in flight, 10 000 and 501^2 39.6 -> 41.5 alone), larger scenes
+// fill the chip without them (120 000 and 301^2 34.2 -> 35.3 in flight), and on
+// a grid too fine for the texels a tile spends longer on its columns than a
+// launch takes.
+WaveTiles wave_tiles_for(const DevParams& P, int n, bool flux, const float* h0,
+                         const float* h1, float* out) {
+    WaveTiles w{h0, h1, out, 0, 1, 0};
+    if (P.W <= 0 || P.H <= 0 || n > kFuseWaveParticles) return w;
+    const auto spans = [](float per_texel, int texels, int n) {
+        // floor(first) .. floor(last) + 1, one more for the rounding of the ends
+        return std::min<double>((double)std::fabs(per_texel) * (texels - 1) + 3.0, n);
+    };
+    for (int side : {32, 16}) {
+        if (side == 32 && P.W % 4 != 0) continue;  // one quad or one texel a thread
+        if (flux && spans(P.ax, side, P.dims[0]) * spans(P.az, side, P.dims[2]) > kWaveTileColumns)
+            continue;
+        const int nx = (P.W + side - 1) / side, ny = (P.H + side - 1) / side;
+        if ((long long)nx * ny > kFuseWaveTiles) continue;
+        w.side = side;
+        w.nx = nx;
+        w.nblk = (nx * ny + 7) / 8 * 8;
+        break;
+    }
+    return w;
 }
 
 hipError_t launch_neighbour_counts(const DevParams& P, const float4* pos, const int* offset,

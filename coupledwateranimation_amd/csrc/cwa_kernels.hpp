@@ -93,9 +93,25 @@ struct NextKeys {
     int* key;
     CellRuns runs;
 };
+// The heightfield's EVOLVE as blocks of the force launch: nblk tiles of
+// side x side texels, nx a row (nblk 0: none, the wave takes its own launch).
+struct WaveTiles {
+    const float* h0;
+    const float* h1;
+    float* out;
+    int nblk, nx, side;
+};
+constexpr int kWaveTileColumns = 128;  // columns a tile's samples may touch
+constexpr int kFuseWaveParticles = 1 << 16;
+constexpr int kFuseWaveTiles = 512;
+static_assert(kFuseWaveParticles <= kFuseLinksMax, "tiles go with the fused run lists");
+// n particles; flux: the step couples (the tiles sum the columns they sample).
+WaveTiles wave_tiles_for(const DevParams& P, int n, bool flux, const float* h0, const float* h1,
+                         float* out);
 // Forces + integration: own record from nrec, id from bid and the velocity
 // pad from vpad (sorted), previous force from the state S in its pre-sort
-// slot list[i]; writes the next state N in sorted order.  fpre (force before
+// slot list[i]; writes the next state N in sorted order.  The launch also
+// sums the column flux (colflux set) and advances the heightfield (wt).  fpre (force before
 // the foam branch) is an optional output for the adjoint tape.
 hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bpos,
                                   const int* bid, const ParticleArrays& S, const int* list,
@@ -103,7 +119,7 @@ hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bp
                                   const float4* nrec, const float* H0, ParticleArrays& N,
                                   float* rho, float* prs, float4* fpre, const float* flux,
                                   float* colflux, const float* vpad, const NextKeys& next,
-                                  hipStream_t st);
+                                  const WaveTiles& wt, hipStream_t st);
 // Neighbour counts (self included) of the last density pass, per sorted slot.
 hipError_t launch_neighbour_counts(const DevParams& P, const float4* pos, const int* offset,
                                    const uint2* nbw, int n, int* out, hipStream_t st);

@@ -480,6 +480,12 @@ void CoupledScene::Step(float dt, hipEvent_t (*ev)[2], const TapeOut* tape) {
     float4* nrec = pick(tape ? tape->nrec : nullptr, particles.nrec());
     float* rho_w = pick(tape ? tape->rho : nullptr, particles.rho_w());
     float* cflux = pick(tape ? tape->colflux : nullptr, colflux.get());
+    const float* H1 = taped_heights ? tape->h_in1 : wave.GetReadImage(1);
+    float* Hout = taped_heights ? tape->h_out : wave.GetWriteImage();
+    // the wave runs in the force launch; a profiled step launches it by
+    // itself, so that both have times of their own
+    WaveTiles wt{};
+    if (n > 0 && !ev) wt = wave_tiles_for(dp_, n, couple, H0, H1, Hout);
     if (n > 0) {
         grid.BuildGrid(particles.A, n, bpos, particles.bid(), st_, ev ? &ev[0][0] : nullptr, lst,
                        off);
@@ -490,26 +496,23 @@ void CoupledScene::Step(float dt, hipEvent_t (*ev)[2], const TapeOut* tape) {
                                  particles.vpad(), st_),
                   "density");
         mark(K_DENSITY, 1);
-        // the same launch sums the particle flux per column when coupled, and
-        // hashes the new positions into the next step's grid
+        // the same launch sums the particle flux per column when coupled,
+        // hashes the new positions into the next step's grid and advances
+        // the wave
         mark(K_FORCE, 0);
         hip_check(launch_force_integrate(dp_, dt, bpos, particles.bid(), particles.A, lst, off, n,
                                          rho_w, nbm, nrec, H0, particles.N, particles.rho(),
                                          particles.prs(), tape ? tape->fpre : nullptr,
                                          particles.flux(), couple ? cflux : nullptr,
-                                         particles.vpad(), grid.FusedNext(), st_),
+                                         particles.vpad(), grid.FusedNext(), wt, st_),
                   "force/integrate");
         mark(K_FORCE, 1);
         particles.Flip();
         grid.KeysFused();
     }
     mark(K_WAVE, 0);
-    if (taped_heights)
-        hip_check(launch_wave(dp_, tape->h_in0, tape->h_in1, tape->h_out, couple ? cflux : nullptr,
-                              dt, st_),
-                  "wave");
-    else
-        wave.Evolve(dp_, couple ? cflux : nullptr, dt, st_);
+    if (wt.nblk == 0)
+        hip_check(launch_wave(dp_, H0, H1, Hout, couple ? cflux : nullptr, dt, st_), "wave");
     mark(K_WAVE, 1);
     wave.PingPong();
     // the scene's own neighbour records and sorted copy now describe this step
