@@ -222,6 +222,76 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int* __restric
     if (total_out && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *total_out = total + prefix;
 }
 
+// The whole scan in one launch, for inputs of up to kScanOneTiles tiles of
+// kScanOneTile: each block sums the elements before its tile itself (from the
+// L2, kScanOneAhead 16-byte loads in flight per thread) instead of waiting for
+// a launch that has summed them.  Quadratic reads, so only while a block's
+// share is a few rounds; the input must not change during the launch, so it
+// must not overlap what is written.
+// SCANFIG
+constexpr int kScanOneThreads = 1024;
+constexpr int kScanOneTile = kScanOneThreads * kScanItems;  // 8192
+constexpr int kScanOneTiles = 8;
+constexpr int kScanOneAhead = 8;
+
+__global__ void __launch_bounds__(kScanOneThreads)
+    k_scan_one(const int* __restrict__ in, int n, int* __restrict__ out,
+               int* __restrict__ total_out, int* __restrict__ zero_out,
+               int* __restrict__ zero_out2) {
+    const int first = blockIdx.x * kScanOneTile;
+    int pre = 0;
+    if (aligned16(in)) {
+        const int4* __restrict__ q = reinterpret_cast<const int4*>(in);
+        const int end = first / 4;  // a multiple of 2 * kScanOneThreads
+        for (int t = threadIdx.x; t < end; t += kScanOneAhead * kScanOneThreads) {
+            int4 a[kScanOneAhead];
+#pragma unroll
+            for (int u = 0; u < kScanOneAhead; ++u) {
+                const int k = t + u * kScanOneThreads;
+                a[u] = k < end ? q[k] : make_int4(0, 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < kScanOneAhead; ++u) pre += a[u].x + a[u].y + a[u].z + a[u].w;
+        }
+    } else {
+        for (int t = threadIdx.x; t < first; t += kScanOneThreads) pre += in[t];
+    }
+    const int base = first + threadIdx.x * kScanItems;
+    int v[kScanItems];
+    load_items(in, base, n, v);
+    int s = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) s += v[k];
+    // one exchange for both: the waves' tile totals and their shares of the prefix
+    constexpr int kWaves = kScanOneThreads / 64;
+    __shared__ int wsum[kWaves], wpre[kWaves];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    const int incl = wave_incl_scan(s);
+    pre = wave_sum_i32(pre);
+    if (lane == 63) {
+        wsum[wid] = incl;
+        wpre[wid] = pre;
+    }
+    __syncthreads();
+    int run = incl - s, total = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+        run += wpre[w] + (w < wid ? wsum[w] : 0);
+        total += wpre[w] + wsum[w];
+    }
+    int o[kScanItems];
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        o[k] = run;
+        run += v[k];
+    }
+    store_items(out, base, n, o);
+    const int z[kScanItems] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (zero_out) store_items(zero_out, base, n, z);
+    if (zero_out2) store_items(zero_out2, base, n, z);
+    if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *total_out = total;
+}
+
 __global__ void k_scan_total(const int* __restrict__ src, int* __restrict__ dst) {
     if (threadIdx.x == 0) *dst = *src;
 }
@@ -239,13 +309,26 @@ size_t scan_workspace_ints(int n) {
     return ws + (size_t)(m + kScanTile - 1) / kScanTile + 1;
 }
 
+// Whether the int arrays [a, a + na) and [b, b + nb) share memory (null: no).
+static bool overlap(const int* a, size_t na, const int* b, size_t nb) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+    return a && b && p < q + nb * sizeof(int) && q < p + na * sizeof(int);
+}
+
 // out has n+1 entries; out[n] = total.  ws holds scan_workspace_ints(n).
-// Up to kScanDirectTiles tiles the tile prefixes are summed inside
+// One launch where k_scan_one takes the input, unless it is scanned in place.
+// Otherwise, up to kScanDirectTiles tiles the tile prefixes are summed inside
 // k_scan_down (two launches); larger inputs recurse on the tile sums.
 hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
                        int* zero_out, int* zero_out2) {
     if (n <= 0) {
         k_fill_i32<<<1, 64, 0, st>>>(out, 1, 0);
+        return hipGetLastError();
+    }
+    if (n <= kScanOneTile * kScanOneTiles && !overlap(in, n, out, (size_t)n + 1) &&
+        !overlap(in, n, zero_out, n) && !overlap(in, n, zero_out2, n)) {
+        k_scan_one<<<(n + kScanOneTile - 1) / kScanOneTile, kScanOneThreads, 0, st>>>(
+            in, n, out, out + n, zero_out, zero_out2);
         return hipGetLastError();
     }
     const int tiles = (n + kScanTile - 1) / kScanTile;

@@ -2,7 +2,8 @@
 
 The wave runs as blocks of the force launch in small scenes and as a launch of
 its own otherwise; a profiled step always launches it by itself.  Both must
-give the same state to the bit."""
+give the same state to the bit.  Small scans take one launch, larger ones and
+scans in place two or more."""
 import numpy as np
 import pytest
 
@@ -37,3 +38,21 @@ def test_wave_in_the_force_launch(gpu, cwa, n, W, H, band):
             states.append(s.readback())
             states[-1]["colflux"] = s.grid_host()["colflux"]
     _same(*states, (n, W, H, band))
+
+
+@pytest.mark.parametrize("n", [1, 8191, 8192, 8193, 65_535, 65_536, 65_537])
+@pytest.mark.parametrize("form", ["apart", "misaligned", "in place"])
+def test_scan_in_one_launch(gpu, cwa, n, form):
+    import torch
+    from coupledwateranimation_amd import _lib
+
+    print(f"scan n={n} {form}", flush=True)
+    x = np.random.default_rng(n).integers(0, 40, n).astype(np.int32)
+    buf = torch.zeros(n + 8, dtype=torch.int32, device=gpu)
+    src = buf[1:n + 1] if form == "misaligned" else buf[:n]
+    src.copy_(torch.from_numpy(x))
+    out = buf if form == "in place" else torch.full((n + 1,), -1, dtype=torch.int32, device=gpu)
+    _lib.check(cwa.lib().cwa_scan_exclusive_i32(src.data_ptr(), out.data_ptr(), n, None))
+    assert np.array_equal(out[:n + 1].cpu().numpy(), np.concatenate([[0], np.cumsum(x)]))
+    if form != "in place":
+        assert np.array_equal(src.cpu().numpy(), x)
