@@ -1078,6 +1078,134 @@ __device__ __forceinline__ void wave_tile(const DevParams& P, const WaveTiles& w
     else wave_single(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
 }
 
+// What the force pass writes (fpre: only for the adjoint tape).
+struct ForceOut {
+    float4* __restrict__ pos;
+    float4* __restrict__ vel;
+    float4* __restrict__ force;
+    int* __restrict__ id;
+    float* __restrict__ rho;
+    float* __restrict__ prs;
+    float4* __restrict__ fpre;
+};
+
+// What a particle needs after its neighbour sums, loaded where it is used:
+// the surface above it and beside it, its density and id.
+struct LateInputs {
+    const DevParams& P;
+    const float* __restrict__ H0;
+    const float* __restrict__ rho_w;
+    const int* __restrict__ bid;
+    float u, v;
+    int i;
+    __device__ __forceinline__ float height() const { return tex_sample(H0, P.W, P.H, u, v); }
+    __device__ __forceinline__ float east_du() const {
+        return tex_sample(H0, P.W, P.H, u + P.du, v);
+    }
+    __device__ __forceinline__ float north_du() const {
+        return tex_sample(H0, P.W, P.H, u, v + P.du);
+    }
+    __device__ __forceinline__ float east() const { return tex_sample(H0, P.W, P.H, u + 1.0f, v); }
+    __device__ __forceinline__ float north() const { return tex_sample(H0, P.W, P.H, u, v + 1.0f); }
+    __device__ __forceinline__ float rho() const { return load_once(&rho_w[i]); }
+    __device__ __forceinline__ int id() const { return load_once(&bid[i]); }
+};
+
+// Everything of the force pass after the neighbour sums: crest, viscosity,
+// torque, drag and wave force, integration, foam, surface and boundary, and
+// the next step's cell key (returned; -1 with key null).
+template <class In>
+__device__ __forceinline__ int force_finish(const DevParams& P, float dt, int i, float4 pi,
+                                            float4 vi, float4 fp, float p_i, const PairAcc& a,
+                                            const In& in, const float* __restrict__ H0,
+                                            const ForceOut& o, int* __restrict__ key) {
+    float vfx = a.vfx, vfy = a.vfy, vfz = a.vfz;
+    if (pi.y > P.crest) {
+        fp.x /= P.brk_mass;
+        fp.y /= P.brk_mass;
+        fp.z /= P.brk_mass;
+        fp.w /= P.brk_mass;
+        vfx *= P.brk_visc;
+        vfy *= P.brk_visc;
+        vfz *= P.brk_visc;
+    }
+    vfx *= P.visc;
+    vfy *= P.visc;
+    vfz *= P.visc;
+    const float height = in.height();
+    float tqx = (pi.y * fp.z - pi.z * fp.y) * P.torque;
+    float tqy = (pi.z * fp.x - pi.x * fp.z) * P.torque;
+    float tqz = (pi.x * fp.y - pi.y * fp.x) * P.torque;
+    float drx = 0.f, dry = 0.f, drz = 0.f, wfx = 0.f, wfy = 0.f, wfz = 0.f;
+    if (coupled(P, pi.y, height)) {
+        // WaveVelocity (force_comp.glsl:117-128)
+        const float hx = in.east_du();
+        const float hy = in.north_du();
+        const float wvx = (hx - height) / dt, wvy = (hy - height) / dt, wvz = (hx - hy) / P.du;
+        drx = -P.drag * (vi.x - wvx);
+        dry = -P.drag * (vi.y - wvy);
+        drz = -P.drag * (vi.z - wvz);
+        // WaveNormal (force_comp.glsl:131-139) = (H(u+1)-H, H(v+1)-H, -1)
+        const float nx = in.east() - height;
+        const float ny = in.north() - height;
+        wfx = -height * nx * P.wforce;
+        wfy = -height * ny * P.wforce;
+        wfz = -height * -1.0f * P.wforce;
+    }
+    float rho = in.rho();
+    float prs = p_i;
+    float Fx = a.pfx + vfx + rho * P.g[0] + tqx + drx + wfx;
+    float Fy = a.pfy + vfy + rho * P.g[1] + tqy + dry + wfy;
+    float Fz = a.pfz + vfz + rho * P.g[2] + tqz + drz + wfz;
+    float Fw = fp.w;
+    if (o.fpre) o.fpre[i] = make_float4(Fx, Fy, Fz, 0.0f);  // taped for the adjoint
+
+    // integrate_comp.glsl:56-92
+    float nvx = vi.x + dt * (Fx / rho), nvy = vi.y + dt * (Fy / rho), nvz = vi.z + dt * (Fz / rho);
+    float npx = pi.x + dt * nvx, npy = pi.y + dt * nvy, npz = pi.z + dt * nvz;
+    const float damp = 1.0f - P.vdamp * dt;
+    nvx *= damp;
+    nvy *= damp;
+    nvz *= damp;
+    if (sqrtf(dist2_fma(nvx, nvy, nvz)) > P.foam_speed) {
+        Fx *= P.foam_f;
+        Fy *= P.foam_f;
+        Fz *= P.foam_f;
+        Fw *= P.foam_f;
+        rho *= P.foam_rho;
+        prs *= P.foam_p;
+        nvx *= P.foam_v;
+        nvy *= P.foam_v;
+        nvz *= P.foam_v;
+    }
+    const float th = tex_sample(H0, P.W, P.H, (npx - P.org[0]) * P.uvs[0],
+                                (npz - P.org[1]) * P.uvs[1]);
+    if (npy < th) npy = th - P.rp;
+    // CheckBoundary (integrate_comp.glsl:135-178)
+    if (npx < P.lo[0]) { npx = P.lo[0]; nvx *= -P.bounce; }
+    else if (npx > P.up[0]) { npx = P.up[0]; nvx *= -P.bounce; }
+    if (npy < P.lo[1]) { npy = P.lo[1]; nvy *= -P.bounce; }
+    else if (npy > P.up[1]) { npy = P.up[1]; nvy *= -P.bounce; }
+    if (npz < P.lo[2]) { npz = P.lo[2]; nvz *= -P.bounce; }
+    else if (npz > P.up[2]) { npz = P.up[2]; nvz *= -P.bounce; }
+    if (P.wake) {
+        if (npy > P.up[1] + P.ceil_extra) { npy = P.up[1] + P.ceil_extra; nvy *= -P.bounce; }
+    }
+    o.pos[i] = make_float4(npx, npy, npz, pi.w);
+    o.vel[i] = make_float4(nvx, nvy, nvz, vi.w);
+    o.force[i] = make_float4(Fx, Fy, Fz, Fw);
+    o.id[i] = in.id();
+    store_once(&o.rho[i], rho);  // not read by the next step (A/B: step -0.7 %)
+    store_once(&o.prs[i], prs);
+    if (!key) return -1;
+    const int ix = cell_axis(npx, P.gmin[0], P.cell, P.dims[0]);
+    const int iy = cell_axis(npy, P.gmin[1], P.cell_y, P.dims[1]);
+    const int iz = cell_axis(npz, P.gmin[2], P.cell, P.dims[2]);
+    const int cell = lin_cell(P.dims, ix, iy, iz);
+    key[i] = cell;
+    return cell;
+}
+
 // ---------------------------------------------------------------------------
 // Forces (force_comp.glsl:62-139) fused with symplectic Euler + boundary
 // (integrate_comp.glsl:56-92, 135-178).  Visits only the neighbours the
@@ -1102,10 +1230,7 @@ __global__ void __launch_bounds__(256) k_force_integrate(
     const float4* __restrict__ force, const int* __restrict__ list,
     const int* __restrict__ offset, int n, const float* __restrict__ rho_w,
     const uint2* __restrict__ nbw, const float4* __restrict__ nrec,
-    const float* __restrict__ H0, float4* __restrict__ pos_o,
-    float4* __restrict__ vel_o, float4* __restrict__ force_o, int* __restrict__ id_o,
-    float* __restrict__ rho_o, float* __restrict__ prs_o, float4* __restrict__ fpre, int nfb,
-    const float* __restrict__ pflux, float* __restrict__ colflux, NextKeys next, WaveTiles wt) {
+    const float* __restrict__ H0, ForceOut out, int nfb, const float* __restrict__ pflux, float* __restrict__ colflux, NextKeys next, WaveTiles wt) {
     const DevParams& P = *Pd;
     __shared__ uint2 s_nb[kNbStage][256];
     static_assert(sizeof(s_nb) >= kWaveTileColumns * sizeof(float), "a tile's column sums");
@@ -1175,93 +1300,10 @@ __global__ void __launch_bounds__(256) k_force_integrate(
                 force_pair(h, pi, vi, p_i, m_spiky_half, m_lap, load_nbr(nrec, j), a);
             });
         }
-        float vfx = a.vfx, vfy = a.vfy, vfz = a.vfz;
-        if (pi.y > P.crest) {
-            fp.x /= P.brk_mass;
-            fp.y /= P.brk_mass;
-            fp.z /= P.brk_mass;
-            fp.w /= P.brk_mass;
-            vfx *= P.brk_visc;
-            vfy *= P.brk_visc;
-            vfz *= P.brk_visc;
-        }
-        vfx *= P.visc;
-        vfy *= P.visc;
-        vfz *= P.visc;
         const float u = (pi.x - P.org[0]) * P.uvs[0];
         const float v = (pi.z - P.org[1]) * P.uvs[1];
-        const float height = tex_sample(H0, P.W, P.H, u, v);
-        float tqx = (pi.y * fp.z - pi.z * fp.y) * P.torque;
-        float tqy = (pi.z * fp.x - pi.x * fp.z) * P.torque;
-        float tqz = (pi.x * fp.y - pi.y * fp.x) * P.torque;
-        float drx = 0.f, dry = 0.f, drz = 0.f, wfx = 0.f, wfy = 0.f, wfz = 0.f;
-        if (coupled(P, pi.y, height)) {
-            // WaveVelocity (force_comp.glsl:117-128)
-            const float hx = tex_sample(H0, P.W, P.H, u + P.du, v);
-            const float hy = tex_sample(H0, P.W, P.H, u, v + P.du);
-            const float wvx = (hx - height) / dt, wvy = (hy - height) / dt, wvz = (hx - hy) / P.du;
-            drx = -P.drag * (vi.x - wvx);
-            dry = -P.drag * (vi.y - wvy);
-            drz = -P.drag * (vi.z - wvz);
-            // WaveNormal (force_comp.glsl:131-139) = (H(u+1)-H, H(v+1)-H, -1)
-            const float nx = tex_sample(H0, P.W, P.H, u + 1.0f, v) - height;
-            const float ny = tex_sample(H0, P.W, P.H, u, v + 1.0f) - height;
-            wfx = -height * nx * P.wforce;
-            wfy = -height * ny * P.wforce;
-            wfz = -height * -1.0f * P.wforce;
-        }
-        float rho = load_once(&rho_w[i]);
-        float prs = p_i;
-        float Fx = a.pfx + vfx + rho * P.g[0] + tqx + drx + wfx;
-        float Fy = a.pfy + vfy + rho * P.g[1] + tqy + dry + wfy;
-        float Fz = a.pfz + vfz + rho * P.g[2] + tqz + drz + wfz;
-        float Fw = fp.w;
-        if (fpre) fpre[i] = make_float4(Fx, Fy, Fz, 0.0f);  // taped for the adjoint
-
-        // integrate_comp.glsl:56-92
-        float nvx = vi.x + dt * (Fx / rho), nvy = vi.y + dt * (Fy / rho), nvz = vi.z + dt * (Fz / rho);
-        float npx = pi.x + dt * nvx, npy = pi.y + dt * nvy, npz = pi.z + dt * nvz;
-        const float damp = 1.0f - P.vdamp * dt;
-        nvx *= damp;
-        nvy *= damp;
-        nvz *= damp;
-        if (sqrtf(dist2_fma(nvx, nvy, nvz)) > P.foam_speed) {
-            Fx *= P.foam_f;
-            Fy *= P.foam_f;
-            Fz *= P.foam_f;
-            Fw *= P.foam_f;
-            rho *= P.foam_rho;
-            prs *= P.foam_p;
-            nvx *= P.foam_v;
-            nvy *= P.foam_v;
-            nvz *= P.foam_v;
-        }
-        const float th = tex_sample(H0, P.W, P.H, (npx - P.org[0]) * P.uvs[0],
-                                    (npz - P.org[1]) * P.uvs[1]);
-        if (npy < th) npy = th - P.rp;
-        // CheckBoundary (integrate_comp.glsl:135-178)
-        if (npx < P.lo[0]) { npx = P.lo[0]; nvx *= -P.bounce; }
-        else if (npx > P.up[0]) { npx = P.up[0]; nvx *= -P.bounce; }
-        if (npy < P.lo[1]) { npy = P.lo[1]; nvy *= -P.bounce; }
-        else if (npy > P.up[1]) { npy = P.up[1]; nvy *= -P.bounce; }
-        if (npz < P.lo[2]) { npz = P.lo[2]; nvz *= -P.bounce; }
-        else if (npz > P.up[2]) { npz = P.up[2]; nvz *= -P.bounce; }
-        if (P.wake) {
-            if (npy > P.up[1] + P.ceil_extra) { npy = P.up[1] + P.ceil_extra; nvy *= -P.bounce; }
-        }
-        pos_o[i] = make_float4(npx, npy, npz, pi.w);
-        vel_o[i] = make_float4(nvx, nvy, nvz, vi.w);
-        force_o[i] = make_float4(Fx, Fy, Fz, Fw);
-        id_o[i] = load_once(&bid[i]);
-        store_once(&rho_o[i], rho);  // not read by the next step (A/B: step -0.7 %)
-        store_once(&prs_o[i], prs);
-        if (next.key) {
-            const int ix = cell_axis(npx, P.gmin[0], P.cell, P.dims[0]);
-            const int iy = cell_axis(npy, P.gmin[1], P.cell_y, P.dims[1]);
-            const int iz = cell_axis(npz, P.gmin[2], P.cell, P.dims[2]);
-            cell = lin_cell(P.dims, ix, iy, iz);
-            next.key[i] = cell;
-        }
+        const LateInputs in{P, H0, rho_w, bid, u, v, i};
+        cell = force_finish(P, dt, i, pi, vi, fp, p_i, a, in, H0, out, next.key);
     }  // valid
     if (next.key) push_runs<true, kLink>(cell, valid, i, next.runs);
 }
@@ -1467,10 +1509,10 @@ hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bp
     const auto kernel = wt.nblk ? k_force_integrate<true, true>
                         : link  ? k_force_integrate<true, false>
                                 : k_force_integrate<false, false>;
+    const ForceOut out{N.pos, N.vel, N.force, N.id, rho, prs, fpre};
     kernel<<<wt.nblk + nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list, offset,
-                                                n, rho_w, nbw, nrec, H0, N.pos, N.vel, N.force,
-                                                N.id, rho, prs, fpre, nfb, flux, colflux, next,
-                                                wt);
+                                                n, rho_w, nbw, nrec, H0, out, nfb, flux, colflux,
+                                                next, wt);
     return hipGetLastError();
 }
 
