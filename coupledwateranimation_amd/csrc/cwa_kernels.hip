@@ -1308,6 +1308,160 @@ __global__ void __launch_bounds__(256) k_force_integrate(
     if (next.key) push_runs<true, kLink>(cell, valid, i, next.runs);
 }
 
+// The force pass of scenes of up to kForceSplitMax particles (and
+// lane_split_limit()): kForceSplit consecutive lanes per particle.  There the
+// pass is one chain of latencies per wave: own record and words, then the
+// neighbours a few at a time, then the surface samples and the stores.  So
+// each lane takes the neighbours whose word bits are its own mod kForceSplit,
+// kSplitBatch records in flight; the first words are loaded without waiting
+// for their count; and everything the end needs (the surface samples, each by
+// one lane of the group, density, id) is loaded before the neighbours.  The
+// group's sums are added in a fixed tree and its first lane finishes the
+// particle.
+// MI355X, one lane -> four, three scenes in flight / alone: 4 096 particles 13.6
+// / 39.0 -> 12.2 / 34.8 us a step, 20 011 (eager) 42.0 -> 37.2 alone, 30 000
+// 15.7 / 38.9 -> 15.3 / 33.8; 65 536 24.3 -> 25.8, 120 000 34.1 -> 37.4 and
+// 240 000 60.1 -> 70.3 in flight, where the chip has enough waves without it.
+constexpr int kForceSplit = 4;
+constexpr int kSplitWords = 8;  // words loaded ahead of their count
+constexpr int kSplitBatch = 8;
+
+template <int kSrc>
+__device__ __forceinline__ float quad_bcast_f(float v) {
+    return __int_as_float(quad_bcast<kSrc>(__float_as_int(v)));
+}
+
+// What force_finish reads, all of it already loaded.
+struct EarlyInputs {
+    float h, hx, hy, h1x, h1y, r;
+    int own_id;
+    __device__ __forceinline__ float height() const { return h; }
+    __device__ __forceinline__ float east_du() const { return hx; }
+    __device__ __forceinline__ float north_du() const { return hy; }
+    __device__ __forceinline__ float east() const { return h1x; }
+    __device__ __forceinline__ float north() const { return h1y; }
+    __device__ __forceinline__ float rho() const { return r; }
+    __device__ __forceinline__ int id() const { return own_id; }
+};
+
+template <bool kLink, bool kWave>
+__global__ void __launch_bounds__(256) k_force_split(
+    const DevParams* __restrict__ Pd, float dt, const float4* __restrict__ bpos,
+    const int* __restrict__ bid, const float* __restrict__ vpad,
+    const float4* __restrict__ force, const int* __restrict__ list,
+    const int* __restrict__ offset, int n, const float* __restrict__ rho_w,
+    const uint2* __restrict__ nbw, const float4* __restrict__ nrec,
+    const float* __restrict__ H0, ForceOut out, int nfb, const float* __restrict__ pflux,
+    float* __restrict__ colflux, NextKeys next, WaveTiles wt) {
+    const DevParams& P = *Pd;
+    __shared__ uint2 s_nb[kNbStage][256];
+    if (kWave && (int)blockIdx.x < wt.nblk) {
+        wave_tile(P, wt, blockIdx.x, offset, colflux ? pflux : nullptr, dt,
+                  reinterpret_cast<float*>(&s_nb[0][0]));
+        return;
+    }
+    const int blk = (int)blockIdx.x - (kWave ? wt.nblk : 0);
+    if (blk >= nfb) {
+        column_flux_sum(offset, pflux, P.dims[0], P.dims[1], P.dims[2], colflux,
+                        ((blk - nfb) * (int)blockDim.x + (int)threadIdx.x) >> 6,
+                        threadIdx.x & 63);
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int sub = threadIdx.x & (kForceSplit - 1);
+    const int i = (blk * 256 + (int)threadIdx.x) / kForceSplit;  // a group shares i
+    int cell = -1;
+    if (i < n) {
+        const int nw_all = load_once(&nb_count(nbw, n)[i]);
+        uint2 w[kSplitWords];
+#pragma unroll
+        for (int k = 0; k < kSplitWords; ++k) w[k] = nbw[(size_t)k * n + i];
+        const float4 own_a = nrec[2 * (size_t)i];      // (x, y, z, p)
+        const float4 own_b = nrec[2 * (size_t)i + 1];  // (vx, vy, vz, 1/rho)
+        const int src = list[i];
+        const float pad = bpos[i].w, vw = vpad[i];
+        EarlyInputs in;
+        in.r = rho_w[i];
+        in.own_id = bid[i];
+        const float4 fp = force[src];
+        const float4 pi = make_float4(own_a.x, own_a.y, own_a.z, pad);
+        const float4 vi = make_float4(own_b.x, own_b.y, own_b.z, vw);
+        // the surface: above the particle, and the sample of this lane
+        const float u = (pi.x - P.org[0]) * P.uvs[0];
+        const float v = (pi.z - P.org[1]) * P.uvs[1];
+        const float du = (sub & 2) ? 1.0f : P.du;
+        const TexTaps here = tex_taps(H0, P.W, P.H, u, v);
+        const TexTaps mine = tex_taps(H0, P.W, P.H, (sub & 1) ? u : u + du, (sub & 1) ? v + du : v);
+        const float p_i = own_a.w;
+        const float h = P.h;
+        const float m_spiky_half = P.m * P.spiky * 0.5f;
+        const float m_lap = P.m * P.lap;
+        PairAcc a{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (nw_all >= 0) {
+            // this lane's bits of the particle's words, the empty ones left out
+            uint2* st = &s_nb[0][threadIdx.x];
+            const uint32_t own_bits = 0x11111111u << sub;
+            int nw = 0;
+#pragma unroll
+            for (int k = 0; k < kSplitWords; ++k) {
+                const uint32_t bits = k < nw_all ? w[k].x & own_bits : 0u;
+                if (bits) st[256 * nw++] = make_uint2(bits, w[k].y);
+            }
+            for (int k = kSplitWords; k < nw_all; ++k) {
+                const uint2 x = nbw[(size_t)k * n + i];
+                if (x.x & own_bits) st[256 * nw++] = make_uint2(x.x & own_bits, x.y);
+            }
+            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+            NbCursor nb(st, 256, nw);
+            for (;;) {
+                int j[kSplitBatch];
+                j[0] = nb.next();
+                if (j[0] < 0) break;
+#pragma unroll
+                for (int q = 1; q < kSplitBatch; ++q) j[q] = nb.next();
+                Nbr r[kSplitBatch];
+#pragma unroll
+                for (int q = 0; q < kSplitBatch; ++q) {
+                    r[q] = Nbr{zero, zero};
+                    if (j[q] >= 0) r[q] = load_nbr(nrec, j[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < kSplitBatch; ++q) {
+                    const bool live = j[q] >= 0;
+                    force_pair(h, pi, vi, p_i, live ? m_spiky_half : 0.0f, live ? m_lap : 0.0f,
+                               r[q], a);
+                }
+            }
+        } else {
+            int t = 0;
+            for_each_candidate_neighbour(P, offset, bpos, i, pi, [&](int j) {
+                if ((t++ & (kForceSplit - 1)) == sub)
+                    force_pair(h, pi, vi, p_i, m_spiky_half, m_lap, load_nbr(nrec, j), a);
+            });
+        }
+        a.pfx = quad_sum(a.pfx);
+        a.pfy = quad_sum(a.pfy);
+        a.pfz = quad_sum(a.pfz);
+        a.vfx = quad_sum(a.vfx);
+        a.vfy = quad_sum(a.vfy);
+        a.vfz = quad_sum(a.vfz);
+        const float s = mine.value();
+        in.h = here.value();
+        in.hx = quad_bcast_f<0>(s);
+        in.hy = quad_bcast_f<1>(s);
+        in.h1x = quad_bcast_f<2>(s);
+        in.h1y = quad_bcast_f<3>(s);
+        if (sub == 0) cell = force_finish(P, dt, i, pi, vi, fp, p_i, a, in, H0, out, next.key);
+    }
+    if (next.key) {
+        // the wave's 16 particles on its first lanes, in slot order
+        constexpr int kPer = 64 / kForceSplit;
+        cell = __shfl(cell, (lane * kForceSplit) & 63, 64);
+        if (lane >= kPer) cell = -1;
+        push_runs<true, kLink>(cell, cell >= 0, i - lane / kForceSplit + lane, next.runs);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Neighbour count of every slot as the last density pass found it (the
 // particle itself included, as the density sum of rho_pres_comp.glsl:60-68
@@ -1501,14 +1655,16 @@ hipError_t launch_force_integrate(const DevParams& P, float dt, const float4* bp
                                   float* colflux, const float* vpad, const NextKeys& next,
                                   const WaveTiles& wt, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    const int nfb = blocks_for(n, 256);
     const long long ncol = colflux ? (long long)P.dims[0] * P.dims[2] : 0;
     const int ncb = blocks_for(ncol * 64, 256);
     const bool link = next.runs.head != nullptr;
     if (wt.nblk && !link) return hipErrorInvalidValue;  // kFuseWaveParticles <= kFuseLinksMax
-    const auto kernel = wt.nblk ? k_force_integrate<true, true>
-                        : link  ? k_force_integrate<true, false>
-                                : k_force_integrate<false, false>;
+    const bool split = link && n <= kForceSplitMax && n <= lane_split_limit();
+    const int nfb = blocks_for(split ? (long long)n * kForceSplit : n, 256);
+    const auto kernel = split     ? (wt.nblk ? k_force_split<true, true> : k_force_split<true, false>)
+                        : wt.nblk ? k_force_integrate<true, true>
+                        : link    ? k_force_integrate<true, false>
+                                  : k_force_integrate<false, false>;
     const ForceOut out{N.pos, N.vel, N.force, N.id, rho, prs, fpre};
     kernel<<<wt.nblk + nfb + ncb, 256, 0, st>>>(P.dev, dt, bpos, bid, vpad, S.force, list, offset,
                                                 n, rho_w, nbw, nrec, H0, out, nfb, flux, colflux,

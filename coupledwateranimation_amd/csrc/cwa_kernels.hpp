@@ -77,8 +77,9 @@ hipError_t launch_box_pairs(const float4* x, const float4* hw, int n, const floa
 // vel_out (the sorted velocities) are optional outputs for the adjoint tape
 // (null: not written).
 // Scenes of up to this many particles run the density pass (and a tape's
-// pair adjoint) with four lanes per particle, larger ones with one lane;
-// read at each density launch and at tape creation.  Default kLaneSplitDefault.
+// pair adjoint, and up to kForceSplitMax the force pass) with four lanes per
+// particle, larger ones with one lane; read at each launch and at tape
+// creation.  Default kLaneSplitDefault.
 constexpr long long kLaneSplitDefault = 1 << 18;
 long long lane_split_limit();
 long long set_lane_split_limit(long long max_n);  // returns the previous limit
@@ -108,6 +109,10 @@ static_assert(kFuseWaveParticles <= kFuseLinksMax, "tiles go with the fused run 
 // n particles; flux: the step couples (the tiles sum the columns they sample).
 WaveTiles wave_tiles_for(const DevParams& P, int n, bool flux, const float* h0, const float* h1,
                          float* out);
+// Scenes of up to this many particles (and lane_split_limit()) run the force
+// pass with four lanes per particle (k_force_split gives both sides' times).
+constexpr int kForceSplitMax = 1 << 15;
+static_assert(kForceSplitMax <= kFuseLinksMax, "the split force pass lists its runs");
 // Forces + integration: own record from nrec, id from bid and the velocity
 // pad from vpad (sorted), previous force from the state S in its pre-sort
 // slot list[i]; writes the next state N in sorted order.  The launch also

@@ -56,3 +56,46 @@ def test_scan_in_one_launch(gpu, cwa, n, form):
     assert np.array_equal(out[:n + 1].cpu().numpy(), np.concatenate([[0], np.cumsum(x)]))
     if form != "in place":
         assert np.array_equal(src.cpu().numpy(), x)
+
+
+def _scene_state(cwa, spec, pos, vel, force, limit, steps):
+    from coupledwateranimation_amd.scene import set_lane_split_limit
+
+    old = set_lane_split_limit(limit)
+    try:
+        with cwa.Scene(spec.params, pos, vel, force, spec.wave_size, spec.height0,
+                       spec.height1) as s:
+            s.step(spec.dt, steps)
+            return s.readback(), s.grid_host()
+    finally:
+        set_lane_split_limit(old)
+
+
+@pytest.mark.parametrize("n,shape", [(1, "block"), (15, "block"), (16, "block"), (17, "block"),
+                                     (63, "block"), (65, "block"), (4097, "block"),
+                                     (2000, "dense"), (32_768, "block"), (32_769, "block")])
+def test_force_with_four_lanes(gpu, cwa, n, shape):
+    """Four lanes per particle against one: the same terms in another order.
+    With up to 64 neighbours a sum of 64 terms, each order within
+    64 * 2^-24 of the terms' total; twice that, for terms that add up to no
+    more than four times the largest force."""
+    from coupledwateranimation_amd import configs
+
+    print(f"force lanes n={n} {shape}", flush=True)
+    spec = configs.dam_break_diff(max(n, 64), 96, 7)
+    rng = np.random.default_rng(n)
+    pos = spec.pos[:n].copy()
+    if shape == "dense":  # every column longer than 64 candidates: the re-search
+        pos[:, :3] = 0.4 + rng.uniform(0.0, 2.0 * spec.params.h, (n, 3))
+    vel, force = np.zeros_like(pos), np.zeros_like(pos)
+    vel[:, :3] = rng.normal(0.0, 0.3, (n, 3))
+    force[:, :3] = rng.normal(0.0, 5.0, (n, 3))
+    (a, _), (b, _) = [_scene_state(cwa, spec, pos, vel, force, k, 1) for k in (-1, 0)]
+    terms = 64 if shape == "block" else n
+    tol = 4 * 2 * terms * 2.0 ** -24
+    for k in ("force", "vel", "pos"):
+        assert np.abs(a[k] - b[k]).max() <= tol * np.abs(b[k]).max(), k
+    # the next grid, from the keys and run lists the pass leaves
+    _, g = _scene_state(cwa, spec, pos, vel, force, -1, 3)
+    assert np.array_equal(g["list"], np.argsort(g["key"], kind="stable"))
+    assert np.array_equal(g["count"], np.bincount(g["key"], minlength=g["count"].size))
