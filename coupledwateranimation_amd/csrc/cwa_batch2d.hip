@@ -20,17 +20,25 @@
 //   scan         exclusive offsets over all cells (cwa_kernels.hip)
 //   k2_scatter   run records into each cell's segment
 //   k2_reorder   stable rank from the run records; state A -> B, sorted
-//   k2_density   persistent, tile queues; B -> q, (rho, p), (p/rho^2, 1/rho)
-//   k2_force     persistent, tile queues; q -> A (forward Euler)
+//   k2_density   tiles; B -> q, (rho, p), (p/rho^2, 1/rho)
+//   k2_force     tiles; q -> A (forward Euler)
 //   k2_wave      one workgroup per scene: column flux sums, the wave
 //                substeps in LDS, flux source; levels updated in place
 // The state ends every step in A, so a captured step replays as is.
 //
-// Tiles.  A tile is up to one block of consecutive slots of one scene.
-// Scenes are bound to per-XCD queues by longest-processing-time
-// assignment of their cost (n_s^2: neighbours per particle grow with n_s in
-// a fixed box); blocks take tiles from their XCD's queue (workgroup i runs
-// on XCD i mod 8) and steal from the other queues when it is empty.
+// Tiles.  A tile is up to one block of consecutive slots of one scene.  Workgroup
+// i runs on XCD i mod 8, so entry e of the tile table belongs to XCD e mod 8:
+// scenes, the costly ones cut into pieces, are bound to XCDs by longest-
+// processing-time assignment of their cost (neighbours per particle grow with
+// n_s in a fixed box), costly tiles first.  With one block per tile, block e
+// takes entry e, and the hardware hands out the blocks of an XCD as its CUs free
+// up.  Fewer, persistent blocks take their XCD's entries from a queue counter
+// and then the other XCDs' (static shares left them unbalanced: 256 scenes at
+// 1 024 blocks of 512, density 803 -> 972 us).  The counter is a serial chain of
+// atomics, which bound the passes when every tile came from it (MI355X, one
+// block of 256 per tile, queue -> table: 256 scenes of 4 M particles, density
+// 1 099 -> 700 us, force 1 558 -> 1 310; 100 scenes of 678 000, 139 -> 54 and
+// 173 -> 91; 24 scenes of 20 000, 17.0 -> 14.0 and 20.8 -> 17.3).
 //
 // Arithmetic follows the float restatement of the oracle
 // (oracle/cwa_oracle2d.hpp) expression by expression, with contraction
@@ -59,7 +67,8 @@ int guarded_call(void (*fn)(void*), void* ctx);
 
 namespace b2d {
 
-constexpr int kNumQueues = 8;   // XCDs of an MI355X
+constexpr int kNumXcd = 8;      // XCDs of an MI355X
+constexpr int kPiecesPerXcd = 8;  // a scene is cut into pieces of at most this share of an XCD
 // Candidates loaded ahead in the density / force loops (the lanes of a tile
 // walk the same candidates, so each load is one address per wave).  Measured
 // on the 256-scene workload (MI355X), cells of H: density 1, 2, 4, 6, 8, 16 ->
@@ -258,9 +267,8 @@ __device__ __forceinline__ void column_rows(const Dev2& P, const int* __restrict
 __global__ void __launch_bounds__(256)
     k2_hash(Dev2 P, const Scene2D* __restrict__ sc, const int* __restrict__ blk_scene,
             const float4* __restrict__ xv, int ntot, int* __restrict__ key,
-            int* __restrict__ rec, int* __restrict__ count, int* __restrict__ queues,
-            int nqueue_words) {
-    if (blockIdx.x == 0 && (int)threadIdx.x < nqueue_words) queues[threadIdx.x] = 0;
+            int* __restrict__ rec, int* __restrict__ count, int* __restrict__ queues) {
+    if (blockIdx.x == 0 && (int)threadIdx.x < 2 * kNumXcd) queues[threadIdx.x] = 0;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     const bool valid = i < ntot;
@@ -330,43 +338,51 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------------------
-// tile queues
+// tiles
 // ---------------------------------------------------------------------------
-// Next tile for a block whose home queue is `home`: its own queue first,
-// then the others in order.  Every queue is finite, so every block ends.
-__device__ __forceinline__ int next_tile(int* __restrict__ queue, const int* __restrict__ qbeg,
-                                         int nq, int home) {
-    for (int k = 0; k < nq; ++k) {
+struct TileTable {
+    const int4* entry;  // scene (-1: none), first slot, end slot
+    int n;              // entries, a multiple of nq
+    int nq;             // XCDs the entries are dealt to in turn
+    int* queue;         // persistent blocks: entries of each XCD already taken,
+    const int* len;     // and how many it has (the others of its n / nq are empty)
+};
+
+// Next entry of a persistent block: its XCD's first, then the others' in
+// order.  Every queue is finite, so every block ends.
+__device__ __forceinline__ int next_entry(const TileTable& T) {
+    const int home = (int)(blockIdx.x % T.nq);
+    for (int k = 0; k < T.nq; ++k) {
         int q = home + k;
-        if (q >= nq) q -= nq;
-        const int cnt = qbeg[q + 1] - qbeg[q];
-        if (cnt == 0) continue;
-        if (__hip_atomic_load(&queue[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt)
+        if (q >= T.nq) q -= T.nq;
+        const int cnt = T.len[q];
+        if (__hip_atomic_load(&T.queue[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt)
             continue;
-        const int idx = atomicAdd(&queue[q], 1);
-        if (idx < cnt) return qbeg[q] + idx;
+        const int idx = atomicAdd(&T.queue[q], 1);
+        if (idx < cnt) return idx * T.nq + q;
     }
     return -1;
 }
 
-struct TileRef {
-    int scene, beg, end;
-};
-
-template <int BS>
-__device__ __forceinline__ bool fetch_tile(int* __restrict__ queue, const int* __restrict__ qbeg,
-                                           const int4* __restrict__ tiles, int nq,
-                                           int* s_tile, TileRef& t) {
-    if (threadIdx.x == 0) s_tile[0] = next_tile(queue, qbeg, nq, (int)(blockIdx.x % nq));
-    __syncthreads();
-    const int id = __builtin_amdgcn_readfirstlane(s_tile[0]);
-    __syncthreads();
-    if (id < 0) return false;
-    const int4 d = tiles[id];
-    t.scene = __builtin_amdgcn_readfirstlane(d.x);
-    t.beg = __builtin_amdgcn_readfirstlane(d.y);
-    t.end = __builtin_amdgcn_readfirstlane(d.z);
-    return true;
+// Runs body(tile) for the block's tiles: entry blockIdx.x, or with
+// kPersistent the entries the block takes from the queues.
+template <bool kPersistent, class Body>
+__device__ __forceinline__ void for_each_tile(const TileTable& T, Body&& body) {
+    if (!kPersistent) {
+        const int4 t = T.entry[blockIdx.x];
+        if (t.x >= 0) body(t);
+        return;
+    }
+    __shared__ int s_entry;
+    for (;;) {
+        if (threadIdx.x == 0) s_entry = next_entry(T);
+        __syncthreads();
+        const int e = __builtin_amdgcn_readfirstlane(s_entry);
+        __syncthreads();
+        if (e < 0) return;
+        const int4 t = T.entry[e];
+        body(t);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -374,10 +390,7 @@ __device__ __forceinline__ bool fetch_tile(int* __restrict__ queue, const int* _
 // ---------------------------------------------------------------------------
 struct DensityArgs {
     const Scene2D* sc;
-    const int4* tiles;
-    const int* qbeg;
-    int* queue;
-    int nq;
+    TileTable tiles;
     const float4* xvB;
     const float2* rpB;
     const int* idfB;
@@ -391,14 +404,12 @@ struct DensityArgs {
     float* flux;
 };
 
-template <int BS>
+template <int BS, bool kPersistent>
 __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A) {
-    __shared__ int s_tile[1];
-    TileRef t;
-    while (fetch_tile<BS>(A.queue, A.qbeg, A.tiles, A.nq, s_tile, t)) {
-        const int i = t.beg + (int)threadIdx.x;
-        if (i >= t.end) continue;
-        const Scene2D S = A.sc[t.scene];
+    for_each_tile<kPersistent>(A.tiles, [&](const int4 t) {
+        const int i = t.y + (int)threadIdx.x;
+        if (i >= t.z) return;
+        const Scene2D S = A.sc[t.x];
         const float* w0 = A.h0 + S.wbeg;
         const float* w1 = A.h1 + S.wbeg;
         const float sL = (float)S.L / (P.hix - P.lox);
@@ -437,7 +448,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
         float rho = rp.x, p = rp.y;
         if (!(y > P.hiy)) {
             const int ix = cell2(x, P.lox, P.hc, P.nx);
-            const int cb = t.scene * P.ncell;
+            const int cb = t.x * P.ncell;
             float acc = 0.0f;
             for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
                 int b, e;
@@ -468,7 +479,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
         A.rpA[i] = make_float2(rho, p);
         A.aj[i] = make_float2(p / (rho * rho), 1.0f / rho);
         A.idfA[i] = (idf & ~(1 << 30)) | (en << 30);
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -476,10 +487,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
 // ---------------------------------------------------------------------------
 struct ForceArgs {
     const Scene2D* sc;
-    const int4* tiles;
-    const int* qbeg;
-    int* queue;
-    int nq;
+    TileTable tiles;
     const float4* q;
     const float2* aj;
     const int* idfA;
@@ -489,25 +497,23 @@ struct ForceArgs {
     float4* xvA;
 };
 
-template <int BS>
+template <int BS, bool kPersistent>
 __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
-    __shared__ int s_tile[1];
-    TileRef t;
-    while (fetch_tile<BS>(A.queue, A.qbeg, A.tiles, A.nq, s_tile, t)) {
-        const int i = t.beg + (int)threadIdx.x;
-        if (i >= t.end) continue;
+    for_each_tile<kPersistent>(A.tiles, [&](const int4 t) {
+        const int i = t.y + (int)threadIdx.x;
+        if (i >= t.z) return;
         const float4 qi = A.q[i];
         const float x = qi.x, y = qi.y, vx = qi.z, vy = qi.w;
         const int idf = A.idfA[i];
         if (((idf >> 30) & 1) == 0) {  // disabled: pass through (:494-498)
             A.xvA[i] = qi;
-            continue;
+            return;
         }
-        const Scene2D S = A.sc[t.scene];
+        const Scene2D S = A.sc[t.x];
         const float ai = A.aj[i].x;
         float apx = 0.0f, apy = 0.0f, avx = 0.0f, avy = 0.0f;
         const int ix = cell2(x, P.lox, P.hc, P.nx);
-        const int cb = t.scene * P.ncell;
+        const int cb = t.x * P.ncell;
         for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
             int b, e;
             column_rows(P, A.off, cb, x, y, ix, cx, b, e);
@@ -586,7 +592,7 @@ __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
         const float ay = apy + avy + P.gy + aty;
         const float v1x = vx + dt * ax, v1y = vy + dt * ay;
         A.xvA[i] = make_float4(x + dt * v1x, y + dt * v1y, v1x, v1y);
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -813,8 +819,8 @@ static const char* kNames[CWA2D_NUM_KERNELS] = {"hash", "scan", "scatter", "reor
 
 struct TileSet {
     DeviceBuffer<int4> tiles;
-    DeviceBuffer<int> qbeg;  // nq + 1
-    int ntiles = 0;
+    DeviceBuffer<int> len;  // entries per XCD
+    int ntiles = 0;  // table entries, empty ones included
 };
 
 class Batch2D {
@@ -911,14 +917,13 @@ class Batch2D {
         count_.resize(ncells_ + 1);
         offset_.resize(ncells_ + 1);
         ws_.resize(scan_workspace_ints(ncells_ + 1));
+        queue_.resize(2 * kNumXcd);
         h0_.resize(wtot_);
         h1_.resize(wtot_);
-        queue_.resize(2 * kNumQueues);
         finite_.resize(1);
         hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
         hip_check(hipMemset(offset_.get(), 0, sizeof(int) * (ncells_ + 1)), "offset zero");
         hip_check(hipMemset(key_.get(), 0, sizeof(int) * ntot_), "key zero");
-        hip_check(hipMemset(queue_.get(), 0, sizeof(int) * 2 * kNumQueues), "queue zero");
 
         tune_.block_density = 256;
         tune_.block_force = 256;
@@ -991,7 +996,7 @@ class Batch2D {
 
     // --- one step on the stream (optionally with events around kernels) ---
     void Step(float dt, bool profile) {
-        const int nq = tune_.xcd_queues ? kNumQueues : 1;
+        const int nq = tune_.xcd_queues ? kNumXcd : 1;
         const TileSet& td = Tiles(tune_.block_density, nq);
         const TileSet& tf = Tiles(tune_.block_force, nq);
         auto mark = [&](int slot, int which) {
@@ -1002,7 +1007,7 @@ class Batch2D {
             mark(B_HASH, first ? 0 : 2);
             k2_hash<<<blocks_for(ntot_, 256), 256, 0, st_>>>(
                 dev_, sc_.get(), blk_scene_.get(), xv_[0].get(), ntot_, key_.get(), rec_.get(),
-                count_.get(), queue_.get(), 2 * kNumQueues);
+                count_.get(), queue_.get());
             hip_check(hipGetLastError(), "hash");
             mark(B_HASH, first ? 1 : 3);
             mark(B_SCAN, first ? 0 : 2);
@@ -1021,17 +1026,15 @@ class Batch2D {
             hip_check(hipGetLastError(), "reorder");
             mark(B_REORDER, first ? 1 : 3);
 
-            DensityArgs da{sc_.get(), td.tiles.get(), td.qbeg.get(), queue_.get(), nq,
-                           xv_[1].get(), rp_[1].get(), idf_[1].get(), offset_.get(), h0_.get(),
+            DensityArgs da{sc_.get(), {td.tiles.get(), td.ntiles, nq, queue_.get(), td.len.get()}, xv_[1].get(), rp_[1].get(), idf_[1].get(), offset_.get(), h0_.get(),
                            h1_.get(), q_.get(), rp_[0].get(), aj_.get(), idf_[0].get(), flux_.get()};
             mark(B_DENSITY, first ? 0 : 2);
-            LaunchDensity(td, da, dt);
+            LaunchDensity(da, dt);
             mark(B_DENSITY, first ? 1 : 3);
-            ForceArgs fa{sc_.get(), tf.tiles.get(), tf.qbeg.get(), queue_.get() + kNumQueues, nq,
-                         q_.get(), aj_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
+            ForceArgs fa{sc_.get(), {tf.tiles.get(), tf.ntiles, nq, queue_.get() + kNumXcd, tf.len.get()}, q_.get(), aj_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
                          xv_[0].get()};
             mark(B_FORCE, first ? 0 : 2);
-            LaunchForce(tf, fa, dt);
+            LaunchForce(fa, dt);
             mark(B_FORCE, first ? 1 : 3);
         }
         mark(B_WAVE, 0);
@@ -1050,7 +1053,7 @@ class Batch2D {
         if (!graph_exec_ || graph_dt_ != dt) {
             InvalidateGraph();
             // tile tables allocate: build them before the capture
-            const int nq = tune_.xcd_queues ? kNumQueues : 1;
+            const int nq = tune_.xcd_queues ? kNumXcd : 1;
             Tiles(tune_.block_density, nq);
             Tiles(tune_.block_force, nq);
             hipGraph_t g = nullptr;
@@ -1295,68 +1298,87 @@ class Batch2D {
         }
     }
 
-    // Tiles of `bs` slots per scene, scenes bound to nq queues by LPT over
-    // n_s^2, tiles of each queue in decreasing scene cost.
+    // The tile table for blocks of `bs` slots, its entries dealt to nq XCDs in
+    // turn (1: one list in order of cost).
     const TileSet& Tiles(int bs, int nq) {
         const int key = bs * 16 + nq;
         auto it = tiles_.find(key);
         if (it != tiles_.end()) return it->second;
+        // a particle's cost: its neighbours grow with n_s, the rest does not
+        const auto cost = [&](int s) { return (double)host_sc_[s].n + 4096.0; };
+        double total = 0.0;
+        for (const Scene2D& S : host_sc_) total += (double)S.n * ((double)S.n + 4096.0);
+        const double most = std::max(total / (nq * kPiecesPerXcd), 1.0);
         std::vector<int> order(ns_);
         std::iota(order.begin(), order.end(), 0);
         std::stable_sort(order.begin(), order.end(),
                          [&](int a, int b) { return host_sc_[a].n > host_sc_[b].n; });
         std::vector<double> load(nq, 0.0);
-        std::vector<std::vector<int>> qs(nq);
+        std::vector<std::vector<int4>> per(nq);
         for (int s : order) {
-            const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-            load[q] += (double)host_sc_[s].n * (double)host_sc_[s].n;
-            qs[q].push_back(s);
-        }
-        std::vector<int4> tl;
-        std::vector<int> qb(nq + 1, 0);
-        for (int q = 0; q < nq; ++q) {
-            qb[q] = (int)tl.size();
-            for (int s : qs[q]) {
-                const Scene2D& S = host_sc_[s];
-                for (int b = S.pbeg; b < S.pbeg + S.n; b += bs)
-                    tl.push_back(make_int4(s, b, std::min(b + bs, S.pbeg + S.n), 0));
+            const Scene2D& S = host_sc_[s];
+            const int end = S.pbeg + S.n;
+            // whole tiles per piece
+            const int piece =
+                (int)std::min<double>((std::floor(most / (cost(s) * bs)) + 1.0) * bs, S.n);
+            for (int p = S.pbeg; p < end; p += piece) {
+                const int stop = std::min(p + piece, end);
+                const int q = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+                load[q] += (double)(stop - p) * cost(s);
+                for (int b = p; b < stop; b += bs)
+                    per[q].push_back(make_int4(s, b, std::min(b + bs, stop), 0));
             }
         }
-        qb[nq] = (int)tl.size();
+        size_t longest = 0;
+        for (const auto& v : per) longest = std::max(longest, v.size());
+        std::vector<int4> tl(longest * nq, make_int4(-1, 0, 0, 0));
+        for (int q = 0; q < nq; ++q)
+            for (size_t k = 0; k < per[q].size(); ++k) tl[k * nq + q] = per[q][k];
         TileSet& t = tiles_[key];
         t.ntiles = (int)tl.size();
         t.tiles.resize(tl.size());
-        t.qbeg.resize(nq + 1);
+        t.len.resize(nq);
+        std::vector<int> len(nq);
+        for (int q = 0; q < nq; ++q) len[q] = (int)per[q].size();
+        hip_check(hipMemcpy(t.len.get(), len.data(), sizeof(int) * nq, hipMemcpyHostToDevice), "tile counts");
         hip_check(hipMemcpy(t.tiles.get(), tl.data(), sizeof(int4) * tl.size(), hipMemcpyHostToDevice), "tiles");
-        hip_check(hipMemcpy(t.qbeg.get(), qb.data(), sizeof(int) * (nq + 1), hipMemcpyHostToDevice), "qbeg");
         return t;
     }
 
-    int GridFor(const TileSet& t, int g) const {
-        const int n = g > 0 ? std::min(g, t.ntiles) : t.ntiles;
-        return std::max(n, 1);
+    // One block per tile, or g persistent blocks when those are fewer.
+    template <int BS>
+    void LaunchDensityOf(const DensityArgs& a, float dt) {
+        const int g = tune_.grid_density;
+        if (g > 0 && g < a.tiles.n)
+            k2_density<BS, true><<<g, BS, 0, st_>>>(dev_, dt, a);
+        else
+            k2_density<BS, false><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
     }
-
-    void LaunchDensity(const TileSet& t, const DensityArgs& a, float dt) {
-        const int g = GridFor(t, tune_.grid_density);
+    template <int BS>
+    void LaunchForceOf(const ForceArgs& a, float dt) {
+        const int g = tune_.grid_force;
+        if (g > 0 && g < a.tiles.n)
+            k2_force<BS, true><<<g, BS, 0, st_>>>(dev_, dt, a);
+        else
+            k2_force<BS, false><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
+    }
+    void LaunchDensity(const DensityArgs& a, float dt) {
         switch (tune_.block_density) {
-            case 64: k2_density<64><<<g, 64, 0, st_>>>(dev_, dt, a); break;
-            case 128: k2_density<128><<<g, 128, 0, st_>>>(dev_, dt, a); break;
-            case 256: k2_density<256><<<g, 256, 0, st_>>>(dev_, dt, a); break;
-            case 512: k2_density<512><<<g, 512, 0, st_>>>(dev_, dt, a); break;
-            default: k2_density<1024><<<g, 1024, 0, st_>>>(dev_, dt, a); break;
+            case 64: LaunchDensityOf<64>(a, dt); break;
+            case 128: LaunchDensityOf<128>(a, dt); break;
+            case 256: LaunchDensityOf<256>(a, dt); break;
+            case 512: LaunchDensityOf<512>(a, dt); break;
+            default: LaunchDensityOf<1024>(a, dt); break;
         }
         hip_check(hipGetLastError(), "density");
     }
-
-    void LaunchForce(const TileSet& t, const ForceArgs& a, float dt) {
-        const int g = GridFor(t, tune_.grid_force);
+    void LaunchForce(const ForceArgs& a, float dt) {
         switch (tune_.block_force) {
-            case 64: k2_force<64><<<g, 64, 0, st_>>>(dev_, dt, a); break;
-            case 128: k2_force<128><<<g, 128, 0, st_>>>(dev_, dt, a); break;
-            case 256: k2_force<256><<<g, 256, 0, st_>>>(dev_, dt, a); break;
-            case 512: k2_force<512><<<g, 512, 0, st_>>>(dev_, dt, a); break;
-            default: k2_force<1024><<<g, 1024, 0, st_>>>(dev_, dt, a); break;
+            case 64: LaunchForceOf<64>(a, dt); break;
+            case 128: LaunchForceOf<128>(a, dt); break;
+            case 256: LaunchForceOf<256>(a, dt); break;
+            case 512: LaunchForceOf<512>(a, dt); break;
+            default: LaunchForceOf<1024>(a, dt); break;
         }
         hip_check(hipGetLastError(), "force");
     }
