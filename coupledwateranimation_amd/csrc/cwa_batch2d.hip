@@ -80,6 +80,10 @@ constexpr int kPiecesPerXcd = 8;  // a scene is cut into pieces of at most this 
 // 899 us; force 3, 4, 6 -> 1555, 1532, 1546 us.
 constexpr int kDensityBatch2D = 4;
 constexpr int kForceBatch2D = 4;
+// Terms of a flux column a lane loads together (256 scenes, 256 threads each: one
+// -> eight 137 -> 59 us; columns of a wave side by side instead: 149 us, and at
+// 1 024 threads 77 against 23).
+constexpr int kFluxAhead = 8;
 constexpr int kRunShift = 26;   // run record: slot | (len - 1) << 26
 constexpr unsigned kRunSlotMask = (1u << kRunShift) - 1u;
 
@@ -623,7 +627,15 @@ __global__ void __launch_bounds__(1024)
         for (int cx = wv; cx < P.nxc; cx += nw) {  // flux column = cell columns 2cx, 2cx + 1
             const int b = off[cb + 2 * cx * P.ny], e = off[cb + min(2 * cx + 2, P.nx) * P.ny];
             float s = 0.0f;
-            for (int k = b + lane; k < e; k += 64) s += flux[k];
+            // kFluxAhead terms of the lane loaded before the first is added
+            for (int k = b + lane; k < e; k += 64 * kFluxAhead) {
+                float f[kFluxAhead];
+#pragma unroll
+                for (int u = 0; u < kFluxAhead; ++u) f[u] = k + 64 * u < e ? flux[k + 64 * u] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < kFluxAhead; ++u)
+                    if (k + 64 * u < e) s += f[u];
+            }
 #pragma unroll
             for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
             if (lane == 0) col[cx] = s;
@@ -990,6 +1002,7 @@ class Batch2D {
         if (t.grid_density < 0 || t.grid_force < 0) throw Error(CWA_EINVAL, "grid must be >= 0");
         tune_ = t;
         tune_.xcd_queues = t.xcd_queues ? 1 : 0;
+        tuned_ = true;
         InvalidateGraph();
     }
     const cwa2d_tuning& Tuning() const { return tune_; }
@@ -1038,7 +1051,10 @@ class Batch2D {
             mark(B_FORCE, first ? 1 : 3);
         }
         mark(B_WAVE, 0);
-        k2_wave<<<ns_, tune_.wave_block, lds_bytes_, st_>>>(dev_, dt, sc_.get(), offset_.get(),
+        // untuned: the largest block, for a scene's column sums and substeps
+        // (MI355X, 256 threads -> 1 024: 256 scenes 59 -> 23 us, 24 small ones
+        // 16.3 -> 9.3, the application's scene 6.2 both)
+        k2_wave<<<ns_, tuned_ ? tune_.wave_block : 1024, lds_bytes_, st_>>>(dev_, dt, sc_.get(), offset_.get(),
                                                              flux_.get(), h0_.get(), h1_.get(), lmax_);
         hip_check(hipGetLastError(), "wave");
         mark(B_WAVE, 1);
@@ -1401,6 +1417,7 @@ class Batch2D {
     DeviceBuffer<float> h0_, h1_;
     std::map<int, TileSet> tiles_;
     cwa2d_tuning tune_{};
+    bool tuned_ = false;  // tune_ was set, not the initial values
     hipStream_t st_ = nullptr;
     hipGraphExec_t graph_exec_ = nullptr;
     float graph_dt_ = 0.0f;
