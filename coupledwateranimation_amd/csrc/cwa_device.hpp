@@ -14,6 +14,7 @@ struct DevParams {
     float h;         // smoothing length
     float h2;        // h*h
     float r2_lt;     // sqrt_rn(r2) < h  <=>  r2 < r2_lt (exact, see host)
+    float pack_scale;  // kPackUnits / h
     float m;         // particle mass
     float m_poly6;   // mass * 315/(64 pi h^9)
     float rho0;      // rest density
@@ -123,6 +124,49 @@ __device__ __forceinline__ void store_once(float* p, float v) { __builtin_nontem
 
 __device__ __forceinline__ int lin_cell(const int dims[3], int ix, int iy, int iz) {
     return grid_column(dims, ix, iz) * dims[1] + iy;
+}
+
+// Packed point: the coordinates in units of h / kPackUnits, modulo 256, one
+// byte each from the lowest (x, y, z; the top byte 0).  The 32-bit difference
+// of two packed points holds their coordinate differences as signed bytes
+// (one unit less where the byte below borrowed), so one dot4 gives a squared
+// distance that finds every neighbour of a point, and few others:
+//   for points with r < h whose scaled coordinates stay below kPackRange, each
+//   byte is off by less than 1 (floor) + 0.25 (rounding) + 1 (borrow; none
+//   in x), the top byte is 0 or -1, so the packed distance is below
+//   kPackUnits + sqrt(1.25^2 + 2 * 2.25^2 + 1) = 87.57 units: kPackLt.
+// Differences beyond 128 units wrap to wrong, also small, values: a reader
+// tests what passes by the exact distance.
+constexpr int kPackUnits = 84;
+constexpr int kPackLt = 7680;                // squared units; 87.57^2 = 7668.5
+constexpr float kPackRange = 1048576.0f;     // 2^20 units
+constexpr int kPackPad = 64;                 // words a reader may load past the last point
+
+__device__ __forceinline__ uint32_t pack_axis(float p, float gmin, float scale) {
+    const float f = floorf((p - gmin) * scale);
+    return (uint32_t)(int)fminf(fmaxf(f, -1073741824.0f), 1073741824.0f) & 255u;
+}
+__device__ __forceinline__ uint32_t pack_point(const DevParams& P, float4 p) {
+    return pack_axis(p.x, P.gmin[0], P.pack_scale) |
+           pack_axis(p.y, P.gmin[1], P.pack_scale) << 8 |
+           pack_axis(p.z, P.gmin[2], P.pack_scale) << 16;
+}
+// Whether a point lies outside kPackRange (NaN included): none of its
+// candidates can be ruled out.
+__device__ __forceinline__ bool pack_far(const DevParams& P, float4 p) {
+    return !(fabsf((p.x - P.gmin[0]) * P.pack_scale) < kPackRange &&
+             fabsf((p.y - P.gmin[1]) * P.pack_scale) < kPackRange &&
+             fabsf((p.z - P.gmin[2]) * P.pack_scale) < kPackRange);
+}
+// Shifts whether b may be a neighbour of a into the lowest bit of bits: the sign
+// of the squared packed distance plus bias (-kPackLt, or INT32_MIN to let every
+// candidate pass; uniform in the wave).  The saturating form of dot4 because
+// it takes the bias as an operand; the other one overwrites its own (a move
+// per candidate).
+__device__ __forceinline__ void pack_test(uint32_t a, uint32_t b, int bias, uint32_t& bits) {
+    const int d = (int)(b - a);
+    const int s = __builtin_amdgcn_sdot4(d, d, bias, true);
+    bits = __builtin_amdgcn_alignbit(bits, (uint32_t)s, 31);
 }
 
 // Candidate slot range of a query point p in column c of its 3 x 3 column

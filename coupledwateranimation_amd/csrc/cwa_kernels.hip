@@ -228,7 +228,6 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_down(const int* __restric
 // a launch that has summed them.  Quadratic reads, so only while a block's
 // share is a few rounds; the input must not change during the launch, so it
 // must not overlap what is written.
-// SCANFIG
 constexpr int kScanOneThreads = 1024;
 constexpr int kScanOneTile = kScanOneThreads * kScanItems;  // 8192
 constexpr int kScanOneTiles = 8;
@@ -435,7 +434,8 @@ __global__ void __launch_bounds__(256) k_stable_reorder(
     const int* __restrict__ key, const int* __restrict__ offset, const int* __restrict__ head,
     const int2* __restrict__ link, int n, const int* __restrict__ item_of,
     int* __restrict__ list, const float4* __restrict__ pos_in,
-    const int* __restrict__ id_in, float4* __restrict__ pos_out, int* __restrict__ id_out) {
+    const int* __restrict__ id_in, float4* __restrict__ pos_out, int* __restrict__ id_out,
+    const DevParams* __restrict__ Pd, uint32_t* __restrict__ packed_out) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     const bool valid = s < n;
@@ -460,8 +460,10 @@ __global__ void __launch_bounds__(256) k_stable_reorder(
         // read once (nt): the previous force pass's output leaves the L2 to the
         // sorted copy this pass writes and the next passes gather from (A/B
         // on one box: step 0.2606 -> 0.2548 ms, the force pass 109.6 -> 104.6 us)
-        pos_out[d] = load_once(&pos_in[s]);
+        const float4 p = load_once(&pos_in[s]);
+        pos_out[d] = p;
         id_out[d] = load_once(&id_in[s]);
+        if (packed_out) packed_out[d] = pack_point(*Pd, p);
     }
 }
 
@@ -593,20 +595,50 @@ __device__ __forceinline__ void density_finish(const DevParams& P, int i, float4
 // Also records the exact neighbour set of every particle as neighbour words
 // (the packed non-empty words of each candidate column's 32-candidate
 // chunks, the particle itself left out; layout at kNbEntries).
+//
+// One lane per particle, in two stages.  The first goes over the candidate
+// columns (rows within h of the particle) and tests the candidates' packed
+// points, 4 bytes and 3 VALU instructions a candidate, which leaves the
+// neighbours and a few more as words in LDS.  The second visits only those, in
+// one flat loop, by the exact distance, and takes the others out of the words.
+// Neighbours are summed in candidate order.
+//
+// What bounds it is the address unit (77 % busy at 1 048 576 particles), by
+// the bytes its loads hand to the lanes: testing all ~120 candidates of a
+// particle by their 16-byte positions took 125.7 us at 1 048 576 particles and
+// 44.5 at 300 007 (3 780 VALU instructions a wave), this takes 87.1 and 33.5
+// (2 490).  Measured at 1 048 576: kPackFirst 16, 20, 24: 102, 88.4, 90.8;
+// kDensityBatch 3, 4, 6, 8: 87.1, 88.4, 91.2, 94.5; batches that end with their
+// word (fewer instructions, more idle loads) 94.9; rows cut to the support
+// sphere per column cost what their candidates save.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_density(const DevParams* __restrict__ Pd, const float4* __restrict__ pos,
-                                                 const float4* __restrict__ vel,
-                                                 const int* __restrict__ list,
-                                                 const int* __restrict__ offset, int n,
-                                                 const float* __restrict__ H0,
-                                                 float* __restrict__ rho_w,
-                                                 float2* __restrict__ pw,
-                                                 float* __restrict__ flux,
-                                                 uint2* __restrict__ nbw,
-                                                 float4* __restrict__ nrec,
-                                                 float* __restrict__ rho_raw,
-                                                 float4* __restrict__ vel_out,
-                                                 float* __restrict__ vpad) {
+struct alignas(4) PackedQuad {
+    uint32_t v[4];
+};
+// Bits kFrom .. kTo - 1: which of the points q[kFrom .. kTo) may be a neighbour.
+template <int kFrom, int kTo>
+__device__ __forceinline__ uint32_t pack_chunk(const uint32_t* __restrict__ q, uint32_t own,
+                                               int bias) {
+    constexpr int kNum = kTo - kFrom;
+    PackedQuad v[kNum / 4];
+#pragma unroll
+    for (int k = 0; k < kNum / 4; ++k)
+        v[k] = *reinterpret_cast<const PackedQuad*>(q + kFrom + 4 * k);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int k = 0; k < kNum; ++k) pack_test(own, v[k / 4].v[k % 4], bias, bits);
+    return __brev(bits) >> (32 - kTo);
+}
+constexpr int kPackFirst = 20;  // candidates of a chunk tested without a look at their number
+constexpr int kDensityBatch = 3;  // exact tests whose loads are in flight together
+
+__global__ void __launch_bounds__(256) k_density(
+    const DevParams* __restrict__ Pd, const float4* __restrict__ pos,
+    const uint32_t* __restrict__ packed, const float4* __restrict__ vel,
+    const int* __restrict__ list, const int* __restrict__ offset, int n,
+    const float* __restrict__ H0, float* __restrict__ rho_w, float2* __restrict__ pw,
+    float* __restrict__ flux, uint2* __restrict__ nbw, float4* __restrict__ nrec,
+    float* __restrict__ rho_raw, float4* __restrict__ vel_out, float* __restrict__ vpad) {
     const DevParams& P = *Pd;
     const int i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -619,37 +651,97 @@ __global__ void __launch_bounds__(256) k_density(const DevParams* __restrict__ P
     const float T = P.r2_lt;
     float acc = 0.0f;
     __shared__ uint2 s_held[kNbHeld][256];
-    NbWriter wr(&s_held[0][threadIdx.x], 256);
-    bool tail = false;  // a column longer than kNbMaxColumn candidates
-#pragma unroll 1
-    for (int c = 0; c < 9; ++c) {
-        int b, e;
-        column_range(P, offset, pi.x, pi.y, pi.z, ix, iz, c, b, e);
-        const float4* __restrict__ q = pos + b;
-        const int len = e - b;
-        uint32_t lo = 0, hi = 0;
-        const int l1 = min(len, 32);
-        int k = 0;
-        for (; k + 1 < l1; k += 2) {
-            const float4 a0 = q[k], a1 = q[k + 1];
-            density_candidate(pi, a0, T, acc, lo, k);
-            density_candidate(pi, a1, T, acc, lo, k + 1);
+    uint2* const held = &s_held[0][threadIdx.x];
+    int w = 0;    // words in LDS
+    int out = 0;  // words given out
+    uint2* plane = nbw + i;
+    // second stage: the words in LDS
+    const auto flush = [&]() {
+        uint32_t cur = 0, base = 0;
+        const int end = w * 256;
+        int t = 0;  // the word after cur's, as an index into held
+        for (;;) {
+            uint32_t j[kDensityBatch], bit[kDensityBatch];
+            int at[kDensityBatch];
+#pragma unroll
+            for (int u = 0; u < kDensityBatch; ++u) {
+                if (cur == 0u && t < end) {
+                    const uint2 v = held[t];
+                    cur = v.x;
+                    base = v.y;
+                    t += 256;
+                }
+                bit[u] = cur & (0u - cur);
+                at[u] = t - 256;
+                j[u] = base + (uint32_t)__builtin_ctz(max(cur, 1u));
+                cur &= cur - 1u;
+            }
+            if (bit[0] == 0u) break;
+            float4 a[kDensityBatch];
+#pragma unroll
+            for (int u = 0; u < kDensityBatch; ++u) a[u] = pos[j[u]];
+#pragma unroll
+            for (int u = 0; u < kDensityBatch; ++u) {
+                const float r2 = dist2_fma(pi.x - a[u].x, pi.y - a[u].y, pi.z - a[u].z);
+                // > 0 exactly for neighbours; slots past the last word count nothing
+                const float ww = fmaxf((u == 0 || bit[u] ? T : 0.0f) - r2, 0.0f);
+                acc = fmaf(ww * ww, ww, acc);
+                if (!(ww > 0.0f)) atomicAnd(&held[at[u]].x, ~bit[u]);
+            }
         }
-        if (k < l1) density_candidate(pi, q[k], T, acc, lo, k);
-        if (len > 32) {
-            const int l2 = min(len, 64);
-            for (k = 32; k < l2; ++k) density_candidate(pi, q[k], T, acc, hi, k - 32);
-            uint32_t none = 0;
-            for (k = 64; k < len; ++k) density_candidate(pi, q[k], T, acc, none, 0);
-            tail |= len > kNbMaxColumn;
+#pragma unroll
+        for (int k = 0; k < kNbHeld; ++k) {
+            if (k < w) {
+                uint2 v = held[k * 256];
+                const uint32_t self = (uint32_t)i - v.y;
+                if (self < 32u) v.x &= ~(1u << self);
+                if (v.x) {
+                    if (out < kNbEntries) {
+                        *plane = v;
+                        plane += n;
+                    }
+                    ++out;
+                }
+            }
         }
-        const uint32_t self = (uint32_t)(i - b);  // i is a candidate of one column
-        if (self < 32u) lo &= ~(1u << self);
-        else if (self < 64u) hi &= ~(1u << (self - 32u));
-        wr.put(nbw, n, i, lo, (uint32_t)b);
-        wr.put(nbw, n, i, hi, (uint32_t)b + 32u);
+        w = 0;
+    };
+    const int ylo = cell_axis(pi.y - P.h - P.grid_eps, P.gmin[1], P.cell_y, P.dims[1]);
+    const int yhi = cell_axis(pi.y + P.h + P.grid_eps, P.gmin[1], P.cell_y, P.dims[1]);
+    const uint32_t own = packed[i];
+    const int bias = __any(pack_far(P, pi)) ? INT32_MIN : -kPackLt;
+    // first cell of column (ix - 1, iz - 1 + k), and the step to the next ix
+    int first[3], step[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int cz = min(max(iz + k - 1, 0), P.dims[2] - 1);
+        first[k] = grid_column(P.dims, ix, cz) * P.dims[1];
+        step[k] = grid_column(P.dims, ix + 1, cz) * P.dims[1] - first[k];
+        first[k] -= step[k];
     }
-    wr.finish(nbw, n, i, tail);
+#pragma unroll 1
+    for (int dx = 0; dx < 3; ++dx) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int cx = ix + dx - 1, cz = iz + k - 1;
+            int b = 0, e = 0;
+            if (cx >= 0 && cx < P.dims[0] && cz >= 0 && cz < P.dims[2]) {
+                b = offset[first[k] + ylo];
+                e = offset[first[k] + yhi + 1];
+            }
+            first[k] += step[k];
+            for (; b < e; b += 32) {
+                const int len = e - b;
+                uint32_t bits = pack_chunk<0, kPackFirst>(packed + b, own, bias);
+                if (len > kPackFirst) bits |= pack_chunk<kPackFirst, 32>(packed + b, own, bias);
+                if (len < 32) bits &= ~(~0u << len);
+                if (bits) held[w++ * 256] = make_uint2(bits, (uint32_t)b);
+                if (__any(w == kNbHeld)) flush();
+            }
+        }
+    }
+    flush();
+    nb_count(nbw, n)[i] = out > kNbEntries ? -1 : out;
     const float u = (pi.x - P.org[0]) * P.uvs[0];
     const float v = (pi.z - P.org[1]) * P.uvs[1];
     density_finish(P, i, pi, vi, acc, tex_sample(H0, P.W, P.H, u, v), rho_w, pw, flux, nrec,
@@ -1591,10 +1683,12 @@ hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStr
 hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,
                                  const int2* link, int n, const int* item_of, int* list,
                                  const float4* pos_in, const int* id_in, float4* pos_out,
-                                 int* id_out, hipStream_t st) {
+                                 int* id_out, hipStream_t st, const DevParams* Pd,
+                                 uint32_t* packed_out) {
     if (n <= 0) return hipSuccess;
     k_stable_reorder<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, head, link, n, item_of, list,
-                                                         pos_in, id_in, pos_out, id_out);
+                                                         pos_in, id_in, pos_out, id_out, Pd,
+                                                         packed_out);
     return hipGetLastError();
 }
 
@@ -1634,15 +1728,16 @@ hipError_t launch_box_pairs(const float4* x, const float4* hw, int n, const floa
 hipError_t launch_density(const DevParams& P, const float4* bpos, const float4* state_vel,
                           const int* list, const int* offset, int n, const float* H0,
                           float* rho_w, float2* pw, float* flux, uint2* nbw, float4* nrec,
-                          float* rho_raw, float4* vel_out, float* vpad, hipStream_t st) {
+                          float* rho_raw, float4* vel_out, float* vpad, const uint32_t* packed,
+                          hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    if (n <= lane_split_limit())
+    if (!packed)
         k_density_split<<<blocks_for((long long)n * kDensitySplit, 256), 256, 0, st>>>(
             P.dev, bpos, state_vel, list, offset, n, H0, rho_w, pw, flux, nbw, nrec, rho_raw,
             vel_out, vpad);
     else
-        k_density<<<blocks_for(n, 256), 256, 0, st>>>(P.dev, bpos, state_vel, list, offset, n,
-                                                      H0, rho_w, pw, flux, nbw, nrec, rho_raw,
+        k_density<<<blocks_for(n, 256), 256, 0, st>>>(P.dev, bpos, packed, state_vel, list, offset,
+                                                      n, H0, rho_w, pw, flux, nbw, nrec, rho_raw,
                                                       vel_out, vpad);
     return hipGetLastError();
 }

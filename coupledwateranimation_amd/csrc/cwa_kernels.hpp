@@ -54,11 +54,14 @@ hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStr
 // hash pass at 1 048 576 particles 51 / 32 us).
 constexpr int kFuseLinksMax = 1 << 18;
 // list[d] = item_of ? item_of[s] : s at each item's stable destination d;
-// with pos_out set, pos_out[d] = pos_in[s] and id_out[d] = id_in[s].
+// with pos_out set, pos_out[d] = pos_in[s] and id_out[d] = id_in[s], and with
+// packed_out set also (Pd: the device parameters) packed_out[d] =
+// pack_point(pos_in[s]).
 hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,
                                  const int2* link, int n, const int* item_of, int* list,
                                  const float4* pos_in, const int* id_in, float4* pos_out,
-                                 int* id_out, hipStream_t st);
+                                 int* id_out, hipStream_t st, const DevParams* Pd = nullptr,
+                                 uint32_t* packed_out = nullptr);
 // Boxes: cells covered per box (ncov, n ints), then the (box, cell) pairs at
 // first[i] = exclusive scan of ncov (pkey: cell, pbox: box index).
 hipError_t launch_box_cover(const float4* x, const float4* hw, int n, const float gmin[3],
@@ -75,7 +78,8 @@ hipError_t launch_box_pairs(const float4* x, const float4* hw, int n, const floa
 // through the step) are written for the force pass.  pw (pressure, 1/rho),
 // rho_raw (density before the wave term and the rest-density clamp) and
 // vel_out (the sorted velocities) are optional outputs for the adjoint tape
-// (null: not written).
+// (null: not written).  packed: the packed points of bpos[0..n) followed by
+// kPackPad readable words for the one-lane pass, null for the four-lane pass.
 // Scenes of up to this many particles run the density pass (and a tape's
 // pair adjoint, and up to kForceSplitMax the force pass) with four lanes per
 // particle, larger ones with one lane; read at each launch and at tape
@@ -87,7 +91,8 @@ long long set_lane_split_limit(long long max_n);  // returns the previous limit
 hipError_t launch_density(const DevParams& P, const float4* bpos, const float4* state_vel,
                           const int* list, const int* offset, int n, const float* H0,
                           float* rho_w, float2* pw, float* flux, uint2* nbw, float4* nrec,
-                          float* rho_raw, float4* vel_out, float* vpad, hipStream_t st);
+                          float* rho_raw, float4* vel_out, float* vpad, const uint32_t* packed,
+                          hipStream_t st);
 // Where the force pass hashes the next step's grid, or key == null for no
 // fused hash.
 struct NextKeys {

@@ -169,10 +169,11 @@ class UniformGrid3D {
     void Init(const GridDesc& g, int max_particles);
     // BuildGrid (UniformGridParticles3D.cpp:170-211) over A.pos[0..n):
     // sorted positions / ids into bpos / bid.  list_out / offset_out
-    // (optional) replace the grid's own list / offsets.
+    // (optional) replace the grid's own list / offsets; packed_out (optional,
+    // with the device parameters Pd) receives the sorted packed points.
     void BuildGrid(const ParticleArrays& A, int n, float4* bpos, int* bid, hipStream_t st,
-                   hipEvent_t* ev = nullptr, int* list_out = nullptr,
-                   int* offset_out = nullptr);
+                   hipEvent_t* ev = nullptr, int* list_out = nullptr, int* offset_out = nullptr,
+                   const DevParams* Pd = nullptr, uint32_t* packed_out = nullptr);
     // Where the force pass of this step hashes the next step's keys.
     NextKeys FusedNext() const {
         return NextKeys{key_[kc_ ^ 1].get(),
@@ -293,6 +294,7 @@ class SphParticles3D {
     float* vpad() const { return vpad_.get(); }
     uint2* nbw() const { return nbw_.get(); }
     float4* nrec() const { return nrec_.get(); }
+    uint32_t* packed() const { return packed_.get(); }
 
    private:
     int n_ = 0;
@@ -300,6 +302,7 @@ class SphParticles3D {
     DeviceSlab slab_;
     DeviceBuffer<uint2> nbw_;  // neighbour words and counts of the last step
     DeviceBuffer<float4> nrec_;   // 2 x n neighbour records of the last step
+    DeviceBuffer<uint32_t> packed_;  // packed points of bpos, with kPackPad words after them
     DeviceBuffer<float4> pos_[2], vel_[2], force_[2], bpos_;
     DeviceBuffer<int> id_[2], bid_;
     DeviceBuffer<float> rho_, prs_, rho_w_, flux_, vpad_;

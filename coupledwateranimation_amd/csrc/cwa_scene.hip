@@ -86,7 +86,8 @@ void UniformGrid3D::ClearCounters(hipStream_t st) {
 }
 
 void UniformGrid3D::BuildGrid(const ParticleArrays& A, int n, float4* bpos, int* bid,
-                              hipStream_t st, hipEvent_t* ev, int* list_out, int* offset_out) {
+                              hipStream_t st, hipEvent_t* ev, int* list_out, int* offset_out,
+                              const DevParams* Pd, uint32_t* packed_out) {
     const int nc = num_cells();
     int* lst = list_out ? list_out : list_.get();
     int* off = offset_out ? offset_out : offset_.get();
@@ -115,7 +116,7 @@ void UniformGrid3D::BuildGrid(const ParticleArrays& A, int n, float4* bpos, int*
     mark(K_SCATTER, 1);
     mark(K_REORDER, 0);
     hip_check(launch_stable_reorder(key, off, head, runs.link, n, nullptr, lst, A.pos, A.id, bpos,
-                                    bid, st),
+                                    bid, st, Pd, packed_out),
               "reorder");
     mark(K_REORDER, 1);
 }
@@ -211,6 +212,7 @@ void SphParticles3D::Allocate(int n) {
     slab_.add(vpad_, m);
     slab_.add(nbw_, nb_buffer_uint2(m));
     slab_.add(nrec_, 2 * m);
+    slab_.add(packed_, m + kPackPad);
     slab_.commit();
     A = ParticleArrays{pos_[0].get(), vel_[0].get(), force_[0].get(), id_[0].get()};
     N = ParticleArrays{pos_[1].get(), vel_[1].get(), force_[1].get(), id_[1].get()};
@@ -285,6 +287,7 @@ DevParams make_devparams(const cwa_params& p, int W, int H) {
     d.h = p.h;
     d.h2 = p.h * p.h;
     d.r2_lt = exact_r2_threshold(p.h);
+    d.pack_scale = (float)kPackUnits / p.h;
     d.m = p.mass;
     const float h2 = p.h * p.h, h6 = h2 * h2 * h2, h9 = h6 * h2 * p.h;
     const float poly6 = 315.0f / (64.0f * pi * h9);
@@ -487,13 +490,14 @@ void CoupledScene::Step(float dt, hipEvent_t (*ev)[2], const TapeOut* tape) {
     WaveTiles wt{};
     if (n > 0 && !ev) wt = wave_tiles_for(dp_, n, couple, H0, H1, Hout);
     if (n > 0) {
+        uint32_t* packed = n > lane_split_limit() ? particles.packed() : nullptr;
         grid.BuildGrid(particles.A, n, bpos, particles.bid(), st_, ev ? &ev[0][0] : nullptr, lst,
-                       off);
+                       off, dp_.dev, packed);
         mark(K_DENSITY, 0);
         hip_check(launch_density(dp_, bpos, particles.A.vel, lst, off, n, H0, rho_w,
                                  tape ? tape->pw : nullptr, particles.flux(), nbm, nrec,
                                  tape ? tape->rho_raw : nullptr, tape ? tape->vel : nullptr,
-                                 particles.vpad(), st_),
+                                 particles.vpad(), packed, st_),
                   "density");
         mark(K_DENSITY, 1);
         // the same launch sums the particle flux per column when coupled,

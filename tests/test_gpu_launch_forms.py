@@ -99,3 +99,48 @@ def test_force_with_four_lanes(gpu, cwa, n, shape):
     _, g = _scene_state(cwa, spec, pos, vel, force, -1, 3)
     assert np.array_equal(g["list"], np.argsort(g["key"], kind="stable"))
     assert np.array_equal(g["count"], np.bincount(g["key"], minlength=g["count"].size))
+
+
+@pytest.mark.parametrize("shape", ["1", "20", "21", "32", "33", "64", "65", "300", "columns",
+                                   "lattice", "far"])
+def test_density_by_packed_points(gpu, cwa, oracle, shape):
+    """The one-lane pass finds every neighbour, whatever the length of a column
+    (chunks of 32 candidates, 20 tested at once), the number of a particle's
+    words (more than eight, more than are recorded) and its distance to the
+    grid.  Its sum differs from the four-lane pass's in order only: within
+    2 * terms * 2^-24 of it, all terms being positive."""
+    from coupledwateranimation_amd import configs
+    from coupledwateranimation_amd.scene import set_lane_split_limit
+
+    print(f"packed density {shape}", flush=True)
+    spec = configs.dam_break_diff(4096, 96, 7)
+    h = spec.params.h
+    cell, lo = spec.params.cell_size, np.array(list(spec.params.grid_min))
+    rng = np.random.default_rng(len(shape))
+    if shape.isdigit():      # one column of so many candidates
+        pos = lo + cell * (3 + 0.9 * rng.random((int(shape), 3)))
+    elif shape == "columns":  # 3 x 3 columns of several chunks each
+        pos = lo + cell * (2 + 3 * rng.random((700, 3)))
+    elif shape == "lattice":
+        pos = spec.pos[:4001, :3].astype(np.float64)
+    else:                    # beyond the range of the packed coordinates, and at the grid
+        pos = np.concatenate([spec.pos[:500, :3], spec.pos[:500, :3] + 20_000 * h])
+    n = len(pos)
+    p4 = np.zeros((n, 4), np.float32)
+    p4[:, :3] = pos
+    zero = np.zeros((96, 96), np.float32)
+    got = []
+    old = set_lane_split_limit(0)
+    try:
+        for limit in (0, 1 << 20):
+            set_lane_split_limit(limit)
+            with cwa.Scene(spec.params, p4, np.zeros_like(p4), None, (96, 96), zero, zero) as s:
+                s.step(spec.dt, 1)
+                got.append((s.neighbour_counts(), s.readback()))
+    finally:
+        set_lane_split_limit(old)
+    counts = oracle.neighbor_counts(spec.params, p4, all_pairs=True)
+    assert np.array_equal(got[0][0], counts) and np.array_equal(got[1][0], counts)
+    assert counts.max() > 1 or n == 1
+    a, b = got[0][1]["rho"], got[1][1]["rho"]
+    assert np.abs(a - b).max() <= 2 * counts.max() * 2.0 ** -24 * np.abs(b).max()
