@@ -277,7 +277,17 @@ constexpr int kNbStage = kNbEntries;
 __device__ __forceinline__ int stage_nb_words(const uint2* __restrict__ nbw, int n, int i,
                                               uint2* s, int stride) {
     const int nw = load_once(&nb_count(nbw, n)[i]);
-    for (int k = 0; k < nw; ++k) s[k * stride] = load_once(&nbw[(size_t)k * n + i]);
+    // most particles have no more words than this: one wait for all of them
+    // (the force pass at 1 048 576 / 300 007 particles 94.1 -> 93.4 / 33.8 -> 33.1 us)
+    constexpr int kAtOnce = 8;
+    uint2 w[kAtOnce];
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k)
+        if (k < nw) w[k] = load_once(&nbw[(size_t)k * n + i]);
+#pragma unroll
+    for (int k = 0; k < kAtOnce; ++k)
+        if (k < nw) s[k * stride] = w[k];
+    for (int k = kAtOnce; k < nw; ++k) s[k * stride] = load_once(&nbw[(size_t)k * n + i]);
     return nw;
 }
 

@@ -913,6 +913,34 @@ __device__ __forceinline__ Nbr load_nbr(const float4* __restrict__ nrec, int j) 
     return Nbr{nrec[2 * (size_t)j], nrec[2 * (size_t)j + 1]};
 }
 
+// The value of the other lane of a pair (lane ^ 1, both active).
+__device__ __forceinline__ int pair_swap(int v) {
+    return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true);
+}
+__device__ __forceinline__ float4 pair_swap(float4 v) {
+    const auto f = [](float x) { return __int_as_float(pair_swap(__float_as_int(x))); };
+    return make_float4(f(v.x), f(v.y), f(v.z), f(v.w));
+}
+__device__ __forceinline__ float4 select4(bool c, float4 a, float4 b) {
+    return make_float4(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z, c ? a.w : b.w);
+}
+
+// load_nbr by the two lanes of a pair together: each load instruction takes
+// both halves of one lane's record, so a record costs the cache one access
+// instead of two, and the lanes swap the halves they loaded for each other.
+// The even lane's record comes with the first half in the even lane, the odd
+// lane's with the first half in the odd lane: what is swapped is always a
+// second half.  The force pass is bound by those accesses (address unit 81 %
+// busy, 45 cache accesses a load instruction): 1 048 576 particles 105 -> 94
+// us, 300 007 38.4 -> 33.8, for 17 VALU instructions more a record.
+__device__ __forceinline__ Nbr load_nbr_pair(const float4* __restrict__ nrec, int j) {
+    const bool odd = threadIdx.x & 1;
+    const int other = pair_swap(j);
+    const float4 x = nrec[2 * (size_t)(odd ? other : j) + (odd ? 1 : 0)];
+    const float4 y = nrec[2 * (size_t)(odd ? j : other) + (odd ? 0 : 1)];
+    return Nbr{select4(odd, y, x), pair_swap(select4(odd, x, y))};
+}
+
 __device__ __forceinline__ void force_pair(float h, float4 pi, float4 vi, float p_i,
                                            float m_spiky_half, float m_lap, const Nbr& nb,
                                            PairAcc& a) {
@@ -1298,6 +1326,12 @@ __device__ __forceinline__ int force_finish(const DevParams& P, float dt, int i,
     return cell;
 }
 
+// Neighbour records in flight per lane.  At 1 048 576 particles 4, 5, 6, 7, 8, 10
+// -> 98.3, 93.8, 94.1, 99.6, 98.9, 101.8 us; at 300 007 6, 8, 10 -> 33.8, 35.9,
+// 36.6; the next batch loaded while one is summed, batches of 2, 3, 4: 104.3,
+// 97.3, 97.7.
+constexpr int kForceBatch = 6;
+
 // ---------------------------------------------------------------------------
 // Forces (force_comp.glsl:62-139) fused with symplectic Euler + boundary
 // (integrate_comp.glsl:56-92, 135-178).  Visits only the neighbours the
@@ -1340,63 +1374,57 @@ __global__ void __launch_bounds__(256) k_force_integrate(
     }
     const int i = xcd_block(blk, nfb) * blockDim.x + threadIdx.x;
     const bool valid = i < n;
+    // lanes past the end stay for their partner's loads, without neighbours
+    const int slot = min(i, n - 1);
+    const float4 own_a = nrec[2 * (size_t)slot];      // (x, y, z, p)
+    const float4 own_b = nrec[2 * (size_t)slot + 1];  // (vx, vy, vz, 1/rho)
+    const int src = load_once(&list[slot]);           // the particle's slot in the state
+    // the previous force is used only after the neighbour loop; issued
+    // here, its load is in flight while the loop runs
+    float4 fp = load_once(&force[src]);
+    const float4 pi = make_float4(own_a.x, own_a.y, own_a.z, load_once(&bpos[slot].w));
+    const float4 vi = make_float4(own_b.x, own_b.y, own_b.z, load_once(&vpad[slot]));
+    const float p_i = own_a.w;
+    const float h = P.h;
+    const float m_spiky_half = P.m * P.spiky * 0.5f;
+    const float m_lap = P.m * P.lap;
+    PairAcc a{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    uint2* st = &s_nb[0][threadIdx.x];
+    const int nw = valid ? stage_nb_words(nbw, n, i, st, 256) : 0;
+    {
+        // kForceBatch neighbours per iteration: every record is loaded
+        // before any pair is evaluated (slots past the end of the list hold
+        // the particle's own record and are evaluated with zero weight); pairs
+        // are accumulated in order
+        NbCursor nb(st, 256, nw);
+        for (;;) {
+            int j[kForceBatch];
+            j[0] = nb.next();
+            if (max(j[0], pair_swap(j[0])) < 0) break;
+#pragma unroll
+            for (int u = 1; u < kForceBatch; ++u) j[u] = nb.next();
+            Nbr r[kForceBatch];
+#pragma unroll
+            for (int u = 0; u < kForceBatch; ++u) r[u] = load_nbr_pair(nrec, j[u] < 0 ? slot : j[u]);
+#pragma unroll
+            for (int u = 0; u < kForceBatch; ++u) {
+                const bool live = j[u] >= 0;
+                force_pair(h, pi, vi, p_i, live ? m_spiky_half : 0.0f, live ? m_lap : 0.0f, r[u],
+                           a);
+            }
+        }
+    }
     int cell = -1;
     if (valid) {
-        const float4 own_a = nrec[2 * (size_t)i];      // (x, y, z, p)
-        const float4 own_b = nrec[2 * (size_t)i + 1];  // (vx, vy, vz, 1/rho)
-        const int src = load_once(&list[i]);           // the particle's slot in the state
-        // the previous force is used only after the neighbour loop; issued
-        // here, its load is in flight while the loop runs
-        float4 fp = load_once(&force[src]);
-        const float4 pi = make_float4(own_a.x, own_a.y, own_a.z, load_once(&bpos[i].w));
-        const float4 vi = make_float4(own_b.x, own_b.y, own_b.z, load_once(&vpad[i]));
-        const float p_i = own_a.w;
-        const float h = P.h;
-        const float m_spiky_half = P.m * P.spiky * 0.5f;
-        const float m_lap = P.m * P.lap;
-        PairAcc a{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        uint2* st = &s_nb[0][threadIdx.x];
-        const int nw = stage_nb_words(nbw, n, i, st, 256);
-        if (nw >= 0) {
-            // kForceBatch neighbours per iteration: every record is loaded
-            // before any pair is evaluated (slots past the end of the list hold
-            // a zero record and are evaluated with zero weight); pairs are
-            // accumulated in order.  At four blocks per CU, with the particle's
-            // own record and previous force also in flight, 4 measured fastest
-            // (MI355X, 1M-particle dam break, same box: 2, 3, 4, 5, 6, 7, 8 ->
-            // 116.6, 112.3, 110.1, 115.2, 115.1, 116.5, 115.9 us).
-            constexpr int kForceBatch = 4;
-            const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-            NbCursor nb(st, 256, nw);
-            for (;;) {
-                int j[kForceBatch];
-                j[0] = nb.next();
-                if (j[0] < 0) break;
-#pragma unroll
-                for (int u = 1; u < kForceBatch; ++u) j[u] = nb.next();
-                Nbr r[kForceBatch];
-#pragma unroll
-                for (int u = 0; u < kForceBatch; ++u) {
-                    r[u] = Nbr{zero, zero};
-                    if (j[u] >= 0) r[u] = load_nbr(nrec, j[u]);
-                }
-#pragma unroll
-                for (int u = 0; u < kForceBatch; ++u) {
-                    const bool live = j[u] >= 0;
-                    force_pair(h, pi, vi, p_i, live ? m_spiky_half : 0.0f, live ? m_lap : 0.0f, r[u],
-                               a);
-                }
-            }
-        } else {
+        if (nw < 0)
             for_each_candidate_neighbour(P, offset, bpos, i, pi, [&](int j) {
                 force_pair(h, pi, vi, p_i, m_spiky_half, m_lap, load_nbr(nrec, j), a);
             });
-        }
         const float u = (pi.x - P.org[0]) * P.uvs[0];
         const float v = (pi.z - P.org[1]) * P.uvs[1];
         const LateInputs in{P, H0, rho_w, bid, u, v, i};
         cell = force_finish(P, dt, i, pi, vi, fp, p_i, a, in, H0, out, next.key);
-    }  // valid
+    }
     if (next.key) push_runs<true, kLink>(cell, valid, i, next.runs);
 }
 
