@@ -71,15 +71,13 @@ constexpr int kNumXcd = 8;      // XCDs of an MI355X
 constexpr int kPiecesPerXcd = 8;  // a scene is cut into pieces of at most this share of an XCD
 // Candidates loaded ahead in the density / force loops (the lanes of a tile
 // walk the same candidates, so each load is one address per wave).  Measured
-// on the 256-scene workload (MI355X), cells of H: density 1, 2, 4, 6, 8, 16 ->
-// 1.42, 1.25, 1.16, 1.13, 1.12, 1.13 ms; force 1, 2, 3, 4, 6, 8 ->
-// 2.63, 2.58, 2.51, 2.49, 2.45, 2.45 ms.  With the shorter columns of H/2
-// cells: density 4 / 8 -> 0.921 / 0.926 ms; force 4, 5, 6, 8 -> 1.885,
-// 1.884, 1.898, 1.980 ms.  Again after the cheaper pair arithmetic (refined
-// hardware square roots and reciprocals): density 3, 4, 6 -> 907, 899,
-// 899 us; force 3, 4, 6 -> 1555, 1532, 1546 us.
-constexpr int kDensityBatch2D = 4;
+// on the 256-scene workload (MI355X): density 2, 4, 6, 8 -> 689, 663, 657, 660
+// us; force 2, 4, 6 -> 1 511, 1 480, 1 497 us.
+constexpr int kDensityBatch2D = 6;
 constexpr int kForceBatch2D = 4;
+constexpr int kReadPast2D = 8;  // points a batch may load past the end of an array
+static_assert(kDensityBatch2D % 2 == 0 && kForceBatch2D % 2 == 0, "points are loaded in pairs");
+static_assert(kDensityBatch2D <= kReadPast2D && kForceBatch2D <= kReadPast2D, "padding");
 // Terms of a flux column a lane loads together (256 scenes, 256 threads each: one
 // -> eight 137 -> 59 us; columns of a wave side by side instead: 149 us, and at
 // 1 024 threads 77 against 23).
@@ -316,7 +314,7 @@ __global__ void __launch_bounds__(256)
     k2_reorder(const int* __restrict__ key, const int* __restrict__ rec,
                const int* __restrict__ offset, const unsigned* __restrict__ runs, int ntot,
                const float4* __restrict__ xvA, const float2* __restrict__ rpA,
-               const int* __restrict__ idfA, float4* __restrict__ xvB,
+               const int* __restrict__ idfA, float2* __restrict__ xyB, float2* __restrict__ velB,
                float2* __restrict__ rpB, int* __restrict__ idfB, int* __restrict__ count,
                int ncells) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -336,7 +334,9 @@ __global__ void __launch_bounds__(256)
     }
     const int d = b + rank + (s - a);
     if (d < b || d >= e) return;  // only on inconsistent run records
-    xvB[d] = xvA[s];
+    const float4 p = xvA[s];
+    xyB[d] = make_float2(p.x, p.y);
+    velB[d] = make_float2(p.z, p.w);
     rpB[d] = rpA[s];
     idfB[d] = idfA[s];
 }
@@ -392,18 +392,39 @@ __device__ __forceinline__ void for_each_tile(const TileTable& T, Body&& body) {
 // ---------------------------------------------------------------------------
 // density / pressure (ComputeDensityPressure, :393-487)
 // ---------------------------------------------------------------------------
+// N consecutive points, two to a 16-byte load: a load keeps the address unit
+// busy for 16 cycles or more whatever its width, and with one load a candidate
+// the density pass kept it busy 93 % of the time (256 scenes of 4 M particles:
+// 773 -> 657 us).
+template <int N>
+struct Points {
+    struct alignas(8) Two {
+        float x0, y0, x1, y1;
+    };
+    Two v[N / 2];
+    __device__ __forceinline__ void load(const float2* __restrict__ p) {
+#pragma unroll
+        for (int k = 0; k < N / 2; ++k) v[k] = *reinterpret_cast<const Two*>(p + 2 * k);
+    }
+    __device__ __forceinline__ float2 operator[](int u) const {
+        return u % 2 ? make_float2(v[u / 2].x1, v[u / 2].y1)
+                     : make_float2(v[u / 2].x0, v[u / 2].y0);
+    }
+};
+
 struct DensityArgs {
     const Scene2D* sc;
     TileTable tiles;
-    const float4* xvB;
+    const float2* xyB;
+    const float2* velB;
     const float2* rpB;
     const int* idfB;
     const int* off;
     const float* h0;
     const float* h1;
-    float4* q;
+    float2* qxy;
+    float4* qva;
     float2* rpA;
-    float2* aj;
     int* idfA;
     float* flux;
 };
@@ -417,8 +438,8 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
         const float* w0 = A.h0 + S.wbeg;
         const float* w1 = A.h1 + S.wbeg;
         const float sL = (float)S.L / (P.hix - P.lox);
-        const float4 p4 = A.xvB[i];
-        float x = p4.x, y = p4.y, vx = p4.z, vy = p4.w;
+        const float2 p0 = A.xyB[i], v0 = A.velB[i];
+        float x = p0.x, y = p0.y, vx = v0.x, vy = v0.y;
         int idf = A.idfB[i];
         int en = (idf >> 30) & 1;
         // enable flag (:400-415); with a zero threshold an enabled particle
@@ -437,7 +458,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
             vx -= 1.75f * vn * bnx;
             vy -= 1.75f * vn * bny;
         }
-        A.q[i] = make_float4(x, y, vx, vy);
+        A.qxy[i] = make_float2(x, y);
         float f = 0.0f;
         if (P.band > 0.0f) {
             const float dd = fabsf(y - wave_at(P, w0, S.L, sL, x));
@@ -457,22 +478,28 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
             for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
                 int b, e;
                 column_rows(P, A.off, cb, x, y, ix, cx, b, e);
-                auto cand = [&](const float4 pj) {
+                auto cand = [&](const float2 pj) {
                     const float dx = x - pj.x, dy = y - pj.y;
                     const float r2 = fmaf(dy, dy, dx * dx);
                     if (r2 < P.HSQ) acc += W_cubic(P, sqrt_rn_clamped(r2));
                 };
                 // kDensityBatch2D candidates loaded before the first is
                 // tested; tested in order
-                int j = b;
-                for (; j + kDensityBatch2D <= e; j += kDensityBatch2D) {
-                    float4 pj[kDensityBatch2D];
-#pragma unroll
-                    for (int u = 0; u < kDensityBatch2D; ++u) pj[u] = A.xvB[j + u];
+                const float2* q = A.xyB + b;
+                int left = e - b;
+                for (; left >= kDensityBatch2D; left -= kDensityBatch2D, q += kDensityBatch2D) {
+                    Points<kDensityBatch2D> pj;
+                    pj.load(q);
 #pragma unroll
                     for (int u = 0; u < kDensityBatch2D; ++u) cand(pj[u]);
                 }
-                for (; j < e; ++j) cand(A.xvB[j]);
+                if (left > 0) {
+                    Points<kDensityBatch2D> pj;
+                    pj.load(q);
+#pragma unroll
+                    for (int u = 0; u < kDensityBatch2D - 1; ++u)
+                        if (u < left) cand(pj[u]);
+                }
             }
             rho = S.mass * acc;
             if (d < P.H) rho += P.psi * W_cubic(P, fmaxf(0.0f, d));
@@ -481,7 +508,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
             p = P.k * (tr * tr * tr - 1.0f);
         }
         A.rpA[i] = make_float2(rho, p);
-        A.aj[i] = make_float2(p / (rho * rho), 1.0f / rho);
+        A.qva[i] = make_float4(vx, vy, p / (rho * rho), 1.0f / rho);
         A.idfA[i] = (idf & ~(1 << 30)) | (en << 30);
     });
 }
@@ -492,8 +519,8 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
 struct ForceArgs {
     const Scene2D* sc;
     TileTable tiles;
-    const float4* q;
-    const float2* aj;
+    const float2* qxy;
+    const float4* qva;
     const int* idfA;
     const int* off;
     const float* h0;
@@ -506,22 +533,23 @@ __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
     for_each_tile<kPersistent>(A.tiles, [&](const int4 t) {
         const int i = t.y + (int)threadIdx.x;
         if (i >= t.z) return;
-        const float4 qi = A.q[i];
-        const float x = qi.x, y = qi.y, vx = qi.z, vy = qi.w;
+        const float2 xyi = A.qxy[i];
+        const float4 vai = A.qva[i];
+        const float x = xyi.x, y = xyi.y, vx = vai.x, vy = vai.y;
         const int idf = A.idfA[i];
         if (((idf >> 30) & 1) == 0) {  // disabled: pass through (:494-498)
-            A.xvA[i] = qi;
+            A.xvA[i] = make_float4(x, y, vx, vy);
             return;
         }
         const Scene2D S = A.sc[t.x];
-        const float ai = A.aj[i].x;
+        const float ai = vai.z;
         float apx = 0.0f, apy = 0.0f, avx = 0.0f, avy = 0.0f;
         const int ix = cell2(x, P.lox, P.hc, P.nx);
         const int cb = t.x * P.ncell;
         for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
             int b, e;
             column_rows(P, A.off, cb, x, y, ix, cx, b, e);
-            auto pair = [&](const float4 qj, const float2 bj) {
+            auto pair = [&](const float2 qj, const float4 va) {
                 const float dx = x - qj.x, dy = y - qj.y;
                 const float r2 = fmaf(dy, dy, dx * dx);
                 if (r2 < P.T && r2 > 0.0f) {  // r2 > 0 also excludes j == i
@@ -539,35 +567,43 @@ __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
                     }
                     const float wg = W_cubic_grad(P, r);
                     const float ux = dx * inv, uy = dy * inv;
-                    const float s = (ai + bj.x) * wg;
+                    const float s = (ai + va.z) * wg;
                     apx -= s * ux;
                     apy -= s * uy;
-                    const float vdr = (vx - qj.z) * dx + (vy - qj.w) * dy;
+                    const float vdr = (vx - va.x) * dx + (vy - va.y) * dy;
                     // dot(vij, rij) / (r^2 + 0.01 H^2) as dot * (1 / ...); the
                     // denominator lies in [2^-40, 2^40] for 2^-16 <= H <= 2^19
                     const float den = r2 + P.c01;
-                    const float tv = bj.y * vdr * recip_rn(den, __builtin_amdgcn_rcpf(den)) * wg;
+                    const float tv = va.w * vdr * recip_rn(den, __builtin_amdgcn_rcpf(den)) * wg;
                     avx -= tv * ux;
                     avy -= tv * uy;
                 }
             };
-            // kForceBatch2D candidates (position / velocity and the pressure
-            // and 1/rho pair) loaded before the first is tested; tested and
-            // accumulated in order.  Loading the pair of every candidate, not
-            // only of the neighbours, trades a few cached loads for the
-            // latency each neighbour otherwise waits on.
+            // kForceBatch2D candidates (position; velocity, pressure term and
+            // 1/rho) loaded before the first is tested; tested and accumulated in
+            // order.  Loading all of every candidate, not only of the
+            // neighbours, trades a few cached loads for the latency each
+            // neighbour otherwise waits on.
             int j = b;
             for (; j + kForceBatch2D <= e; j += kForceBatch2D) {
-                float4 qj[kForceBatch2D];
+                Points<kForceBatch2D> pj;
+                pj.load(A.qxy + j);
+                float4 va[kForceBatch2D];
 #pragma unroll
-                for (int u = 0; u < kForceBatch2D; ++u) qj[u] = A.q[j + u];
-                float2 bj[kForceBatch2D];
+                for (int u = 0; u < kForceBatch2D; ++u) va[u] = A.qva[j + u];
 #pragma unroll
-                for (int u = 0; u < kForceBatch2D; ++u) bj[u] = A.aj[j + u];
-#pragma unroll
-                for (int u = 0; u < kForceBatch2D; ++u) pair(qj[u], bj[u]);
+                for (int u = 0; u < kForceBatch2D; ++u) pair(pj[u], va[u]);
             }
-            for (; j < e; ++j) pair(A.q[j], A.aj[j]);
+            if (j < e) {
+                Points<kForceBatch2D> pj;
+                pj.load(A.qxy + j);
+                float4 va[kForceBatch2D - 1];
+#pragma unroll
+                for (int u = 0; u < kForceBatch2D - 1; ++u) va[u] = A.qva[j + u];
+#pragma unroll
+                for (int u = 0; u < kForceBatch2D - 1; ++u)
+                    if (j + u < e) pair(pj[u], va[u]);
+            }
         }
         const float cv = P.visc_pre * S.mass;
         avx *= cv;
@@ -916,12 +952,14 @@ class Batch2D {
         hip_check(hipMemcpy(wbeg_.get(), wb.data(), sizeof(int) * ns_, hipMemcpyHostToDevice), "wbeg");
 
         for (int k = 0; k < 2; ++k) {
-            xv_[k].resize(ntot_);
             rp_[k].resize(ntot_);
             idf_[k].resize(ntot_);
         }
-        q_.resize(ntot_);
-        aj_.resize(ntot_);
+        xv_.resize(ntot_);
+        xy_.resize(ntot_ + kReadPast2D);
+        vel_.resize(ntot_);
+        qxy_.resize(ntot_ + kReadPast2D);
+        qva_.resize(ntot_ + kReadPast2D);
         flux_.resize(ntot_);
         key_.resize(ntot_);
         rec_.resize(ntot_);
@@ -972,7 +1010,7 @@ class Batch2D {
         for (long long i = 0; i < 4ll * ntot_; ++i)
             if (!std::isfinite(xv[i])) throw Error(CWA_EINVAL, "non-finite particle state");
         hip_check(hipStreamSynchronize(st_), "sync");
-        hip_check(hipMemcpy(xv_[0].get(), xv, sizeof(float4) * ntot_, hipMemcpyHostToDevice), "xv");
+        hip_check(hipMemcpy(xv_.get(), xv, sizeof(float4) * ntot_, hipMemcpyHostToDevice), "xv");
         hip_check(hipMemcpy(rp_[0].get(), rp.data(), sizeof(float2) * ntot_, hipMemcpyHostToDevice), "rp");
         hip_check(hipMemcpy(idf_[0].get(), idf.data(), sizeof(int) * ntot_, hipMemcpyHostToDevice), "idf");
         std::vector<float> z(wtot_, 0.0f);
@@ -1019,7 +1057,7 @@ class Batch2D {
             const bool first = sub == 0;
             mark(B_HASH, first ? 0 : 2);
             k2_hash<<<blocks_for(ntot_, 256), 256, 0, st_>>>(
-                dev_, sc_.get(), blk_scene_.get(), xv_[0].get(), ntot_, key_.get(), rec_.get(),
+                dev_, sc_.get(), blk_scene_.get(), xv_.get(), ntot_, key_.get(), rec_.get(),
                 count_.get(), queue_.get());
             hip_check(hipGetLastError(), "hash");
             mark(B_HASH, first ? 1 : 3);
@@ -1033,19 +1071,19 @@ class Batch2D {
             mark(B_SCATTER, first ? 1 : 3);
             mark(B_REORDER, first ? 0 : 2);
             k2_reorder<<<blocks_for(std::max(ntot_, ncells_), 256), 256, 0, st_>>>(
-                key_.get(), rec_.get(), offset_.get(), runs_.get(), ntot_, xv_[0].get(),
-                rp_[0].get(), idf_[0].get(), xv_[1].get(), rp_[1].get(), idf_[1].get(),
-                count_.get(), ncells_);
+                key_.get(), rec_.get(), offset_.get(), runs_.get(), ntot_, xv_.get(),
+                rp_[0].get(), idf_[0].get(), xy_.get(), vel_.get(), rp_[1].get(),
+                idf_[1].get(), count_.get(), ncells_);
             hip_check(hipGetLastError(), "reorder");
             mark(B_REORDER, first ? 1 : 3);
 
-            DensityArgs da{sc_.get(), {td.tiles.get(), td.ntiles, nq, queue_.get(), td.len.get()}, xv_[1].get(), rp_[1].get(), idf_[1].get(), offset_.get(), h0_.get(),
-                           h1_.get(), q_.get(), rp_[0].get(), aj_.get(), idf_[0].get(), flux_.get()};
+            DensityArgs da{sc_.get(), {td.tiles.get(), td.ntiles, nq, queue_.get(), td.len.get()}, xy_.get(), vel_.get(), rp_[1].get(), idf_[1].get(), offset_.get(),
+                           h0_.get(), h1_.get(), qxy_.get(), qva_.get(), rp_[0].get(), idf_[0].get(), flux_.get()};
             mark(B_DENSITY, first ? 0 : 2);
             LaunchDensity(da, dt);
             mark(B_DENSITY, first ? 1 : 3);
-            ForceArgs fa{sc_.get(), {tf.tiles.get(), tf.ntiles, nq, queue_.get() + kNumXcd, tf.len.get()}, q_.get(), aj_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
-                         xv_[0].get()};
+            ForceArgs fa{sc_.get(), {tf.tiles.get(), tf.ntiles, nq, queue_.get() + kNumXcd, tf.len.get()}, qxy_.get(), qva_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
+                         xv_.get()};
             mark(B_FORCE, first ? 0 : 2);
             LaunchForce(fa, dt);
             mark(B_FORCE, first ? 1 : 3);
@@ -1109,7 +1147,7 @@ class Batch2D {
 
     void CheckFinite() {
         hip_check(hipMemsetAsync(finite_.get(), 0, sizeof(int), st_), "finite zero");
-        hip_check(launch_check_finite(reinterpret_cast<const float*>(xv_[0].get()), 4ull * ntot_,
+        hip_check(launch_check_finite(reinterpret_cast<const float*>(xv_.get()), 4ull * ntot_,
                                       finite_.get(), st_), "finite xv");
         hip_check(launch_check_finite(h0_.get(), (size_t)wtot_, finite_.get(), st_), "finite h0");
         int flag = 0;
@@ -1128,7 +1166,7 @@ class Batch2D {
     void Render(float* points_xy, float* wave) {
         if (points_xy) {
             k2_points<<<blocks_for(ntot_, 256), 256, 0, st_>>>(
-                xv_[0].get(), ntot_, reinterpret_cast<float2*>(points_xy));
+                xv_.get(), ntot_, reinterpret_cast<float2*>(points_xy));
             hip_check(hipGetLastError(), "render points");
         }
         if (wave)
@@ -1147,7 +1185,7 @@ class Batch2D {
         v->grid_nx = dev_.nx;
         v->grid_ny = dev_.ny;
         v->cells_total = ncells_;
-        v->xv = reinterpret_cast<float*>(xv_[0].get());
+        v->xv = reinterpret_cast<float*>(xv_.get());
         v->rp = reinterpret_cast<float*>(rp_[0].get());
         v->idf = idf_[0].get();
         v->key = key_.get();
@@ -1163,7 +1201,7 @@ class Batch2D {
         std::vector<float4> x(ntot_);
         std::vector<float2> r(ntot_);
         std::vector<int> idf(ntot_);
-        hip_check(hipMemcpy(x.data(), xv_[0].get(), sizeof(float4) * ntot_, hipMemcpyDeviceToHost), "xv");
+        hip_check(hipMemcpy(x.data(), xv_.get(), sizeof(float4) * ntot_, hipMemcpyDeviceToHost), "xv");
         hip_check(hipMemcpy(r.data(), rp_[0].get(), sizeof(float2) * ntot_, hipMemcpyDeviceToHost), "rp");
         hip_check(hipMemcpy(idf.data(), idf_[0].get(), sizeof(int) * ntot_, hipMemcpyDeviceToHost), "idf");
         for (int s = 0; s < ns_; ++s) {
@@ -1289,13 +1327,13 @@ class Batch2D {
                 hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, b.st_), "snapshot");
             };
             if (!restore) {
-                cp(xv.get(), b.xv_[0].get(), sizeof(float4) * b.ntot_);
+                cp(xv.get(), b.xv_.get(), sizeof(float4) * b.ntot_);
                 cp(rp.get(), b.rp_[0].get(), sizeof(float2) * b.ntot_);
                 cp(idf.get(), b.idf_[0].get(), sizeof(int) * b.ntot_);
                 cp(h0.get(), b.h0_.get(), sizeof(float) * b.wtot_);
                 cp(h1.get(), b.h1_.get(), sizeof(float) * b.wtot_);
             } else {
-                cp(b.xv_[0].get(), xv.get(), sizeof(float4) * b.ntot_);
+                cp(b.xv_.get(), xv.get(), sizeof(float4) * b.ntot_);
                 cp(b.rp_[0].get(), rp.get(), sizeof(float2) * b.ntot_);
                 cp(b.idf_[0].get(), idf.get(), sizeof(int) * b.ntot_);
                 cp(b.h0_.get(), h0.get(), sizeof(float) * b.wtot_);
@@ -1406,11 +1444,12 @@ class Batch2D {
     std::vector<Scene2D> host_sc_;
     DeviceBuffer<Scene2D> sc_;
     DeviceBuffer<int> blk_scene_, pbeg_, wbeg_;
-    DeviceBuffer<float4> xv_[2];
+    DeviceBuffer<float4> xv_;
+    DeviceBuffer<float2> xy_, vel_;  // sorted copy, read in order by the density pass
     DeviceBuffer<float2> rp_[2];
     DeviceBuffer<int> idf_[2];
-    DeviceBuffer<float4> q_;
-    DeviceBuffer<float2> aj_;
+    DeviceBuffer<float2> qxy_;  // what the force pass reads: positions, and velocity,
+    DeviceBuffer<float4> qva_;  // pressure term and 1/rho
     DeviceBuffer<float> flux_;
     DeviceBuffer<int> key_, rec_, count_, offset_, ws_, queue_, finite_;
     DeviceBuffer<unsigned> runs_;
