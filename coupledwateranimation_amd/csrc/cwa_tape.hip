@@ -79,12 +79,6 @@ class Tape {
                         "the scene was reinitialised or its grid, coupling band or wave mode "
                         "changed after the tape was created");
     }
-    template <class T>
-    void copy(T* dst, const T* src, size_t count) {
-        if (count)
-            hip_check(hipMemcpyAsync(dst, src, count * sizeof(T), hipMemcpyDeviceToDevice, st_),
-                      "tape copy");
-    }
 
     CoupledScene& S_;
     hipStream_t st_;
@@ -195,28 +189,32 @@ void Tape::plan_step_tape(StepTape& t) {
 
 void Tape::save(Ckpt& c) {
     const auto& A = S_.particles.A;
-    copy(c.pos.get(), A.pos, n_);
-    copy(c.vel.get(), A.vel, n_);
-    copy(c.force.get(), A.force, n_);
-    copy(c.id.get(), A.id, n_);
-    copy(c.rho.get(), S_.particles.rho(), n_);
-    copy(c.prs.get(), S_.particles.prs(), n_);
-    copy(c.h0.get(), S_.wave.GetReadImage(0), (size_t)W_ * H_);
-    copy(c.h1.get(), S_.wave.GetReadImage(1), (size_t)W_ * H_);
+    CopyList l;
+    l.add(c.pos.get(), A.pos, n_);
+    l.add(c.vel.get(), A.vel, n_);
+    l.add(c.force.get(), A.force, n_);
+    l.add(c.id.get(), A.id, n_);
+    l.add(c.rho.get(), S_.particles.rho(), n_);
+    l.add(c.prs.get(), S_.particles.prs(), n_);
+    l.add(c.h0.get(), S_.wave.GetReadImage(0), (size_t)W_ * H_);
+    l.add(c.h1.get(), S_.wave.GetReadImage(1), (size_t)W_ * H_);
+    hip_check(launch_copy_list(l, st_), "tape save");
 }
 
 void Tape::restore(const Ckpt& c, bool heights) {
     auto& A = S_.particles.A;
-    copy(A.pos, c.pos.get(), n_);
-    copy(A.vel, c.vel.get(), n_);
-    copy(A.force, c.force.get(), n_);
-    copy(A.id, c.id.get(), n_);
-    copy(S_.particles.rho(), c.rho.get(), n_);
-    copy(S_.particles.prs(), c.prs.get(), n_);
+    CopyList l;
+    l.add(A.pos, c.pos.get(), n_);
+    l.add(A.vel, c.vel.get(), n_);
+    l.add(A.force, c.force.get(), n_);
+    l.add(A.id, c.id.get(), n_);
+    l.add(S_.particles.rho(), c.rho.get(), n_);
+    l.add(S_.particles.prs(), c.prs.get(), n_);
     if (heights) {
-        copy(S_.wave.GetReadImage(0), c.h0.get(), (size_t)W_ * H_);
-        copy(S_.wave.GetReadImage(1), c.h1.get(), (size_t)W_ * H_);
+        l.add(S_.wave.GetReadImage(0), c.h0.get(), (size_t)W_ * H_);
+        l.add(S_.wave.GetReadImage(1), c.h1.get(), (size_t)W_ * H_);
     }
+    hip_check(launch_copy_list(l, st_), "tape restore");
     S_.grid.ClearCounters(st_);
 }
 
@@ -271,14 +269,12 @@ void Tape::BackwardSeeded() {
 }
 
 void Tape::reduce_partials(hipStream_t st) {
-    const int wslots[5] = {GRAD_LAMBDA_X, GRAD_LAMBDA_Z, GRAD_ATTEN, GRAD_BETA, GRAD_KAPPA};
-    const int pslots[3] = {GRAD_VISC, GRAD_GAS_CONST, GRAD_REST_RHO};
-    hip_check(launch_reduce_partials(acc_wave_.get(), (int)(acc_wave_.size() / 5), 5, wslots,
-                                     pgrad_.get(), st),
-              "reduce");
-    hip_check(launch_reduce_partials(acc_pair_.get(), (int)(acc_pair_.size() / 3), 3, pslots,
-                                     pgrad_.get(), st),
-              "reduce");
+    const PartialSums p{{acc_wave_.get(), acc_pair_.get()},
+                        {(int)(acc_wave_.size() / 5), (int)(acc_pair_.size() / 3)},
+                        {5, 3},
+                        {GRAD_LAMBDA_X, GRAD_LAMBDA_Z, GRAD_ATTEN, GRAD_BETA, GRAD_KAPPA,
+                         GRAD_VISC, GRAD_GAS_CONST, GRAD_REST_RHO}};
+    hip_check(launch_reduce_partials(p, pgrad_.get(), st), "reduce");
 }
 
 void Tape::Forward(float dt) {

@@ -144,3 +144,35 @@ def test_density_by_packed_points(gpu, cwa, oracle, shape):
     assert counts.max() > 1 or n == 1
     a, b = got[0][1]["rho"], got[1][1]["rho"]
     assert np.abs(a - b).max() <= 2 * counts.max() * 2.0 ** -24 * np.abs(b).max()
+
+
+@pytest.mark.parametrize("n,W,H", [(1, 3, 5), (2, 4, 4), (3, 7, 3), (255, 33, 31), (1025, 16, 64),
+                                   (4099, 65, 63)])
+def test_tape_copies_whole_states(gpu, cwa, n, W, H):
+    """Checkpoints and the final state come back as they were, whatever remains
+    past the last 16 bytes of an array: a backward pass (which replays the steps
+    from the checkpoints) leaves the forward's final state, and a plain run gives
+    that state too."""
+    from coupledwateranimation_amd import configs
+    from coupledwateranimation_amd.gradient import Tape
+
+    print(f"tape copies n={n} {W}x{H}", flush=True)
+    spec = configs.dam_break_diff(max(n, 64), 64, 5)
+    rng = np.random.default_rng(n)
+    vel = np.zeros((n, 4), np.float32)
+    vel[:, :3] = rng.normal(0.0, 0.3, (n, 3))
+    h = rng.normal(0.0, 0.02, (2, H, W)).astype(np.float32)
+    make = lambda: cwa.Scene(spec.params, spec.pos[:n].copy(), vel, None, (W, H),  # noqa: E731
+                             h[0], h[1])
+    with make() as plain:
+        plain.step(spec.dt, 7)
+        ref = plain.readback()
+    with make() as s:
+        tape = Tape(s, 7, 3)
+        tape.forward(spec.dt)
+        _same(s.readback(), ref, "forward")
+        grads = [tape.backward(dheight0=np.ones((H, W), np.float32)) for _ in range(2)]
+        _same(s.readback(), ref, "backward")
+        tape.close()
+    assert grads[0][0] == grads[1][0]
+    assert np.array_equal(grads[0][2], grads[1][2])
