@@ -75,6 +75,14 @@ constexpr int kPiecesPerXcd = 8;  // a scene is cut into pieces of at most this 
 // us; force 2, 4, 6 -> 1 511, 1 480, 1 497 us.
 constexpr int kDensityBatch2D = 6;
 constexpr int kForceBatch2D = 4;
+// Batches of up to this many particles run density and force with four lanes per
+// particle (quad_candidates): there a pass is one chain of candidates per wave,
+// on a chip with waves to spare.  With more, the four lanes' 16 additions a round
+// cost more than they hide.  MI355X, us a step, one lane -> four: 24 scenes of 20
+// 324 particles 55.9 -> 45.6, 8 of 32 768 59.7 -> 49.4, one of 30 000 140 -> 92, 4 of
+// 50 287 97.5 -> 68.5, 64 of 68 236 54.8 -> 51.7, 4 of 120 000 149 -> 158, 40 of 141 448
+// 73 -> 74, 10 of 254 690 189 -> 239, 160 of 700 520 150 -> 208.
+constexpr int kQuadMax2D = 80000;
 constexpr int kReadPast2D = 8;  // points a batch may load past the end of an array
 static_assert(kDensityBatch2D % 2 == 0 && kForceBatch2D % 2 == 0, "points are loaded in pairs");
 static_assert(kDensityBatch2D <= kReadPast2D && kForceBatch2D <= kReadPast2D, "padding");
@@ -368,13 +376,25 @@ __device__ __forceinline__ int next_entry(const TileTable& T) {
     return -1;
 }
 
-// Runs body(tile) for the block's tiles: entry blockIdx.x, or with
-// kPersistent the entries the block takes from the queues.
-template <bool kPersistent, class Body>
+// How a pass is laid out on the chip.
+enum class Form {
+    tiles,       // a block per tile, a lane per particle
+    quads,       // four blocks per tile, four lanes per particle
+    persistent,  // blocks that take their tiles from the queues, a lane per particle
+};
+
+// Runs body(tile, slot of the thread's particle) for the block's tiles.
+template <Form kForm, class Body>
 __device__ __forceinline__ void for_each_tile(const TileTable& T, Body&& body) {
-    if (!kPersistent) {
+    if (kForm == Form::tiles) {
         const int4 t = T.entry[blockIdx.x];
-        if (t.x >= 0) body(t);
+        if (t.x >= 0) body(t, t.y + (int)threadIdx.x);
+        return;
+    }
+    if (kForm == Form::quads) {  // a tile's four blocks on the XCD of its entry
+        const int b = blockIdx.x, q = T.nq;
+        const int4 t = T.entry[b / (4 * q) * q + b % q];
+        if (t.x >= 0) body(t, t.y + (int)((b / q % 4 * blockDim.x + threadIdx.x) / 4));
         return;
     }
     __shared__ int s_entry;
@@ -385,7 +405,7 @@ __device__ __forceinline__ void for_each_tile(const TileTable& T, Body&& body) {
         __syncthreads();
         if (e < 0) return;
         const int4 t = T.entry[e];
-        body(t);
+        body(t, t.y + (int)threadIdx.x);
     }
 }
 
@@ -412,6 +432,64 @@ struct Points {
     }
 };
 
+// The candidates of a particle shared by four lanes, in rounds of four
+// consecutive ones: load(j) gives what a lane needs of its candidate, and
+// sum(candidate, whether there is one) is called in all four lanes, round by
+// round, so that each can add the terms of the four in candidate order: the same
+// sums as one lane's, to the bit.  The lanes look up the five column ranges
+// at once, and a column's first kQuadAhead rounds are loaded while the column
+// before is summed (1, 2, 3, 4 rounds: 24 scenes 45.3, 45.6, 46.1, 46.8 us a step, 4
+// dense scenes of 120 000 particles 166, 158, 161, 166).  Force / density at 24 small
+// scenes 14.7 / 13.1 -> 9.0 / 8.5 us.
+constexpr int kQuadAhead = 2;
+template <class Load, class Sum>
+__device__ __forceinline__ void quad_candidates(const Dev2& P, const int* __restrict__ off, int cb,
+                                                float x, float y, int sub, Load&& load,
+                                                Sum&& sum) {
+    const int ix = cell2(x, P.lox, P.hc, P.nx);
+    int rb[2] = {0, 0}, re[2] = {0, 0};  // cell columns ix - 2 + sub, ix + 2 (first lane)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int cx = ix - 2 + sub + 4 * q;
+        if ((q == 0 || sub == 0) && cx >= 0 && cx < P.nx)
+            column_rows(P, off, cb, x, y, ix, cx, rb[q], re[q]);
+    }
+    int b[5] = {quad_bcast<0>(rb[0]), quad_bcast<1>(rb[0]), quad_bcast<2>(rb[0]),
+                quad_bcast<3>(rb[0]), quad_bcast<0>(rb[1])};
+    int e[5] = {quad_bcast<0>(re[0]), quad_bcast<1>(re[0]), quad_bcast<2>(re[0]),
+                quad_bcast<3>(re[0]), quad_bcast<0>(re[1])};
+    using Cand = decltype(load(0));
+    Cand next[kQuadAhead];
+    const auto ahead = [&](int first, int end) {
+#pragma unroll
+        for (int u = 0; u < kQuadAhead; ++u)
+            if (first + 4 * u < end) next[u] = load(min(first + 4 * u + sub, end - 1));
+    };
+    ahead(b[0], e[0]);
+#pragma unroll 1
+    for (int c = 0; c < 5; ++c) {
+        const int first = b[0], end = e[0];
+        Cand cur[kQuadAhead];
+#pragma unroll
+        for (int u = 0; u < kQuadAhead; ++u) cur[u] = next[u];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            b[k] = b[k + 1];
+            e[k] = e[k + 1];
+        }
+        if (c < 4) ahead(b[0], e[0]);
+        for (int j = first; j < end;) {
+#pragma unroll
+            for (int u = 0; u < kQuadAhead; ++u)
+                if (j + 4 * u < end) sum(cur[u], j + 4 * u + sub < end);
+            j += 4 * kQuadAhead;
+#pragma unroll
+            for (int u = 0; u < kQuadAhead; ++u)
+                if (j + 4 * u < end) cur[u] = load(min(j + 4 * u + sub, end - 1));
+        }
+    }
+}
+
 struct DensityArgs {
     const Scene2D* sc;
     TileTable tiles;
@@ -429,11 +507,12 @@ struct DensityArgs {
     float* flux;
 };
 
-template <int BS, bool kPersistent>
+template <int BS, Form kForm>
 __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A) {
-    for_each_tile<kPersistent>(A.tiles, [&](const int4 t) {
-        const int i = t.y + (int)threadIdx.x;
-        if (i >= t.z) return;
+    for_each_tile<kForm>(A.tiles, [&](const int4 t, const int i) {
+        if (i >= t.z) return;  // with quads the four lanes of a particle
+        constexpr bool kQuads = kForm == Form::quads;
+        const int sub = kQuads ? threadIdx.x & 3 : 0;
         const Scene2D S = A.sc[t.x];
         const float* w0 = A.h0 + S.wbeg;
         const float* w1 = A.h1 + S.wbeg;
@@ -458,7 +537,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
             vx -= 1.75f * vn * bnx;
             vy -= 1.75f * vn * bny;
         }
-        A.qxy[i] = make_float2(x, y);
+        if (sub == 0) A.qxy[i] = make_float2(x, y);
         float f = 0.0f;
         if (P.band > 0.0f) {
             const float dd = fabsf(y - wave_at(P, w0, S.L, sL, x));
@@ -468,37 +547,53 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
                 f = S.mass / P.rho0 * vy * tq * tq;
             }
         }
-        A.flux[i] = f;
+        if (sub == 0) A.flux[i] = f;
         float2 rp = A.rpB[i];
         float rho = rp.x, p = rp.y;
         if (!(y > P.hiy)) {
-            const int ix = cell2(x, P.lox, P.hc, P.nx);
             const int cb = t.x * P.ncell;
             float acc = 0.0f;
-            for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
-                int b, e;
-                column_rows(P, A.off, cb, x, y, ix, cx, b, e);
-                auto cand = [&](const float2 pj) {
-                    const float dx = x - pj.x, dy = y - pj.y;
-                    const float r2 = fmaf(dy, dy, dx * dx);
-                    if (r2 < P.HSQ) acc += W_cubic(P, sqrt_rn_clamped(r2));
-                };
-                // kDensityBatch2D candidates loaded before the first is
-                // tested; tested in order
-                const float2* q = A.xyB + b;
-                int left = e - b;
-                for (; left >= kDensityBatch2D; left -= kDensityBatch2D, q += kDensityBatch2D) {
-                    Points<kDensityBatch2D> pj;
-                    pj.load(q);
+            const auto add = [&](float w) { acc += w; };
+            // a candidate's W, given to `to` when it is a neighbour
+            const auto near = [&](const float2 pj, auto&& to) {
+                const float dx = x - pj.x, dy = y - pj.y;
+                const float r2 = fmaf(dy, dy, dx * dx);
+                if (r2 < P.HSQ) to(W_cubic(P, sqrt_rn_clamped(r2)));
+            };
+            if constexpr (kQuads) {
+                quad_candidates(
+                    P, A.off, cb, x, y, sub, [&](int j) { return A.xyB[j]; },
+                    [&](const float2 pj, bool some) {
+                        float w = 0.0f;
+                        if (some) near(pj, [&](float v) { w = v; });
+                        add(quad_bcast_f<0>(w));
+                        add(quad_bcast_f<1>(w));
+                        add(quad_bcast_f<2>(w));
+                        add(quad_bcast_f<3>(w));
+                    });
+            } else {
+                const auto cand = [&](const float2 pj) { near(pj, add); };
+                const int ix = cell2(x, P.lox, P.hc, P.nx);
+                for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
+                    int b, e;
+                    column_rows(P, A.off, cb, x, y, ix, cx, b, e);
+                    // kDensityBatch2D candidates loaded before the first is
+                    // tested; tested in order
+                    const float2* q = A.xyB + b;
+                    int left = e - b;
+                    for (; left >= kDensityBatch2D; left -= kDensityBatch2D, q += kDensityBatch2D) {
+                        Points<kDensityBatch2D> pj;
+                        pj.load(q);
 #pragma unroll
-                    for (int u = 0; u < kDensityBatch2D; ++u) cand(pj[u]);
-                }
-                if (left > 0) {
-                    Points<kDensityBatch2D> pj;
-                    pj.load(q);
+                        for (int u = 0; u < kDensityBatch2D; ++u) cand(pj[u]);
+                    }
+                    if (left > 0) {
+                        Points<kDensityBatch2D> pj;
+                        pj.load(q);
 #pragma unroll
-                    for (int u = 0; u < kDensityBatch2D - 1; ++u)
-                        if (u < left) cand(pj[u]);
+                        for (int u = 0; u < kDensityBatch2D - 1; ++u)
+                            if (u < left) cand(pj[u]);
+                    }
                 }
             }
             rho = S.mass * acc;
@@ -507,6 +602,7 @@ __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A
             const float tr = rho / P.rho0;
             p = P.k * (tr * tr * tr - 1.0f);
         }
+        if (sub != 0) return;
         A.rpA[i] = make_float2(rho, p);
         A.qva[i] = make_float4(vx, vy, p / (rho * rho), 1.0f / rho);
         A.idfA[i] = (idf & ~(1 << 30)) | (en << 30);
@@ -528,81 +624,120 @@ struct ForceArgs {
     float4* xvA;
 };
 
-template <int BS, bool kPersistent>
+template <int BS, Form kForm>
 __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
-    for_each_tile<kPersistent>(A.tiles, [&](const int4 t) {
-        const int i = t.y + (int)threadIdx.x;
-        if (i >= t.z) return;
+    for_each_tile<kForm>(A.tiles, [&](const int4 t, const int i) {
+        if (i >= t.z) return;  // with quads the four lanes of a particle
+        constexpr bool kQuads = kForm == Form::quads;
+        const int sub = kQuads ? threadIdx.x & 3 : 0;
         const float2 xyi = A.qxy[i];
         const float4 vai = A.qva[i];
         const float x = xyi.x, y = xyi.y, vx = vai.x, vy = vai.y;
         const int idf = A.idfA[i];
         if (((idf >> 30) & 1) == 0) {  // disabled: pass through (:494-498)
-            A.xvA[i] = make_float4(x, y, vx, vy);
+            if (sub == 0) A.xvA[i] = make_float4(x, y, vx, vy);
             return;
         }
         const Scene2D S = A.sc[t.x];
         const float ai = vai.z;
         float apx = 0.0f, apy = 0.0f, avx = 0.0f, avy = 0.0f;
-        const int ix = cell2(x, P.lox, P.hc, P.nx);
         const int cb = t.x * P.ncell;
-        for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
-            int b, e;
-            column_rows(P, A.off, cb, x, y, ix, cx, b, e);
-            auto pair = [&](const float2 qj, const float4 va) {
-                const float dx = x - qj.x, dy = y - qj.y;
-                const float r2 = fmaf(dy, dy, dx * dx);
-                if (r2 < P.T && r2 > 0.0f) {  // r2 > 0 also excludes j == i
-                    // r2 < T <= 2^38 (h <= 2^19); below 2^-80 the library square
-                    // root and division
-                    const bool wide = r2 < 0x1p-80f;
-                    float r, inv;
-                    if (__builtin_expect(wide, 0)) {
-                        r = sqrtf(r2);
-                        inv = 1.0f / r;
-                    } else {
-                        float h;
-                        r = sqrt_rn_mid(r2, h);
-                        inv = recip_rn(r, h + h);  // 2h: within 2 ulp of 1 / r
-                    }
-                    const float wg = W_cubic_grad(P, r);
-                    const float ux = dx * inv, uy = dy * inv;
-                    const float s = (ai + va.z) * wg;
-                    apx -= s * ux;
-                    apy -= s * uy;
-                    const float vdr = (vx - va.x) * dx + (vy - va.y) * dy;
-                    // dot(vij, rij) / (r^2 + 0.01 H^2) as dot * (1 / ...); the
-                    // denominator lies in [2^-40, 2^40] for 2^-16 <= H <= 2^19
-                    const float den = r2 + P.c01;
-                    const float tv = va.w * vdr * recip_rn(den, __builtin_amdgcn_rcpf(den)) * wg;
-                    avx -= tv * ux;
-                    avy -= tv * uy;
-                }
-            };
-            // kForceBatch2D candidates (position; velocity, pressure term and
-            // 1/rho) loaded before the first is tested; tested and accumulated in
-            // order.  Loading all of every candidate, not only of the
-            // neighbours, trades a few cached loads for the latency each
-            // neighbour otherwise waits on.
-            int j = b;
-            for (; j + kForceBatch2D <= e; j += kForceBatch2D) {
-                Points<kForceBatch2D> pj;
-                pj.load(A.qxy + j);
-                float4 va[kForceBatch2D];
-#pragma unroll
-                for (int u = 0; u < kForceBatch2D; ++u) va[u] = A.qva[j + u];
-#pragma unroll
-                for (int u = 0; u < kForceBatch2D; ++u) pair(pj[u], va[u]);
+        // A candidate's terms; false (and nothing written) for one that is no
+        // neighbour.
+        struct Terms {
+            float px = 0.0f, py = 0.0f, vx = 0.0f, vy = 0.0f;
+        };
+        const auto terms = [&](const float2 qj, const float4 va, Terms& w) {
+            const float dx = x - qj.x, dy = y - qj.y;
+            const float r2 = fmaf(dy, dy, dx * dx);
+            if (!(r2 < P.T && r2 > 0.0f)) return false;  // r2 > 0 also excludes j == i
+            // r2 < T <= 2^38 (h <= 2^19); below 2^-80 the library square
+            // root and division
+            const bool wide = r2 < 0x1p-80f;
+            float r, inv;
+            if (__builtin_expect(wide, 0)) {
+                r = sqrtf(r2);
+                inv = 1.0f / r;
+            } else {
+                float h;
+                r = sqrt_rn_mid(r2, h);
+                inv = recip_rn(r, h + h);  // 2h: within 2 ulp of 1 / r
             }
-            if (j < e) {
-                Points<kForceBatch2D> pj;
-                pj.load(A.qxy + j);
-                float4 va[kForceBatch2D - 1];
+            const float wg = W_cubic_grad(P, r);
+            const float ux = dx * inv, uy = dy * inv;
+            const float s = (ai + va.z) * wg;
+            w.px = s * ux;
+            w.py = s * uy;
+            const float vdr = (vx - va.x) * dx + (vy - va.y) * dy;
+            // dot(vij, rij) / (r^2 + 0.01 H^2) as dot * (1 / ...); the
+            // denominator lies in [2^-40, 2^40] for 2^-16 <= H <= 2^19
+            const float den = r2 + P.c01;
+            const float tv = va.w * vdr * recip_rn(den, __builtin_amdgcn_rcpf(den)) * wg;
+            w.vx = tv * ux;
+            w.vy = tv * uy;
+            return true;
+        };
+        const auto add = [&](float px, float py, float wx, float wy) {
+            apx -= px;
+            apy -= py;
+            avx -= wx;
+            avy -= wy;
+        };
+        if constexpr (kQuads) {
+            struct Cand {
+                float2 xy;
+                float4 va;
+            };
+            // a term of +0 leaves a sum as it is (the sums never hold -0)
+            quad_candidates(
+                P, A.off, cb, x, y, sub, [&](int j) { return Cand{A.qxy[j], A.qva[j]}; },
+                [&](const Cand& c, bool some) {
+                    Terms w;
+                    if (some) (void)terms(c.xy, c.va, w);
+                    add(quad_bcast_f<0>(w.px), quad_bcast_f<0>(w.py), quad_bcast_f<0>(w.vx),
+                        quad_bcast_f<0>(w.vy));
+                    add(quad_bcast_f<1>(w.px), quad_bcast_f<1>(w.py), quad_bcast_f<1>(w.vx),
+                        quad_bcast_f<1>(w.vy));
+                    add(quad_bcast_f<2>(w.px), quad_bcast_f<2>(w.py), quad_bcast_f<2>(w.vx),
+                        quad_bcast_f<2>(w.vy));
+                    add(quad_bcast_f<3>(w.px), quad_bcast_f<3>(w.py), quad_bcast_f<3>(w.vx),
+                        quad_bcast_f<3>(w.vy));
+                });
+            if (sub != 0) return;
+        } else {
+            const auto pair = [&](const float2 qj, const float4 va) {
+                Terms w;
+                if (terms(qj, va, w)) add(w.px, w.py, w.vx, w.vy);
+            };
+            const int ix = cell2(x, P.lox, P.hc, P.nx);
+            for (int cx = max(ix - 2, 0); cx <= min(ix + 2, P.nx - 1); ++cx) {
+                int b, e;
+                column_rows(P, A.off, cb, x, y, ix, cx, b, e);
+                // kForceBatch2D candidates (position; velocity, pressure term and
+                // 1/rho) loaded before the first is tested; tested and accumulated in
+                // order.  Loading all of every candidate, not only of the
+                // neighbours, trades a few cached loads for the latency each
+                // neighbour otherwise waits on.
+                int j = b;
+                for (; j + kForceBatch2D <= e; j += kForceBatch2D) {
+                    Points<kForceBatch2D> pj;
+                    pj.load(A.qxy + j);
+                    float4 va[kForceBatch2D];
 #pragma unroll
-                for (int u = 0; u < kForceBatch2D - 1; ++u) va[u] = A.qva[j + u];
+                    for (int u = 0; u < kForceBatch2D; ++u) va[u] = A.qva[j + u];
 #pragma unroll
-                for (int u = 0; u < kForceBatch2D - 1; ++u)
-                    if (j + u < e) pair(pj[u], va[u]);
+                    for (int u = 0; u < kForceBatch2D; ++u) pair(pj[u], va[u]);
+                }
+                if (j < e) {
+                    Points<kForceBatch2D> pj;
+                    pj.load(A.qxy + j);
+                    float4 va[kForceBatch2D - 1];
+#pragma unroll
+                    for (int u = 0; u < kForceBatch2D - 1; ++u) va[u] = A.qva[j + u];
+#pragma unroll
+                    for (int u = 0; u < kForceBatch2D - 1; ++u)
+                        if (j + u < e) pair(pj[u], va[u]);
+                }
             }
         }
         const float cv = P.visc_pre * S.mass;
@@ -1400,21 +1535,27 @@ class Batch2D {
     }
 
     // One block per tile, or g persistent blocks when those are fewer.
+    // kQuadMax2D's rule; persistent blocks are a tuning choice
+    bool quads() const { return ntot_ <= kQuadMax2D; }
     template <int BS>
     void LaunchDensityOf(const DensityArgs& a, float dt) {
         const int g = tune_.grid_density;
         if (g > 0 && g < a.tiles.n)
-            k2_density<BS, true><<<g, BS, 0, st_>>>(dev_, dt, a);
+            k2_density<BS, Form::persistent><<<g, BS, 0, st_>>>(dev_, dt, a);
+        else if (quads())
+            k2_density<BS, Form::quads><<<4 * a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
         else
-            k2_density<BS, false><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
+            k2_density<BS, Form::tiles><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
     }
     template <int BS>
     void LaunchForceOf(const ForceArgs& a, float dt) {
         const int g = tune_.grid_force;
         if (g > 0 && g < a.tiles.n)
-            k2_force<BS, true><<<g, BS, 0, st_>>>(dev_, dt, a);
+            k2_force<BS, Form::persistent><<<g, BS, 0, st_>>>(dev_, dt, a);
+        else if (quads())
+            k2_force<BS, Form::quads><<<4 * a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
         else
-            k2_force<BS, false><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
+            k2_force<BS, Form::tiles><<<a.tiles.n, BS, 0, st_>>>(dev_, dt, a);
     }
     void LaunchDensity(const DensityArgs& a, float dt) {
         switch (tune_.block_density) {

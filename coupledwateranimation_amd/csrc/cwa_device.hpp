@@ -413,6 +413,27 @@ __device__ __forceinline__ RunInfo wave_runs(int c) {
     return r;
 }
 
+// Lane kSrc's value, for the four lanes of an aligned group (all active).
+template <int kSrc>
+__device__ __forceinline__ int quad_bcast(int v) {
+    return __builtin_amdgcn_mov_dpp(v, kSrc * 0x55, 0xf, 0xf, true);
+}
+__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+    return v;
+}
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
+    return v;
+}
+
+template <int kSrc>
+__device__ __forceinline__ float quad_bcast_f(float v) {
+    return __int_as_float(quad_bcast<kSrc>(__float_as_int(v)));
+}
+
 // Blocks are dealt to the 8 XCDs round-robin by workgroup id; remap so that
 // XCD k runs one contiguous 1/8 of the logical blocks (its L2 then holds one
 // spatial slab of the sorted particles).  Bijective for any grid size.

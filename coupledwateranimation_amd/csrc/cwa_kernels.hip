@@ -768,22 +768,6 @@ constexpr int kDensitySplit = 4;
 constexpr int kAhead = 24;  // candidates of a column loaded ahead
 constexpr int kSplitAhead = kAhead / kDensitySplit;
 
-// Lane kSrc's value, for the four lanes of an aligned group (all active).
-template <int kSrc>
-__device__ __forceinline__ int quad_bcast(int v) {
-    return __builtin_amdgcn_mov_dpp(v, kSrc * 0x55, 0xf, 0xf, true);
-}
-__device__ __forceinline__ uint32_t quad_or(uint32_t v) {
-    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);  // lane ^ 1
-    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);  // lane ^ 2
-    return v;
-}
-__device__ __forceinline__ float quad_sum(float v) {
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
-    v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
-    return v;
-}
-
 // The lane's first U candidates of slots [b, e), every kDensitySplit-th; slots past the end
 // hold a point infinitely far away.
 template <int U>
@@ -1445,11 +1429,6 @@ __global__ void __launch_bounds__(256) k_force_integrate(
 constexpr int kForceSplit = 4;
 constexpr int kSplitWords = 8;  // words loaded ahead of their count
 constexpr int kSplitBatch = 8;
-
-template <int kSrc>
-__device__ __forceinline__ float quad_bcast_f(float v) {
-    return __int_as_float(quad_bcast<kSrc>(__float_as_int(v)));
-}
 
 // What force_finish reads, all of it already loaded.
 struct EarlyInputs {

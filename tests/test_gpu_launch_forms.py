@@ -176,3 +176,34 @@ def test_tape_copies_whole_states(gpu, cwa, n, W, H):
         tape.close()
     assert grads[0][0] == grads[1][0]
     assert np.array_equal(grads[0][2], grads[1][2])
+
+
+@pytest.mark.parametrize("counts", [(1,), (2, 3, 5), (15, 16, 17, 1), (63, 64, 65, 257), (4097, 700),
+                                    (20_000,)])
+def test_batched_pairs_with_four_lanes(gpu, cwa, counts):
+    """Batches of up to 80 000 particles sum a particle's candidates with four
+    lanes, larger ones with one: the same scenes, alone and with others that make
+    the batch large, to the bit."""
+    from coupledwateranimation_amd import batch2d
+
+    print(f"batched lanes {counts}", flush=True)
+    others = (30_000, 30_000, 30_000)
+    n, nw = sum(counts), 40 * len(counts)
+    got = []
+    for sizes in (counts, counts + others):
+        spec = batch2d.dam_break_batch(sizes, [40] * len(sizes), seed=3)
+        rng = np.random.default_rng(n)
+        spec.xv[:n, 2:] = rng.normal(0.0, 0.5, (n, 2))
+        spec.xv[:n:7, 0] = spec.xv[0, 0]  # some on a line, two points on each other
+        if n > 1:
+            spec.xv[1, :2] = spec.xv[0, :2]
+        spec.enabled = np.ones(spec.n_total, np.int32)
+        spec.enabled[:n:5] = 0
+        b = spec.make()
+        b.step(spec.dt, 3)
+        r = b.readback()
+        b.close()
+        got.append({k: np.ascontiguousarray(r[k][:n]) for k in ("xv", "rp", "enabled")} |
+                   {k: np.ascontiguousarray(r[k][:nw]) for k in ("h0", "h1")})
+    for k in got[0]:
+        assert np.array_equal(got[0][k].view(np.uint32), got[1][k].view(np.uint32)), k
