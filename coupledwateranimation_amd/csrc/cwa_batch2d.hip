@@ -15,13 +15,12 @@
 // Packing.  Scene s owns the slot range [pbeg_s, pbeg_s + n_s) and the
 // global cells [s*C, (s+1)*C) (C = nx*ny cells of size H/2, y fastest), so
 // one counting sort over all cells keeps every scene inside its own slot
-// range.  A step is 7 launches for any number of scenes:
-//   k2_hash      cell keys, wave-aggregated count atomics (run heads)
+// range.  A step is at most 7 launches for any number of scenes:
+//   k2_hash      cell keys, counts and run lists of a call's first step
 //   scan         exclusive offsets over all cells (cwa_kernels.hip)
-//   k2_scatter   run records into each cell's segment
-//   k2_reorder   stable rank from the run records; state A -> B, sorted
+//   k2_reorder   stable rank from the run lists; state A -> B, sorted
 //   k2_density   tiles; B -> q, (rho, p), (p/rho^2, 1/rho)
-//   k2_force     tiles; q -> A (forward Euler)
+//   k2_force     tiles; q -> A (forward Euler), and the next step's keys
 //   k2_wave      one workgroup per scene: column flux sums, the wave
 //                substeps in LDS, flux source; levels updated in place
 // The state ends every step in A, so a captured step replays as is.
@@ -90,8 +89,6 @@ static_assert(kDensityBatch2D <= kReadPast2D && kForceBatch2D <= kReadPast2D, "p
 // -> eight 137 -> 59 us; columns of a wave side by side instead: 149 us, and at
 // 1 024 threads 77 against 23).
 constexpr int kFluxAhead = 8;
-constexpr int kRunShift = 26;   // run record: slot | (len - 1) << 26
-constexpr unsigned kRunSlotMask = (1u << kRunShift) - 1u;
 
 // Per-scene table (device).
 struct Scene2D {
@@ -272,76 +269,74 @@ __device__ __forceinline__ void column_rows(const Dev2& P, const int* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// grid: hash / count
+// grid: hash / count.  The keys, counts and run lists (cwa_kernels.hip) of a
+// build come from k2_hash, or within one call of several steps or substeps
+// from the force pass before, which hashes the positions it writes (key null:
+// it does not).  A call's last pass leaves counts and lists empty, as the next
+// call may start from positions the caller has written.
+// Small batches are bound by their launches: two fewer a substep (the hash, and
+// the pass that placed the runs in their cells) took 20 eager steps of 24 small
+// scenes from 637 to 474 us and 10 steps of the application's scene, eight
+// copies, from 331 to 288, three batches in flight; 256 scenes unchanged.
 // ---------------------------------------------------------------------------
+struct Keys2D {
+    int* key;
+    CellRuns runs;
+};
+
+// Cell of a point of scene s.
+__device__ __forceinline__ int cell_of(const Dev2& P, int s, float x, float y) {
+    return s * P.ncell + cell2(x, P.lox, P.hc, P.nx) * P.ny + cell2(y, P.loy, P.hc, P.ny);
+}
+
 __global__ void __launch_bounds__(256)
     k2_hash(Dev2 P, const Scene2D* __restrict__ sc, const int* __restrict__ blk_scene,
-            const float4* __restrict__ xv, int ntot, int* __restrict__ key,
-            int* __restrict__ rec, int* __restrict__ count, int* __restrict__ queues) {
-    if (blockIdx.x == 0 && (int)threadIdx.x < 2 * kNumXcd) queues[threadIdx.x] = 0;
+            const float4* __restrict__ xv, int ntot, Keys2D out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
     const bool valid = i < ntot;
     int c = -1;
     if (valid) {
         int s = blk_scene[blockIdx.x];
         while (i >= sc[s].pbeg + sc[s].n) ++s;
         const float4 p = xv[i];
-        const int ix = cell2(p.x, P.lox, P.hc, P.nx);
-        const int iy = cell2(p.y, P.loy, P.hc, P.ny);
-        c = s * P.ncell + ix * P.ny + iy;
-        key[i] = c;
+        c = cell_of(P, s, p.x, p.y);
+        out.key[i] = c;
     }
-    // One atomicAdd per run of equal keys (slots of a wave are nearly
-    // sorted), issued by the run head for the whole run.
-    const RunInfo r = wave_runs(c);
-    int base = 0;
-    if (r.head && valid) base = atomicAdd(&count[c], r.run_end - lane);
-    if (valid) rec[i] = r.head ? base : -(lane - r.my_head);
+    push_runs<true, true>(c, valid, i, out.runs);
 }
 
-// Run heads write (slot, length) at their place in the cell's segment.
+// Stable destination: a run's first lane walks its cell's run list and counts
+// the items before its own slot; the run itself is contiguous.  Also clears
+// the counts for the next build (the density pass clears the lists) and the
+// tile queues.
 __global__ void __launch_bounds__(256)
-    k2_scatter(const int* __restrict__ key, const int* __restrict__ rec,
-               const int* __restrict__ offset, int ntot, unsigned* __restrict__ runs) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const bool valid = i < ntot;
-    const int c = valid ? key[i] : -1;
-    const RunInfo r = wave_runs(c);
-    if (valid && r.head) {
-        const unsigned len1 = (unsigned)(r.run_end - lane - 1);
-        runs[offset[c] + rec[i]] = (unsigned)i | (len1 << kRunShift);
-    }
-}
-
-// Stable destination: slots of the cell before this slot's run start come
-// from the runs that start earlier; the run itself is contiguous.  Also
-// clears the counts for the next build.
-__global__ void __launch_bounds__(256)
-    k2_reorder(const int* __restrict__ key, const int* __restrict__ rec,
-               const int* __restrict__ offset, const unsigned* __restrict__ runs, int ntot,
+    k2_reorder(Keys2D in, const int* __restrict__ offset, int ntot,
                const float4* __restrict__ xvA, const float2* __restrict__ rpA,
                const int* __restrict__ idfA, float2* __restrict__ xyB, float2* __restrict__ velB,
-               float2* __restrict__ rpB, int* __restrict__ idfB, int* __restrict__ count,
-               int ncells) {
+               float2* __restrict__ rpB, int* __restrict__ idfB, int ncells,
+               int* __restrict__ queues) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < ncells) count[s] = 0;
-    if (s >= ntot) return;
-    const int c = key[s];
-    const int r = rec[s];
-    const int a = r >= 0 ? s : s + r;
-    const int b = offset[c], e = offset[c + 1];
+    const int lane = threadIdx.x & 63;
+    if (s < 2 * kNumXcd) queues[s] = 0;
+    if (s < ncells) in.runs.count[s] = 0;
+    const bool valid = s < ntot;
+    const int c = valid ? in.key[s] : -1;
+    const RunInfo r = wave_runs(c);
     int rank = 0;
-    for (int p = b; p < e;) {
-        const unsigned u = runs[p];
-        const int st = (int)(u & kRunSlotMask);
-        const int len = (int)(u >> kRunShift) + 1;
-        if (st < a) rank += len;
-        p += len;
+    if (valid && r.head) {
+        const int b = offset[c];
+        int left = offset[c + 1] - b;
+        for (int q = in.runs.head[c]; q > 0 && left > 0;) {
+            const int2 u = in.runs.link[q - 1];
+            // a run the force pass listed may go on past this one's first slot
+            if (q - 1 < s) rank += min(u.y, s - (q - 1));
+            left -= max(u.y, 1);
+            q = u.x;
+        }
+        rank += b;
     }
-    const int d = b + rank + (s - a);
-    if (d < b || d >= e) return;  // only on inconsistent run records
+    const int d = __shfl(rank, r.my_head, 64) + (lane - r.my_head);
+    if (!valid || d < 0 || d >= ntot) return;  // out of range only on inconsistent lists
     const float4 p = xvA[s];
     xyB[d] = make_float2(p.x, p.y);
     velB[d] = make_float2(p.z, p.w);
@@ -505,10 +500,13 @@ struct DensityArgs {
     float2* rpA;
     int* idfA;
     float* flux;
+    int* head;  // run lists of the grid, cleared for the next build
+    int ncells;
 };
 
 template <int BS, Form kForm>
 __global__ void __launch_bounds__(BS) k2_density(Dev2 P, float dt, DensityArgs A) {
+    for (int c = blockIdx.x * BS + threadIdx.x; c < A.ncells; c += gridDim.x * BS) A.head[c] = 0;
     for_each_tile<kForm>(A.tiles, [&](const int4 t, const int i) {
         if (i >= t.z) return;  // with quads the four lanes of a particle
         constexpr bool kQuads = kForm == Form::quads;
@@ -622,21 +620,22 @@ struct ForceArgs {
     const float* h0;
     const float* h1;
     float4* xvA;
+    Keys2D next;
 };
 
 template <int BS, Form kForm>
 __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
-    for_each_tile<kForm>(A.tiles, [&](const int4 t, const int i) {
-        if (i >= t.z) return;  // with quads the four lanes of a particle
-        constexpr bool kQuads = kForm == Form::quads;
-        const int sub = kQuads ? threadIdx.x & 3 : 0;
+    constexpr bool kQuads = kForm == Form::quads;
+    const int sub = kQuads ? threadIdx.x & 3 : 0;
+    // The new position of particle i (with quads in the first of its four lanes).
+    const auto advance = [&](const int4 t, const int i) {
         const float2 xyi = A.qxy[i];
         const float4 vai = A.qva[i];
         const float x = xyi.x, y = xyi.y, vx = vai.x, vy = vai.y;
         const int idf = A.idfA[i];
         if (((idf >> 30) & 1) == 0) {  // disabled: pass through (:494-498)
             if (sub == 0) A.xvA[i] = make_float4(x, y, vx, vy);
-            return;
+            return xyi;
         }
         const Scene2D S = A.sc[t.x];
         const float ai = vai.z;
@@ -703,7 +702,7 @@ __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
                     add(quad_bcast_f<3>(w.px), quad_bcast_f<3>(w.py), quad_bcast_f<3>(w.vx),
                         quad_bcast_f<3>(w.vy));
                 });
-            if (sub != 0) return;
+            if (sub != 0) return xyi;
         } else {
             const auto pair = [&](const float2 qj, const float4 va) {
                 Terms w;
@@ -766,7 +765,27 @@ __global__ void __launch_bounds__(BS) k2_force(Dev2 P, float dt, ForceArgs A) {
         const float ax = apx + avx + P.gx + 0.0f;
         const float ay = apy + avy + P.gy + aty;
         const float v1x = vx + dt * ax, v1y = vy + dt * ay;
-        A.xvA[i] = make_float4(x + dt * v1x, y + dt * v1y, v1x, v1y);
+        const float2 x1 = make_float2(x + dt * v1x, y + dt * v1y);
+        A.xvA[i] = make_float4(x1.x, x1.y, v1x, v1y);
+        return x1;
+    };
+    for_each_tile<kForm>(A.tiles, [&](const int4 t, int i) {
+        int c = -1;
+        if (i < t.z) {  // with quads the same in the four lanes of a particle
+            const float2 p = advance(t, i);
+            if (A.next.key && sub == 0) {
+                c = cell_of(P, t.x, p.x, p.y);
+                A.next.key[i] = c;
+            }
+        }
+        if (!A.next.key) return;
+        if (kQuads) {  // the wave's 16 particles on its first lanes, in slot order
+            const int lane = threadIdx.x & 63;
+            c = __shfl(c, (lane * 4) & 63, 64);
+            if (lane >= 16) c = -1;
+            i += lane - lane / 4;
+        }
+        push_runs<true, true>(c, c >= 0, i, A.next.runs);
     });
 }
 
@@ -1097,8 +1116,8 @@ class Batch2D {
         qva_.resize(ntot_ + kReadPast2D);
         flux_.resize(ntot_);
         key_.resize(ntot_);
-        rec_.resize(ntot_);
-        runs_.resize(ntot_);
+        link_.resize(ntot_);
+        head_.resize(ncells_ + 1);
         count_.resize(ncells_ + 1);
         offset_.resize(ncells_ + 1);
         ws_.resize(scan_workspace_ints(ncells_ + 1));
@@ -1106,7 +1125,7 @@ class Batch2D {
         h0_.resize(wtot_);
         h1_.resize(wtot_);
         finite_.resize(1);
-        hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
+        ZeroLists();
         hip_check(hipMemset(offset_.get(), 0, sizeof(int) * (ncells_ + 1)), "offset zero");
         hip_check(hipMemset(key_.get(), 0, sizeof(int) * ntot_), "key zero");
 
@@ -1122,7 +1141,9 @@ class Batch2D {
     }
 
     ~Batch2D() {
-        if (graph_exec_) (void)hipGraphExecDestroy(graph_exec_);
+        for (auto& row : graph_exec_)
+            for (hipGraphExec_t e : row)
+                if (e) (void)hipGraphExecDestroy(e);
         for (auto& e : ev_)
             for (auto& x : e)
                 if (x) (void)hipEventDestroy(x);
@@ -1151,7 +1172,7 @@ class Batch2D {
         std::vector<float> z(wtot_, 0.0f);
         hip_check(hipMemcpy(h0_.get(), h0 ? h0 : z.data(), sizeof(float) * wtot_, hipMemcpyHostToDevice), "h0");
         hip_check(hipMemcpy(h1_.get(), h1 ? h1 : z.data(), sizeof(float) * wtot_, hipMemcpyHostToDevice), "h1");
-        hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
+        ZeroLists();
         hip_check(hipDeviceSynchronize(), "reinit");
     }
 
@@ -1181,47 +1202,51 @@ class Batch2D {
     const cwa2d_tuning& Tuning() const { return tune_; }
 
     // --- one step on the stream (optionally with events around kernels) ---
-    void Step(float dt, bool profile) {
+    // keyed: the force pass of the step before hashed its positions; key_next:
+    // this one's does for the next.
+    void Step(float dt, bool profile, bool keyed = false, bool key_next = false) {
         const int nq = tune_.xcd_queues ? kNumXcd : 1;
         const TileSet& td = Tiles(tune_.block_density, nq);
         const TileSet& tf = Tiles(tune_.block_force, nq);
         auto mark = [&](int slot, int which) {
             if (profile) hip_check(hipEventRecord(ev_[slot][which], st_), "event");
         };
+        const Keys2D keys{key_.get(), {count_.get(), head_.get(), link_.get()}};
         for (int sub = 0; sub < dev_.nsph; ++sub) {
             const bool first = sub == 0;
+            const bool last = sub == dev_.nsph - 1;
+            const bool hash_next = last ? key_next : true;
             mark(B_HASH, first ? 0 : 2);
-            k2_hash<<<blocks_for(ntot_, 256), 256, 0, st_>>>(
-                dev_, sc_.get(), blk_scene_.get(), xv_.get(), ntot_, key_.get(), rec_.get(),
-                count_.get(), queue_.get());
-            hip_check(hipGetLastError(), "hash");
+            if (!keyed) {
+                k2_hash<<<blocks_for(ntot_, 256), 256, 0, st_>>>(
+                    dev_, sc_.get(), blk_scene_.get(), xv_.get(), ntot_, keys);
+                hip_check(hipGetLastError(), "hash");
+            }
             mark(B_HASH, first ? 1 : 3);
             mark(B_SCAN, first ? 0 : 2);
             hip_check(launch_scan(count_.get(), offset_.get(), ncells_, ws_.get(), st_, nullptr), "scan");
             mark(B_SCAN, first ? 1 : 3);
-            mark(B_SCATTER, first ? 0 : 2);
-            k2_scatter<<<blocks_for(ntot_, 256), 256, 0, st_>>>(key_.get(), rec_.get(), offset_.get(),
-                                                                ntot_, runs_.get());
-            hip_check(hipGetLastError(), "scatter");
+            mark(B_SCATTER, first ? 0 : 2);  // the runs are listed where the keys are counted
             mark(B_SCATTER, first ? 1 : 3);
             mark(B_REORDER, first ? 0 : 2);
             k2_reorder<<<blocks_for(std::max(ntot_, ncells_), 256), 256, 0, st_>>>(
-                key_.get(), rec_.get(), offset_.get(), runs_.get(), ntot_, xv_.get(),
-                rp_[0].get(), idf_[0].get(), xy_.get(), vel_.get(), rp_[1].get(),
-                idf_[1].get(), count_.get(), ncells_);
+                keys, offset_.get(), ntot_, xv_.get(), rp_[0].get(), idf_[0].get(), xy_.get(),
+                vel_.get(), rp_[1].get(), idf_[1].get(), ncells_, queue_.get());
             hip_check(hipGetLastError(), "reorder");
             mark(B_REORDER, first ? 1 : 3);
 
             DensityArgs da{sc_.get(), {td.tiles.get(), td.ntiles, nq, queue_.get(), td.len.get()}, xy_.get(), vel_.get(), rp_[1].get(), idf_[1].get(), offset_.get(),
-                           h0_.get(), h1_.get(), qxy_.get(), qva_.get(), rp_[0].get(), idf_[0].get(), flux_.get()};
+                           h0_.get(), h1_.get(), qxy_.get(), qva_.get(), rp_[0].get(), idf_[0].get(), flux_.get(),
+                           head_.get(), ncells_};
             mark(B_DENSITY, first ? 0 : 2);
             LaunchDensity(da, dt);
             mark(B_DENSITY, first ? 1 : 3);
             ForceArgs fa{sc_.get(), {tf.tiles.get(), tf.ntiles, nq, queue_.get() + kNumXcd, tf.len.get()}, qxy_.get(), qva_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
-                         xv_.get()};
+                         xv_.get(), hash_next ? keys : Keys2D{}};
             mark(B_FORCE, first ? 0 : 2);
             LaunchForce(fa, dt);
             mark(B_FORCE, first ? 1 : 3);
+            keyed = hash_next;
         }
         mark(B_WAVE, 0);
         // untuned: the largest block, for a scene's column sums and substeps
@@ -1234,34 +1259,43 @@ class Batch2D {
     }
 
     void StepN(float dt, int steps) {
-        for (int k = 0; k < steps; ++k) Step(dt, false);
+        for (int k = 0; k < steps; ++k) Step(dt, false, k > 0, k + 1 < steps);
         if (params_.check_finite) CheckFinite();
     }
 
+    // One step a graph: by whether its keys come from the step before and whether
+    // it hashes for the next (a call of one step: neither).
     void StepGraph(float dt, int steps) {
-        if (!graph_exec_ || graph_dt_ != dt) {
-            InvalidateGraph();
-            // tile tables allocate: build them before the capture
-            const int nq = tune_.xcd_queues ? kNumXcd : 1;
-            Tiles(tune_.block_density, nq);
-            Tiles(tune_.block_force, nq);
-            hipGraph_t g = nullptr;
-            hip_check(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal), "capture");
-            try {
-                Step(dt, false);
-            } catch (...) {
-                (void)hipStreamEndCapture(st_, &g);
-                if (g) (void)hipGraphDestroy(g);
-                throw;
-            }
-            hip_check(hipStreamEndCapture(st_, &g), "end capture");
-            const hipError_t e = hipGraphInstantiate(&graph_exec_, g, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(g);
-            hip_check(e, "graph instantiate");
-            graph_dt_ = dt;
+        if (graph_dt_ != dt) InvalidateGraph();
+        graph_dt_ = dt;
+        for (int k = 0; k < steps; ++k) {
+            const bool keyed = k > 0, next = k + 1 < steps;
+            hipGraphExec_t& exec = graph_exec_[keyed][next];
+            if (!exec) CaptureGraph(exec, dt, keyed, next);
+            hip_check(hipGraphLaunch(exec, st_), "graph launch");
         }
-        for (int k = 0; k < steps; ++k) hip_check(hipGraphLaunch(graph_exec_, st_), "graph launch");
         if (params_.check_finite) CheckFinite();
+    }
+
+    void CaptureGraph(hipGraphExec_t& exec, float dt, bool keyed, bool next) {
+        // tile tables allocate: build them before the capture
+        const int nq = tune_.xcd_queues ? kNumXcd : 1;
+        Tiles(tune_.block_density, nq);
+        Tiles(tune_.block_force, nq);
+        hipGraph_t g = nullptr;
+        hip_check(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal), "capture");
+        try {
+            Step(dt, false, keyed, next);
+        } catch (...) {
+            (void)hipStreamEndCapture(st_, &g);
+            if (g) (void)hipGraphDestroy(g);
+            throw;
+        }
+        hip_check(hipStreamEndCapture(st_, &g), "end capture");
+        const hipError_t e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(g);
+        if (e != hipSuccess) exec = nullptr;
+        hip_check(e, "graph instantiate");
     }
 
     void StepProfiled(float dt, cwa2d_kernel_times* t) {
@@ -1480,11 +1514,13 @@ class Batch2D {
     };
 
     void InvalidateGraph() {
-        if (graph_exec_) {
-            (void)hipStreamSynchronize(st_);
-            (void)hipGraphExecDestroy(graph_exec_);
-            graph_exec_ = nullptr;
-        }
+        for (auto& row : graph_exec_)
+            for (hipGraphExec_t& e : row) {
+                if (!e) continue;
+                (void)hipStreamSynchronize(st_);
+                (void)hipGraphExecDestroy(e);
+                e = nullptr;
+            }
     }
 
     // The tile table for blocks of `bs` slots, its entries dealt to nq XCDs in
@@ -1537,6 +1573,10 @@ class Batch2D {
     // One block per tile, or g persistent blocks when those are fewer.
     // kQuadMax2D's rule; persistent blocks are a tuning choice
     bool quads() const { return ntot_ <= kQuadMax2D; }
+    void ZeroLists() {
+        hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
+        hip_check(hipMemset(head_.get(), 0, sizeof(int) * (ncells_ + 1)), "list zero");
+    }
     template <int BS>
     void LaunchDensityOf(const DensityArgs& a, float dt) {
         const int g = tune_.grid_density;
@@ -1592,14 +1632,14 @@ class Batch2D {
     DeviceBuffer<float2> qxy_;  // what the force pass reads: positions, and velocity,
     DeviceBuffer<float4> qva_;  // pressure term and 1/rho
     DeviceBuffer<float> flux_;
-    DeviceBuffer<int> key_, rec_, count_, offset_, ws_, queue_, finite_;
-    DeviceBuffer<unsigned> runs_;
+    DeviceBuffer<int> key_, count_, head_, offset_, ws_, queue_, finite_;
+    DeviceBuffer<int2> link_;
     DeviceBuffer<float> h0_, h1_;
     std::map<int, TileSet> tiles_;
     cwa2d_tuning tune_{};
     bool tuned_ = false;  // tune_ was set, not the initial values
     hipStream_t st_ = nullptr;
-    hipGraphExec_t graph_exec_ = nullptr;
+    hipGraphExec_t graph_exec_[2][2] = {};  // by keyed, next (StepGraph)
     float graph_dt_ = 0.0f;
     hipEvent_t ev_[CWA2D_NUM_KERNELS][4] = {};
 };

@@ -413,6 +413,29 @@ __device__ __forceinline__ RunInfo wave_runs(int c) {
     return r;
 }
 
+// Where the items of a build are counted and their runs listed: count and head
+// per cell (both zero on entry), link per item.  With head null the hash and
+// force passes only count the items.
+struct CellRuns {
+    int* count;
+    int* head;
+    int2* link;
+};
+// Counts the runs of equal cells c among the wave's consecutive items (item i
+// in this lane; invalid lanes last) and lists them, by each run's first lane.
+template <bool kCount, bool kLink>
+__device__ __forceinline__ void push_runs(int c, bool valid, int i, const CellRuns& r) {
+    const int lane = threadIdx.x & 63;
+    const RunInfo w = wave_runs(c);
+    if (w.head && valid) {
+        const int len = w.run_end - lane;
+        int older = 0;
+        if (kLink) older = atomicExch(&r.head[c], i + 1);
+        if (kCount) atomicAdd(&r.count[c], len);
+        if (kLink) r.link[i] = make_int2(older, len);
+    }
+}
+
 // Lane kSrc's value, for the four lanes of an aligned group (all active).
 template <int kSrc>
 __device__ __forceinline__ int quad_bcast(int v) {

@@ -375,19 +375,6 @@ hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
 // kFuseLinksMax particles do.  In larger ones k_link_runs lists them
 // (kFuseLinksMax gives both sides' times).
 // ---------------------------------------------------------------------------
-template <bool kCount, bool kLink>
-__device__ __forceinline__ void push_runs(int c, bool valid, int i, const CellRuns& r) {
-    const int lane = threadIdx.x & 63;
-    const RunInfo w = wave_runs(c);
-    if (w.head && valid) {
-        const int len = w.run_end - lane;
-        int older = 0;
-        if (kLink) older = atomicExch(&r.head[c], i + 1);
-        if (kCount) atomicAdd(&r.count[c], len);
-        if (kLink) r.link[i] = make_int2(older, len);
-    }
-}
-
 // Cell hash + count of particle slots (ComputeCellIndex / Index / ComputeCounts,
 // ugrid_particles_cs.glsl:90-108, with the y-fastest linearisation).
 template <bool kLink>

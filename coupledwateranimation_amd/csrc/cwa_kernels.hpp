@@ -31,14 +31,6 @@ hipError_t launch_fill_i32(int* p, int n, int v, hipStream_t st);
 // Zeroes offset[0..n] and a, b, c, d[0..n) (each may be null).
 hipError_t launch_clear_cells(int* offset, int* a, int* b, int* c, int* d, int n,
                               hipStream_t st);
-// Where the items of a build are counted and their runs listed: count and head
-// per cell (both zero on entry), link per item.  With head null the hash and
-// force passes only count the items.
-struct CellRuns {
-    int* count;
-    int* head;
-    int2* link;
-};
 // Stable counting sort of keyed items: count (keys of particle positions, or
 // given keys) with the cells' run lists, scan, reorder.
 hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* key,

@@ -207,3 +207,41 @@ def test_batched_pairs_with_four_lanes(gpu, cwa, counts):
                    {k: np.ascontiguousarray(r[k][:nw]) for k in ("h0", "h1")})
     for k in got[0]:
         assert np.array_equal(got[0][k].view(np.uint32), got[1][k].view(np.uint32)), k
+
+
+@pytest.mark.parametrize("counts", [(1,), (5, 63, 65), (1000, 2049, 17), (30_000, 30_001, 30_003)])
+@pytest.mark.parametrize("substeps", [1, 2])
+def test_batched_keys_from_the_step_before(gpu, cwa, counts, substeps):
+    """A call of several steps hashes each step's keys in the force pass before;
+    calls of one step hash them afresh.  Same grid and state to the bit, eager and
+    from graphs, also when the caller moves particles between calls."""
+    import torch
+    from coupledwateranimation_amd import batch2d
+
+    print(f"batched keys {counts} x{substeps}", flush=True)
+    spec = batch2d.dam_break_batch(counts, [33] * len(counts), seed=4)
+    spec.params.sph_substeps = substeps
+    rng = np.random.default_rng(sum(counts))
+    spec.xv[:, 2:] = rng.normal(0.0, 3.0, (spec.n_total, 2))  # cells change
+    got = []
+    for calls, graph in (([1] * 7, False), ([7], False), ([3, 1, 3], True), ([2, 5], True)):
+        b = spec.make()
+        done = 0
+        for c in calls:
+            b.step(spec.dt, c, graph=graph)
+            done += c
+        state = b.readback() | {f"slot_{k}": np.asarray(v) for k, v in b.slots().items()}
+        # the caller puts the particles elsewhere: the next call starts from there
+        class View:
+            __cuda_array_interface__ = {"data": (int(b.views().xv), False),
+                                        "shape": (spec.n_total, 4), "typestr": "<f4",
+                                        "version": 2}
+        torch.as_tensor(View(), device=gpu)[:, :2] *= 0.5
+        torch.cuda.synchronize()
+        b.step(spec.dt, 2, graph=graph)
+        state |= {f"moved_{k}": v for k, v in b.readback().items()}
+        b.close()
+        got.append(state)
+    for other in got[1:]:
+        for k, v in got[0].items():
+            assert np.array_equal(v, other[k], equal_nan=v.dtype.kind == "f"), k
