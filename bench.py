@@ -46,13 +46,14 @@ BYTES_PER_PARTICLE = {
 BYTES_PER_CELL = 8          # scan: read count + write offset
 BYTES_PER_WAVE_CELL = 12    # read h^n, h^(n-1); write h^(n+1)
 
-# Batched 2D step (SoA: xv float4, rp float2, idf int, q float4, aj float2).
+# Batched 2D step (SoA: xv float4, rp float2, idf int, sorted xy float2 and
+# vel float2, qxy float2 and qva float4).
 BYTES_PER_PARTICLE_2D = {
-    "hash": 24,      # read xv; write key, run record
-    "scatter": 8,    # read key, run record
-    "reorder": 64,   # read key, record, xv, rp, idf; write xv, rp, idf
-    "density": 68,   # read xv, rp, idf; write q, rp, aj, idf, flux
-    "force": 44,     # read q, aj, idf; write xv
+    "hash": 20,      # read xv; write key
+    "scatter": 0,    # the runs are listed by the pass that counts the keys
+    "reorder": 60,   # read key, xv, rp, idf; write xy, vel, rp, idf
+    "density": 68,   # read xy, vel, rp, idf; write qxy, qva, rp, idf, flux
+    "force": 44,     # read qxy, qva, idf; write xv
 }
 BYTES_PER_WAVE_CELL_2D = 16  # read and write both levels (substeps stay in LDS)
 
@@ -99,8 +100,8 @@ def parse():
 # rocprofv3 kernel name prefix -> (workload key, kernel key of kernel_ms)
 KERNEL_KEYS = [
     ("cwa::b2d::k2_density<", "batched", "density"), ("cwa::b2d::k2_force<", "batched", "force"),
-    ("cwa::b2d::k2_hash(", "batched", "hash"), ("cwa::b2d::k2_scatter(", "batched", "scatter"),
-    ("cwa::b2d::k2_reorder(", "batched", "reorder"), ("cwa::b2d::k2_wave(", "batched", "wave"),
+    ("cwa::b2d::k2_hash(", "batched", "hash"), ("cwa::b2d::k2_reorder(", "batched", "reorder"),
+    ("cwa::b2d::k2_wave(", "batched", "wave"),
     ("cwa::k_density(", "plain", "density"), ("cwa::k_force_integrate<", "plain", "force_integrate"),
     ("cwa::k_hash_count<", "plain", "hash"), ("cwa::k_link_runs(", "plain", "scatter"),
     ("cwa::k_stable_reorder(", "plain", "reorder"), ("cwa::k_wave4(", "plain", "wave"),

@@ -211,10 +211,11 @@ __device__ __forceinline__ void column_range(const DevParams& P, const int* __re
 // particle i are packed, in candidate order:
 //   nbw[k*n + i]                 word k, k < count
 //   nb_count(nbw, n)[i]          count, or -1: the particle has more words
-//                                than kNbEntries or a column longer than
-//                                kNbMaxColumn candidates, and its consumers
-//                                re-search its neighbours with the exact
-//                                distance test instead
+//                                than kNbEntries (in the four-lane density
+//                                pass also: a column longer than kNbMaxColumn
+//                                candidates), and its consumers re-search its
+//                                neighbours with the exact distance test
+//                                instead
 // in one buffer of nb_buffer_uint2(n) uint2 (the counts follow the words).
 // Only a particle's non-empty words are written and read back.
 // ---------------------------------------------------------------------------
@@ -315,8 +316,8 @@ struct NbCursor {
 };
 
 // Neighbours of particle i (slot i, position pi) in candidate order by the
-// exact distance test, excluding i: the path for particles with a column
-// of more than 64 candidates.
+// exact distance test, excluding i: the path for particles without a full
+// record of words.
 template <class F>
 __device__ __forceinline__ void for_each_candidate_neighbour(const DevParams& P,
                                                              const int* __restrict__ offset,
