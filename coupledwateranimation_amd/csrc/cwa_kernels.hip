@@ -66,6 +66,12 @@ __global__ void __launch_bounds__(256) k_clear_cells(ClearList l, int n) {
 // four wave totals.
 // ---------------------------------------------------------------------------
 constexpr int kScanThreads = 256;
+
+// Lists the run of counted item i (every lane of the wave calls it).
+__device__ __forceinline__ void link_runs(int i, const LinkRuns& lr) {
+    const bool valid = i < lr.n;
+    push_runs<false, true>(valid ? lr.key[i] : -1, valid, i, CellRuns{nullptr, lr.head, lr.link});
+}
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;  // 2048
 constexpr int kScanDirectTiles = 1024;  // tile prefixes summed in-kernel up to here
@@ -163,8 +169,19 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(const int* __restri
     if (zero_out2) store_items(zero_out2, base, n, z);
 }
 
+// Sum of one tile per block.  With runs listed (lr.n > 0) the blocks past the
+// tiles do k_link_runs' work: both passes only read what is there before them, and
+// a launch of its own takes about as long as either's work (MI355X, runs + sums -> one
+// launch: 300 007 particles 5.2 + 4.5 -> 5.3 us, 1 048 576 6.7 + 4.9 -> 7.2; 24 steps at
+// 300 007 1 416 -> 1 386 us).
 __global__ void __launch_bounds__(kScanThreads) k_scan_reduce(const int* __restrict__ in, int n,
-                                                              int* __restrict__ part) {
+                                                              int* __restrict__ part, int tiles,
+                                                              LinkRuns lr) {
+    static_assert(kScanThreads == 256, "the item passes' blocks");
+    if ((int)blockIdx.x >= tiles) {
+        link_runs(((int)blockIdx.x - tiles) * kScanThreads + (int)threadIdx.x, lr);
+        return;
+    }
     const int base = blockIdx.x * kScanTile + threadIdx.x * kScanItems;
     int v[kScanItems];
     load_items(in, base, n, v);
@@ -311,10 +328,21 @@ size_t scan_workspace_ints(int n) {
     return ws + (size_t)(m + kScanTile - 1) / kScanTile + 1;
 }
 
+// Runs of items that are already counted.
+__global__ void __launch_bounds__(256) k_link_runs(LinkRuns lr) {
+    link_runs(blockIdx.x * blockDim.x + threadIdx.x, lr);
+}
+
 // Whether the int arrays [a, a + na) and [b, b + nb) share memory (null: no).
 static bool overlap(const int* a, size_t na, const int* b, size_t nb) {
     const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
     return a && b && p < q + nb * sizeof(int) && q < p + na * sizeof(int);
+}
+
+static bool takes_one_launch(const int* in, const int* out, int n, const int* zero_out,
+                             const int* zero_out2) {
+    return n <= kScanOneTile * kScanOneTiles && !overlap(in, n, out, (size_t)n + 1) &&
+           !overlap(in, n, zero_out, n) && !overlap(in, n, zero_out2, n);
 }
 
 // out has n+1 entries; out[n] = total.  ws holds scan_workspace_ints(n).
@@ -322,13 +350,15 @@ static bool overlap(const int* a, size_t na, const int* b, size_t nb) {
 // Otherwise, up to kScanDirectTiles tiles the tile prefixes are summed inside
 // k_scan_down (two launches); larger inputs recurse on the tile sums.
 hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
-                       int* zero_out, int* zero_out2) {
+                       int* zero_out, int* zero_out2, const LinkRuns& lr) {
+    const int link_blocks = (lr.n + kScanThreads - 1) / kScanThreads;
+    const bool reduces = n > kScanTile && !takes_one_launch(in, out, n, zero_out, zero_out2);
+    if (lr.n > 0 && !reduces) k_link_runs<<<link_blocks, kScanThreads, 0, st>>>(lr);
     if (n <= 0) {
         k_fill_i32<<<1, 64, 0, st>>>(out, 1, 0);
         return hipGetLastError();
     }
-    if (n <= kScanOneTile * kScanOneTiles && !overlap(in, n, out, (size_t)n + 1) &&
-        !overlap(in, n, zero_out, n) && !overlap(in, n, zero_out2, n)) {
+    if (takes_one_launch(in, out, n, zero_out, zero_out2)) {
         k_scan_one<<<(n + kScanOneTile - 1) / kScanOneTile, kScanOneThreads, 0, st>>>(
             in, n, out, out + n, zero_out, zero_out2);
         return hipGetLastError();
@@ -340,7 +370,7 @@ hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
         return hipGetLastError();
     }
     int* part = ws;
-    k_scan_reduce<<<tiles, kScanThreads, 0, st>>>(in, n, part);
+    k_scan_reduce<<<tiles + link_blocks, kScanThreads, 0, st>>>(in, n, part, tiles, lr);
     if (tiles <= kScanDirectTiles) {
         k_scan_down<<<tiles, kScanThreads, 0, st>>>(in, n, part, out, out + n, zero_out,
                                                     zero_out2);
@@ -404,15 +434,6 @@ __global__ void __launch_bounds__(256) k_key_count(const int* __restrict__ key, 
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
     push_runs<true, true>(valid ? key[i] : -1, valid, i, runs);
-}
-
-// Runs of items that are already counted.
-__global__ void __launch_bounds__(256) k_link_runs(const int* __restrict__ key, int n,
-                                                   int* __restrict__ head,
-                                                   int2* __restrict__ link) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < n;
-    push_runs<false, true>(valid ? key[i] : -1, valid, i, CellRuns{nullptr, head, link});
 }
 
 // Stable destination of every item; list[d] = item_of[item] (or the item
@@ -1673,7 +1694,7 @@ hipError_t launch_key_count(const int* key, int n, const CellRuns& runs, hipStre
 
 hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    k_link_runs<<<blocks_for(n, 256), 256, 0, st>>>(key, n, head, link);
+    k_link_runs<<<blocks_for(n, 256), 256, 0, st>>>(LinkRuns{key, n, head, link});
     return hipGetLastError();
 }
 

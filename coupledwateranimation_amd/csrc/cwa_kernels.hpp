@@ -24,9 +24,18 @@ struct ParticleArrays {
 };
 
 size_t scan_workspace_ints(int n);
-// zero_out and zero_out2 (optional, n ints each) are cleared in the same pass.
+// Items that are counted, whose runs are still to be listed (n 0: none).
+struct LinkRuns {
+    const int* key;
+    int n;
+    int* head;
+    int2* link;
+};
+// zero_out and zero_out2 (optional, n ints each) are cleared in the same pass;
+// lr's runs are listed in it or beside it.
 hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
-                       int* zero_out = nullptr, int* zero_out2 = nullptr);
+                       int* zero_out = nullptr, int* zero_out2 = nullptr,
+                       const LinkRuns& lr = LinkRuns{});
 hipError_t launch_fill_i32(int* p, int n, int v, hipStream_t st);
 // Zeroes offset[0..n] and a, b, c, d[0..n) (each may be null).
 hipError_t launch_clear_cells(int* offset, int* a, int* b, int* c, int* d, int n,

@@ -103,16 +103,18 @@ void UniformGrid3D::BuildGrid(const ParticleArrays& A, int n, float4* bpos, int*
         hip_check(launch_hash_count(A.pos, n, g_, key, runs, st), "hash");
     mark(K_HASH, 1);
     keys_ready_ = false;
+    // a profiled build lists the runs by themselves, so that both have times of their own
+    const LinkRuns lr{key, fuse_links_ ? 0 : n, head, runs.link};
     mark(K_SCAN, 0);
     hip_check(launch_scan(runs.count, off, nc, ws_.get(), st, count_[cur_ ^ 1].get(),
-                          head_[cur_ ^ 1].get()),
+                          head_[cur_ ^ 1].get(), ev ? LinkRuns{} : lr),
               "scan");
     mark(K_SCAN, 1);
     last_ = cur_;
     cur_ ^= 1;
     last_kc_ = kc_;
     mark(K_SCATTER, 0);
-    if (!fuse_links_) hip_check(launch_link_runs(key, n, head, runs.link, st), "link runs");
+    if (ev && lr.n > 0) hip_check(launch_link_runs(key, n, head, runs.link, st), "link runs");
     mark(K_SCATTER, 1);
     mark(K_REORDER, 0);
     hip_check(launch_stable_reorder(key, off, head, runs.link, n, nullptr, lst, A.pos, A.id, bpos,

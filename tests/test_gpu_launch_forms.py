@@ -245,3 +245,28 @@ def test_batched_keys_from_the_step_before(gpu, cwa, counts, substeps):
     for other in got[1:]:
         for k, v in got[0].items():
             assert np.array_equal(v, other[k], equal_nan=v.dtype.kind == "f"), k
+
+
+@pytest.mark.parametrize("n", [262_144, 262_145, 270_011])
+@pytest.mark.parametrize("coarse", [1, 2])
+def test_runs_listed_beside_the_scan(gpu, cwa, n, coarse):
+    """Builds of more than 2^18 particles list their runs in the scan's launch of
+    tile sums, or by themselves where the scan takes one launch (65 536 cells or
+    fewer): the list is the stable order of the keys on each."""
+    from coupledwateranimation_amd import configs
+
+    print(f"runs beside the scan n={n} coarse={coarse}", flush=True)
+    spec = configs.dam_break_large(3, n=n, wave=64)
+    p = spec.params.copy()
+    p.cell_size *= coarse
+    for a in range(3):
+        p.grid_dims[a] = max(1, -(-p.grid_dims[a] // coarse))
+    rng = np.random.default_rng(n)
+    vel = np.zeros_like(spec.pos)
+    vel[:, :3] = rng.normal(0.0, 1.0, (n, 3))
+    with cwa.Scene(p, spec.pos, vel, None, spec.wave_size, spec.height0, spec.height1) as s:
+        s.step(spec.dt, 3)
+        g = s.grid_host()
+    assert np.array_equal(g["list"], np.argsort(g["key"], kind="stable"))
+    assert np.array_equal(g["count"], np.bincount(g["key"], minlength=g["count"].size))
+    assert np.array_equal(g["offset"], np.concatenate([[0], np.cumsum(g["count"])]))
