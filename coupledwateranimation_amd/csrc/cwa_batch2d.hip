@@ -51,6 +51,7 @@
 #include <map>
 #include <numeric>
 #include <string>
+#include <tuple>
 #include <vector>
 
 #include "../../include/cwa2d.h"
@@ -1141,9 +1142,8 @@ class Batch2D {
     }
 
     ~Batch2D() {
-        for (auto& row : graph_exec_)
-            for (hipGraphExec_t e : row)
-                if (e) (void)hipGraphExecDestroy(e);
+        for (auto& g : graphs_)
+            if (g.second) (void)hipGraphExecDestroy(g.second);
         for (auto& e : ev_)
             for (auto& x : e)
                 if (x) (void)hipEventDestroy(x);
@@ -1263,21 +1263,40 @@ class Batch2D {
         if (params_.check_finite) CheckFinite();
     }
 
-    // One step a graph: by whether its keys come from the step before and whether
-    // it hashes for the next (a call of one step: neither).
+    // Steps of a captured run: whether its keys come from the step before it, and
+    // whether it hashes for a step after it (Step).
+    struct GraphForm {
+        bool keyed, next;
+        int steps;
+        bool operator<(const GraphForm& o) const {
+            return std::tie(keyed, next, steps) < std::tie(o.keyed, o.next, o.steps);
+        }
+    };
+    static constexpr int kGraphSteps = 8;
+
+    // Graphs of up to kGraphSteps steps, captured when first needed: a call of that
+    // many is one of them, a longer one a first step, runs of kGraphSteps and the
+    // rest.  Every replay between two steps costs the host a launch and the GPU
+    // a gap (MI355X, three batches in flight, a graph a step -> these: 6 steps of 19
+    // scenes of 6 601 particles 203 -> 122 us a call, 60 steps 1 260 -> 766, 10 steps of
+    // the application's scene, eight copies, 311 -> 237; graphs of 4 and 16 steps: 161 and
+    // 128, 784 and 757, 238 and 236).
     void StepGraph(float dt, int steps) {
         if (graph_dt_ != dt) InvalidateGraph();
         graph_dt_ = dt;
-        for (int k = 0; k < steps; ++k) {
-            const bool keyed = k > 0, next = k + 1 < steps;
-            hipGraphExec_t& exec = graph_exec_[keyed][next];
-            if (!exec) CaptureGraph(exec, dt, keyed, next);
+        for (int done = 0; done < steps;) {
+            const int left = steps - done;
+            const int n = left <= kGraphSteps ? left : done == 0 ? 1 : kGraphSteps;
+            const GraphForm form{done > 0, left > n, n};
+            hipGraphExec_t& exec = graphs_[form];
+            if (!exec) CaptureGraph(exec, dt, form);
             hip_check(hipGraphLaunch(exec, st_), "graph launch");
+            done += n;
         }
         if (params_.check_finite) CheckFinite();
     }
 
-    void CaptureGraph(hipGraphExec_t& exec, float dt, bool keyed, bool next) {
+    void CaptureGraph(hipGraphExec_t& exec, float dt, const GraphForm& f) {
         // tile tables allocate: build them before the capture
         const int nq = tune_.xcd_queues ? kNumXcd : 1;
         Tiles(tune_.block_density, nq);
@@ -1285,7 +1304,8 @@ class Batch2D {
         hipGraph_t g = nullptr;
         hip_check(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal), "capture");
         try {
-            Step(dt, false, keyed, next);
+            for (int k = 0; k < f.steps; ++k)
+                Step(dt, false, f.keyed || k > 0, f.next || k + 1 < f.steps);
         } catch (...) {
             (void)hipStreamEndCapture(st_, &g);
             if (g) (void)hipGraphDestroy(g);
@@ -1514,13 +1534,11 @@ class Batch2D {
     };
 
     void InvalidateGraph() {
-        for (auto& row : graph_exec_)
-            for (hipGraphExec_t& e : row) {
-                if (!e) continue;
-                (void)hipStreamSynchronize(st_);
-                (void)hipGraphExecDestroy(e);
-                e = nullptr;
-            }
+        if (graphs_.empty()) return;
+        (void)hipStreamSynchronize(st_);
+        for (auto& g : graphs_)
+            if (g.second) (void)hipGraphExecDestroy(g.second);
+        graphs_.clear();
     }
 
     // The tile table for blocks of `bs` slots, its entries dealt to nq XCDs in
@@ -1639,7 +1657,7 @@ class Batch2D {
     cwa2d_tuning tune_{};
     bool tuned_ = false;  // tune_ was set, not the initial values
     hipStream_t st_ = nullptr;
-    hipGraphExec_t graph_exec_[2][2] = {};  // by keyed, next (StepGraph)
+    std::map<GraphForm, hipGraphExec_t> graphs_;
     float graph_dt_ = 0.0f;
     hipEvent_t ev_[CWA2D_NUM_KERNELS][4] = {};
 };

@@ -224,7 +224,8 @@ def test_batched_keys_from_the_step_before(gpu, cwa, counts, substeps):
     rng = np.random.default_rng(sum(counts))
     spec.xv[:, 2:] = rng.normal(0.0, 3.0, (spec.n_total, 2))  # cells change
     got = []
-    for calls, graph in (([1] * 7, False), ([7], False), ([3, 1, 3], True), ([2, 5], True)):
+    for calls, graph in (([1] * 23, False), ([23], False), ([3, 1, 8, 9, 2], True),
+                         ([6, 17], True), ([23], True)):
         b = spec.make()
         done = 0
         for c in calls:
