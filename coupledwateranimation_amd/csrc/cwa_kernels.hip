@@ -1126,71 +1126,96 @@ __device__ __forceinline__ void column_flux_sum(const int* __restrict__ offset,
 // sample (column_flux_sum's order, so the same bits) into LDS, kTileColBatch
 // columns of a wave at a time; tiles are small enough that this takes a few
 // rounds (wave_tiles_for gives the rule).
+//
+// That rule went by the parameters of the launch.  A graph replayed with others
+// keeps its tiles, so how much of a tile is advanced at once is decided here,
+// by the columns it samples with the parameters the kernel reads: the whole
+// tile while their sums fit in the LDS, else parts of half the side, a quarter,
+// ... (a single texel samples at most four columns).
 // ---------------------------------------------------------------------------
 constexpr int kTileColBatch = 4;
+// Column sums a block has room for, the neighbour words' LDS; colflux_quad may
+// load one more (the column east of the last), whose value it does not use.
+constexpr int kTileColumnsHeld = kNbStage * 256 * 2 - 1;
 
 __device__ __forceinline__ void wave_tile(const DevParams& P, const WaveTiles& w, int tile,
                                           const int* __restrict__ offset,
                                           const float* __restrict__ pflux, float dt,
                                           float* __restrict__ s_col) {
     const int tx = tile % w.nx, ty = tile / w.nx;
-    const int i_lo = tx * w.side, j_lo = ty * w.side;
-    const int i_hi = min(i_lo + w.side, P.W) - 1, j_hi = min(j_lo + w.side, P.H) - 1;
-    if (j_lo >= P.H) return;  // padding blocks
+    if (ty * w.side >= P.H) return;  // padding blocks
     const int nx = P.dims[0], ny = P.dims[1], nz = P.dims[2];
-    int x0 = 0, z0 = 0, ncx = 0;
     const bool flux = pflux != nullptr;
-    if (flux) {
-        // column coordinates are monotone in the texel index, so the tile's
-        // first and last texels bound what it samples
-        const int xa = floor_index(column_x(P, i_lo), nx), xb = floor_index(column_x(P, i_hi), nx);
-        const int za = floor_index(column_z(P, j_lo), nz), zb = floor_index(column_z(P, j_hi), nz);
-        x0 = min(max(min(xa, xb), 0), nx - 1);
-        z0 = min(max(min(za, zb), 0), nz - 1);
-        ncx = min(max(max(xa, xb) + 1, 0), nx - 1) - x0 + 1;
-        const int ncz = min(max(max(za, zb) + 1, 0), nz - 1) - z0 + 1;
-        const int nc = min(ncx * ncz, kWaveTileColumns);  // wave_tiles_for's bound
-        const int lane = threadIdx.x & 63;
-        for (int q0 = ((int)threadIdx.x >> 6) * kTileColBatch; q0 < nc; q0 += 4 * kTileColBatch) {
-            int k[kTileColBatch], e[kTileColBatch], longest = 0;
-            float s[kTileColBatch];
-#pragma unroll
-            for (int u = 0; u < kTileColBatch; ++u) {
-                s[u] = 0.0f;
-                k[u] = e[u] = 0;
-                if (q0 + u < nc) {
-                    const int c = grid_column(P.dims, x0 + (q0 + u) % ncx, z0 + (q0 + u) / ncx);
-                    k[u] = offset[c * ny];
-                    e[u] = offset[(c + 1) * ny];
-                }
+    for (int side = w.side, level = 0, part = 0; part >> (2 * level) == 0; ++part) {
+        const int i_lo = tx * w.side + (part & ((1 << level) - 1)) * side;
+        const int j_lo = ty * w.side + (part >> level) * side;
+        if (i_lo >= P.W || j_lo >= P.H) continue;
+        const int i_hi = min(i_lo + side, P.W) - 1, j_hi = min(j_lo + side, P.H) - 1;
+        int x0 = 0, z0 = 0, ncx = 0;
+        if (flux) {
+            // column coordinates are monotone in the texel index, so the part's
+            // first and last texels bound what it samples
+            const int xa = floor_index(column_x(P, i_lo), nx);
+            const int xb = floor_index(column_x(P, i_hi), nx);
+            const int za = floor_index(column_z(P, j_lo), nz);
+            const int zb = floor_index(column_z(P, j_hi), nz);
+            x0 = min(max(min(xa, xb), 0), nx - 1);
+            z0 = min(max(min(za, zb), 0), nz - 1);
+            ncx = min(max(max(xa, xb) + 1, 0), nx - 1) - x0 + 1;
+            const int ncz = min(max(max(za, zb) + 1, 0), nz - 1) - z0 + 1;
+            if ((long long)ncx * ncz > kTileColumnsHeld) {  // again, in parts of half the side
+                side >>= 1;
+                ++level;
+                part = -1;
+                continue;
             }
-#pragma unroll
-            for (int u = 0; u < kTileColBatch; ++u) {
-                longest = max(longest, e[u] - k[u]);
-                k[u] += lane;
-            }
-            for (; longest > 0; longest -= 64) {
+            const int nc = ncx * ncz;
+            const int lane = threadIdx.x & 63;
+            if (level > 0) __syncthreads();  // the part before has read its columns
+            for (int q0 = ((int)threadIdx.x >> 6) * kTileColBatch; q0 < nc;
+                 q0 += 4 * kTileColBatch) {
+                int k[kTileColBatch], e[kTileColBatch], longest = 0;
+                float s[kTileColBatch];
 #pragma unroll
                 for (int u = 0; u < kTileColBatch; ++u) {
-                    if (k[u] < e[u]) s[u] += pflux[k[u]];
-                    k[u] += 64;
+                    s[u] = 0.0f;
+                    k[u] = e[u] = 0;
+                    if (q0 + u < nc) {
+                        const int c = grid_column(P.dims, x0 + (q0 + u) % ncx, z0 + (q0 + u) / ncx);
+                        k[u] = offset[c * ny];
+                        e[u] = offset[(c + 1) * ny];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kTileColBatch; ++u) {
+                    longest = max(longest, e[u] - k[u]);
+                    k[u] += lane;
+                }
+                for (; longest > 0; longest -= 64) {
+#pragma unroll
+                    for (int u = 0; u < kTileColBatch; ++u) {
+                        if (k[u] < e[u]) s[u] += pflux[k[u]];
+                        k[u] += 64;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kTileColBatch; ++u) {
+                    s[u] = wave_sum_f32(s[u]);
+                    if (lane == 0 && q0 + u < nc) s_col[q0 + u] = s[u];
                 }
             }
-#pragma unroll
-            for (int u = 0; u < kTileColBatch; ++u) {
-                s[u] = wave_sum_f32(s[u]);
-                if (lane == 0 && q0 + u < nc) s_col[q0 + u] = s[u];
-            }
+            __syncthreads();
         }
-        __syncthreads();
+        const auto cf = [&](int ix, int iz) { return s_col[(iz - z0) * ncx + (ix - x0)]; };
+        const int per = P.W % 4 == 0 && side % 4 == 0 ? 4 : 1;  // texels per thread along u
+        const int across = side / per;  // a power of two; across * side <= 256 threads
+        const int i = i_lo + ((int)threadIdx.x & (across - 1)) * per;
+        const int j = j_lo + ((int)threadIdx.x >> __builtin_ctz(across));
+        if (i <= i_hi && j <= j_hi) {
+            if (per == 4) wave_quad(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
+            else wave_single(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
+        }
     }
-    const auto cf = [&](int ix, int iz) { return s_col[(iz - z0) * ncx + (ix - x0)]; };
-    const int per = P.W % 4 == 0 ? 4 : 1;  // texels per thread along u
-    const int across = w.side / per;       // across * side <= 256 threads
-    const int i = i_lo + (int)threadIdx.x % across * per, j = j_lo + (int)threadIdx.x / across;
-    if (i > i_hi || j > j_hi) return;
-    if (per == 4) wave_quad(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
-    else wave_single(P, w.h0, w.h1, w.out, i, j, flux, cf, dt);
 }
 
 // What the force pass writes (fpre: only for the adjoint tape).
@@ -1354,7 +1379,7 @@ __global__ void __launch_bounds__(256) k_force_integrate(
     const float* __restrict__ H0, ForceOut out, int nfb, const float* __restrict__ pflux, float* __restrict__ colflux, NextKeys next, WaveTiles wt) {
     const DevParams& P = *Pd;
     __shared__ uint2 s_nb[kNbStage][256];
-    static_assert(sizeof(s_nb) >= kWaveTileColumns * sizeof(float), "a tile's column sums");
+    static_assert(sizeof(s_nb) >= (kTileColumnsHeld + 1) * sizeof(float), "a tile's column sums");
     if (kWave && (int)blockIdx.x < wt.nblk) {
         wave_tile(P, wt, blockIdx.x, offset, colflux ? pflux : nullptr, dt,
                   reinterpret_cast<float*>(&s_nb[0][0]));

@@ -108,7 +108,7 @@ struct WaveTiles {
     float* out;
     int nblk, nx, side;
 };
-constexpr int kWaveTileColumns = 128;  // columns a tile's samples may touch
+constexpr int kWaveTileColumns = 128;  // columns a tile's samples may touch when it is chosen
 constexpr int kFuseWaveParticles = 1 << 16;
 constexpr int kFuseWaveTiles = 512;
 static_assert(kFuseWaveParticles <= kFuseLinksMax, "tiles go with the fused run lists");

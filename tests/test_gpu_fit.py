@@ -106,6 +106,46 @@ def test_fit_graph_reads_updated_parameters(gpu, cwa):
         sc.close()
 
 
+@pytest.mark.parametrize("cells,wave,factors", [
+    (20, 64, (0.25, 1.0, 2.0)), (20, 61, (0.3,)), (100, 512, (1 / 16, 1 / 64, 1 / 1024))])
+def test_fit_graph_follows_the_wave_scale(gpu, cwa, cells, wave, factors):
+    """The heightfield spread over more of the grid, or less, than when the fit
+    was captured: a tile's texels then sample more columns than the tile was
+    chosen for (at 0.25 all 20 x 20, with 100 x 100 more than one tile can hold)."""
+    from coupledwateranimation_amd import configs
+    from coupledwateranimation_amd.fit import FitBatch
+    from coupledwateranimation_amd.scene import Scene
+
+    spec = configs.dam_break_diff(3000, wave, 9)
+    p = spec.params
+    p.mass *= (1.0 / cells / p.h) ** 3
+    p.h = 1.0 / cells
+    configs.grid_for_box(p, (0.0, 0.0, 0.0), (1.0, 1.0, 1.0), p.h)
+    assert p.grid_dims[0] == p.grid_dims[2] == cells
+    steps = 6
+    target = np.zeros((wave, wave), np.float32)
+    with Scene(p, spec.pos, spec.vel, None, spec.wave_size, spec.height0, spec.height1) as sc:
+        fb = FitBatch([sc], [target], steps, 3, spec.dt)
+        for f in factors:
+            _say(f"wave scale {cells} cells {wave}^2 x {f}")
+            q = p.copy()
+            q.wave_uv_scale[:] = [f * v for v in p.wave_uv_scale]
+            sc.set_params(q)
+            (loss,), (grad,) = fb.run()
+            with Scene(q, spec.pos, spec.vel, None, spec.wave_size, spec.height0,
+                       spec.height1) as plain:
+                plain.step_profiled(spec.dt, steps)  # the wave in a launch of its own
+                ref = plain.readback()
+            got = sc.readback()
+            for k in ("height0", "height1", "pos"):
+                assert np.array_equal(got[k], ref[k]), (f, k)
+            loss_e, g_e = _eager(spec, q, target, steps, 3)
+            assert _rel(loss, loss_e) < 1e-9, f
+            for k in SCALARS:
+                assert _rel(grad[k], g_e[k]) < 1e-4, (f, k, grad[k], g_e[k])
+        fb.close()
+
+
 def test_descent_lowers_every_loss(gpu, cwa):
     """The accepted loss of every scene never rises (rejected proposals
     halve the step) and ends below the initial one, and the mean error of
