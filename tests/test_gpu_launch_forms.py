@@ -40,6 +40,33 @@ def test_wave_in_the_force_launch(gpu, cwa, n, W, H, band):
     _same(*states, (n, W, H, band))
 
 
+@pytest.mark.parametrize("sx,sz", [(1, 1), (-1, 1), (1, -1), (-1, -1)])
+@pytest.mark.parametrize("n,W,H", [(4096, 128, 100), (4096, 131, 64), (50_000, 256, 256)])
+def test_wave_tiles_mirrored_and_replayed(gpu, cwa, n, W, H, sx, sz):
+    """A heightfield mirrored along an axis, stepped eagerly, from graphs and with
+    the wave in a launch of its own."""
+    from coupledwateranimation_amd import configs
+
+    print(f"wave tiles n={n} {W}x{H} {sx} {sz}", flush=True)
+    spec = configs.dam_break_diff(n, 64, 5)
+    p = spec.params.copy()
+    for a, sign in ((0, sx), (1, sz)):
+        if sign < 0:
+            p.wave_origin[a] += 1.0 / p.wave_uv_scale[a]
+            p.wave_uv_scale[a] *= -1.0
+    h = np.random.default_rng(n).normal(0.0, 0.02, (2, H, W)).astype(np.float32)
+    states = []
+    for form in ("step", "graph", "profiled"):
+        with cwa.Scene(p, spec.pos, spec.vel, None, (W, H), h[0], h[1]) as s:
+            if form == "profiled":
+                s.step_profiled(spec.dt, 15)
+            else:
+                s.step(spec.dt, 15, graph=form == "graph")
+            states.append(s.readback())
+    _same(states[0], states[2], "eager")
+    _same(states[1], states[2], "graph")
+
+
 @pytest.mark.parametrize("n", [1, 8191, 8192, 8193, 65_535, 65_536, 65_537])
 @pytest.mark.parametrize("form", ["apart", "misaligned", "in place"])
 def test_scan_in_one_launch(gpu, cwa, n, form):
