@@ -1201,6 +1201,20 @@ class Batch2D {
     }
     const cwa2d_tuning& Tuning() const { return tune_; }
 
+    // The launches of a call.  Between its steps the counts and run lists hold the
+    // next step's keys; a call that fails there leaves them so, and the next
+    // one, which hashes afresh, clears them first.
+    template <class F>
+    void WithLists(F&& launches) {
+        if (lists_left_)
+            hip_check(launch_clear_cells(nullptr, count_.get(), head_.get(), nullptr, nullptr,
+                                         ncells_, st_),
+                      "clear lists");
+        lists_left_ = true;
+        launches();
+        lists_left_ = false;
+    }
+
     // --- one step on the stream (optionally with events around kernels) ---
     // keyed: the force pass of the step before hashed its positions; key_next:
     // this one's does for the next.
@@ -1259,7 +1273,9 @@ class Batch2D {
     }
 
     void StepN(float dt, int steps) {
-        for (int k = 0; k < steps; ++k) Step(dt, false, k > 0, k + 1 < steps);
+        WithLists([&] {
+            for (int k = 0; k < steps; ++k) Step(dt, false, k > 0, k + 1 < steps);
+        });
         if (params_.check_finite) CheckFinite();
     }
 
@@ -1284,15 +1300,24 @@ class Batch2D {
     void StepGraph(float dt, int steps) {
         if (graph_dt_ != dt) InvalidateGraph();
         graph_dt_ = dt;
-        for (int done = 0; done < steps;) {
-            const int left = steps - done;
-            const int n = left <= kGraphSteps ? left : done == 0 ? 1 : kGraphSteps;
-            const GraphForm form{done > 0, left > n, n};
+        const auto each_run = [&](auto&& f) {
+            for (int done = 0; done < steps;) {
+                const int left = steps - done;
+                const int n = left <= kGraphSteps ? left : done == 0 ? 1 : kGraphSteps;
+                f(GraphForm{done > 0, left > n, n});
+                done += n;
+            }
+        };
+        // all of them before the first runs: a capture that fails leaves the state as it was
+        each_run([&](const GraphForm& form) {
             hipGraphExec_t& exec = graphs_[form];
             if (!exec) CaptureGraph(exec, dt, form);
-            hip_check(hipGraphLaunch(exec, st_), "graph launch");
-            done += n;
-        }
+        });
+        WithLists([&] {
+            each_run([&](const GraphForm& form) {
+                hip_check(hipGraphLaunch(graphs_[form], st_), "graph launch");
+            });
+        });
         if (params_.check_finite) CheckFinite();
     }
 
@@ -1319,7 +1344,7 @@ class Batch2D {
     }
 
     void StepProfiled(float dt, cwa2d_kernel_times* t) {
-        Step(dt, true);
+        WithLists([&] { Step(dt, true); });
         hip_check(hipStreamSynchronize(st_), "sync");
         for (int k = 0; k < CWA2D_NUM_KERNELS; ++k) {
             float ms = 0.0f;
@@ -1435,7 +1460,7 @@ class Batch2D {
         for (auto& c : cands) {
             snap.Restore(*this);
             SetTuning(c.t);
-            Step(dt, false);  // warm caches and tiles for this setting
+            WithLists([&] { Step(dt, false); });  // warm caches and tiles for this setting
             snap.Restore(*this);
             for (int k = 0; k < steps; ++k) {
                 StepProfiled(dt, &kt);
@@ -1594,6 +1619,7 @@ class Batch2D {
     void ZeroLists() {
         hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
         hip_check(hipMemset(head_.get(), 0, sizeof(int) * (ncells_ + 1)), "list zero");
+        lists_left_ = false;
     }
     template <int BS>
     void LaunchDensityOf(const DensityArgs& a, float dt) {
@@ -1655,6 +1681,7 @@ class Batch2D {
     DeviceBuffer<float> h0_, h1_;
     std::map<int, TileSet> tiles_;
     cwa2d_tuning tune_{};
+    bool lists_left_ = false;  // a call ended before its last step (WithLists)
     bool tuned_ = false;  // tune_ was set, not the initial values
     hipStream_t st_ = nullptr;
     std::map<GraphForm, hipGraphExec_t> graphs_;
