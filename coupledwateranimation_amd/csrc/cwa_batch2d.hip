@@ -1135,7 +1135,10 @@ class Batch2D {
         tune_.grid_density = 0;
         tune_.grid_force = 0;
         tune_.xcd_queues = 1;
-        tune_.wave_block = 256;
+        // the largest block, for a scene's column sums and substeps (MI355X, 256
+        // threads -> 1 024: 256 scenes 59 -> 23 us, 24 small ones 16.3 -> 9.3, the
+        // application's scene 6.2 both)
+        tune_.wave_block = 1024;
         tune_.ms_per_step = 0.0f;
         for (auto& e : ev_)
             for (auto& x : e) hip_check(hipEventCreate(&x), "event");
@@ -1196,7 +1199,6 @@ class Batch2D {
         if (t.grid_density < 0 || t.grid_force < 0) throw Error(CWA_EINVAL, "grid must be >= 0");
         tune_ = t;
         tune_.xcd_queues = t.xcd_queues ? 1 : 0;
-        tuned_ = true;
         InvalidateGraph();
     }
     const cwa2d_tuning& Tuning() const { return tune_; }
@@ -1263,10 +1265,7 @@ class Batch2D {
             keyed = hash_next;
         }
         mark(B_WAVE, 0);
-        // untuned: the largest block, for a scene's column sums and substeps
-        // (MI355X, 256 threads -> 1 024: 256 scenes 59 -> 23 us, 24 small ones
-        // 16.3 -> 9.3, the application's scene 6.2 both)
-        k2_wave<<<ns_, tuned_ ? tune_.wave_block : 1024, lds_bytes_, st_>>>(dev_, dt, sc_.get(), offset_.get(),
+        k2_wave<<<ns_, tune_.wave_block, lds_bytes_, st_>>>(dev_, dt, sc_.get(), offset_.get(),
                                                              flux_.get(), h0_.get(), h1_.get(), lmax_);
         hip_check(hipGetLastError(), "wave");
         mark(B_WAVE, 1);
@@ -1682,7 +1681,6 @@ class Batch2D {
     std::map<int, TileSet> tiles_;
     cwa2d_tuning tune_{};
     bool lists_left_ = false;  // a call ended before its last step (WithLists)
-    bool tuned_ = false;  // tune_ was set, not the initial values
     hipStream_t st_ = nullptr;
     std::map<GraphForm, hipGraphExec_t> graphs_;
     float graph_dt_ = 0.0f;

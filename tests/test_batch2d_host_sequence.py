@@ -64,3 +64,13 @@ def test_a_failed_capture_runs_nothing(run, nth):
     assert rc < 0 and lines[-1] == "failed instantiation"
     assert not any(x.startswith(("replay", "launch")) for x in lines)
     assert rc1 == 0 and _launches(after, "k2_wave") == 20 and _launches(after, "k2_hash") == 1
+
+
+def test_settings_read_are_the_settings_that_run(run):
+    """The wave pass's block as get_tuning reports it, before and after another
+    setting is written back with it."""
+    _, (_, first), _, (_, second) = run("tuning")
+    name, threads = first[0].split()
+    assert name == "wave_block"
+    for lines in (first, second):
+        assert [x.split()[2] for x in lines if x.startswith("launch k2_wave ")] == [threads]
