@@ -1501,10 +1501,10 @@ class Batch2D {
                 best.wave_block = wbk;
             }
         }
-        // the chosen setting, timed as a graph replay
+        // the chosen setting, timed as graph replays: the same call before, for its captures
         snap.Restore(*this);
         SetTuning(best);
-        StepGraph(dt, 1);
+        StepGraph(dt, steps);
         Sync();
         snap.Restore(*this);
         hipEvent_t a = ev_[0][0], b = ev_[0][1];

@@ -74,3 +74,13 @@ def test_settings_read_are_the_settings_that_run(run):
     assert name == "wave_block"
     for lines in (first, second):
         assert [x.split()[2] for x in lines if x.startswith("launch k2_wave ")] == [threads]
+
+
+def test_the_tuner_times_replays_alone(run):
+    """No graph is captured between the events that time the chosen setting."""
+    ((rc, lines),) = run("tune")
+    assert rc == 0
+    first, last = [k for k, x in enumerate(lines) if x == "event"][-2:]
+    timed = lines[first + 1:last]
+    assert _launches(timed, "k2_wave") == 3
+    assert "replay" in timed and "capture" not in timed
