@@ -405,8 +405,9 @@ hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
 // The wave layout (blocks of 256 over the same item range) is identical in
 // both item passes, so both see the same runs.  The lists need no offsets, so
 // whoever counts the keys can also list the runs; builds of up to
-// kFuseLinksMax particles do.  In larger ones k_link_runs lists them
-// (kFuseLinksMax gives both sides' times).
+// kFuseLinksMax particles do.  In larger ones k_link_runs lists them, and in large
+// builds outside a scene k_place_runs puts them side by side in their cell's
+// segment instead (kFuseLinksMax and kListRunsMax give both sides' times).
 // ---------------------------------------------------------------------------
 // Cell hash + count of particle slots (ComputeCellIndex / Index / ComputeCounts,
 // ugrid_particles_cs.glsl:90-108, with the y-fastest linearisation).
@@ -429,18 +430,38 @@ __global__ void __launch_bounds__(256) k_hash_count(const float4* __restrict__ p
 }
 
 // Count and runs of items whose keys are already known.
+template <bool kLink>
 __global__ void __launch_bounds__(256) k_key_count(const int* __restrict__ key, int n,
                                                    CellRuns runs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool valid = i < n;
-    push_runs<true, true>(valid ? key[i] : -1, valid, i, runs);
+    push_runs<true, kLink>(valid ? key[i] : -1, valid, i, runs);
+}
+
+// The runs of counted items at a place in their cells' segments: (first item, length)
+// at the place of the run's first lane, which leaves as many free as the run has
+// items.  fill: zero on entry.
+__global__ void __launch_bounds__(256) k_place_runs(const int* __restrict__ key,
+                                                    const int* __restrict__ offset,
+                                                    int* __restrict__ fill, int n,
+                                                    int2* __restrict__ runs) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool valid = i < n;
+    const int c = valid ? key[i] : -1;
+    const RunInfo r = wave_runs(c);
+    if (valid && r.head) {
+        const int len = r.run_end - (int)(threadIdx.x & 63);
+        runs[offset[c] + atomicAdd(&fill[c], len)] = make_int2(i, len);
+    }
 }
 
 // Stable destination of every item; list[d] = item_of[item] (or the item
 // itself), and the particle positions and ids move to their sorted slots
 // when pos_out is set (the passes that follow read velocities and forces in
 // their pre-sort slots through list).  The walk ends with the cell's count,
-// whatever the links hold.
+// whatever the links hold.  kLists: the cells' run lists, else the runs placed in
+// their segments (link; head is not used).
+template <bool kLists>
 __global__ void __launch_bounds__(256) k_stable_reorder(
     const int* __restrict__ key, const int* __restrict__ offset, const int* __restrict__ head,
     const int2* __restrict__ link, int n, const int* __restrict__ item_of,
@@ -455,12 +476,21 @@ __global__ void __launch_bounds__(256) k_stable_reorder(
     int rank = 0;
     if (valid && r.head) {
         const int b = offset[c];
-        int left = offset[c + 1] - b;
-        for (int q = head[c]; q > 0 && left > 0;) {
-            const int2 u = link[q - 1];
-            if (q - 1 < s) rank += u.y;
-            left -= max(u.y, 1);
-            q = u.x;
+        const int e = offset[c + 1];
+        if (kLists) {
+            int left = e - b;
+            for (int q = head[c]; q > 0 && left > 0;) {
+                const int2 u = link[q - 1];
+                if (q - 1 < s) rank += u.y;
+                left -= max(u.y, 1);
+                q = u.x;
+            }
+        } else {
+            for (int q = b; q < e;) {
+                const int2 u = link[q];
+                if (u.x < s) rank += u.y;
+                q += max(u.y, 1);
+            }
         }
         rank += b;
     }
@@ -1713,7 +1743,8 @@ hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* k
 
 hipError_t launch_key_count(const int* key, int n, const CellRuns& runs, hipStream_t st) {
     if (n <= 0) return hipSuccess;
-    k_key_count<<<blocks_for(n, 256), 256, 0, st>>>(key, n, runs);
+    if (runs.head) k_key_count<true><<<blocks_for(n, 256), 256, 0, st>>>(key, n, runs);
+    else k_key_count<false><<<blocks_for(n, 256), 256, 0, st>>>(key, n, runs);
     return hipGetLastError();
 }
 
@@ -1723,15 +1754,22 @@ hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStr
     return hipGetLastError();
 }
 
+hipError_t launch_place_runs(const int* key, const int* offset, int* fill, int n, int2* runs,
+                             hipStream_t st) {
+    if (n <= 0) return hipSuccess;
+    k_place_runs<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, fill, n, runs);
+    return hipGetLastError();
+}
+
 hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,
                                  const int2* link, int n, const int* item_of, int* list,
                                  const float4* pos_in, const int* id_in, float4* pos_out,
                                  int* id_out, hipStream_t st, const DevParams* Pd,
                                  uint32_t* packed_out) {
     if (n <= 0) return hipSuccess;
-    k_stable_reorder<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, head, link, n, item_of, list,
-                                                         pos_in, id_in, pos_out, id_out, Pd,
-                                                         packed_out);
+    const auto kernel = head ? k_stable_reorder<true> : k_stable_reorder<false>;
+    kernel<<<blocks_for(n, 256), 256, 0, st>>>(key, offset, head, link, n, item_of, list, pos_in,
+                                               id_in, pos_out, id_out, Pd, packed_out);
     return hipGetLastError();
 }
 

@@ -46,6 +46,8 @@ hipError_t launch_hash_count(const float4* pos, int n, const GridDesc& g, int* k
                              const CellRuns& runs, hipStream_t st);
 hipError_t launch_key_count(const int* key, int n, const CellRuns& runs, hipStream_t st);
 hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStream_t st);
+hipError_t launch_place_runs(const int* key, const int* offset, int* fill, int n, int2* runs,
+                             hipStream_t st);
 // Builds of up to this many particles list their runs in the pass that counts
 // the keys, larger ones in a pass of their own: each run's push waits for its
 // exchange, at the end of waves that hold the force pass's LDS.  A launch less
@@ -54,8 +56,20 @@ hipError_t launch_link_runs(const int* key, int n, int* head, int2* link, hipStr
 // 27.2 us, 300 007 71.0 / 71.1 us, 1 048 576 285 / 276 us; the first step's
 // hash pass at 1 048 576 particles 51 / 32 us).
 constexpr int kFuseLinksMax = 1 << 18;
+// Grid builds outside a scene, whose items come in any order, place their runs in
+// the cells' segments (launch_place_runs) above these numbers of points and of
+// (box, cell) pairs.  With a run per item, a list is one load from anywhere for
+// every item of the cell; placed runs lie side by side (MI355X, listed ->
+// placed, random points in 100^3, 50^3 and 25^3 cells: 700 000 points 117 -> 112,
+// 126 -> 132, 241 -> 234 us, 1 000 000 158 -> 150, 200 -> 180, 472 -> 412, 2 000 000
+// 339 -> 297, 632 -> 480, 2 751 -> 1 907; points nearly in order, 1 000 000: 57 -> 54,
+// 73 -> 75, 144 -> 151.  Pairs of boxes: 540 000 144 -> 172, 2 160 000 554 -> 559,
+// 3 240 000 1 059 -> 1 011, 5 400 000 3 143 -> 2 746).
+constexpr int kListRunsMax = 3 << 18;
+constexpr int kListPairsMax = 1 << 21;
 // list[d] = item_of ? item_of[s] : s at each item's stable destination d;
-// with pos_out set, pos_out[d] = pos_in[s] and id_out[d] = id_in[s], and with
+// head null: link holds the runs placed in the cells' segments.  With pos_out
+// set, pos_out[d] = pos_in[s] and id_out[d] = id_in[s], and with
 // packed_out set also (Pd: the device parameters) packed_out[d] =
 // pack_point(pos_in[s]).
 hipError_t launch_stable_reorder(const int* key, const int* offset, const int* head,

@@ -1085,6 +1085,21 @@ int cwa_scan_exclusive_i32(const int32_t* d_in, int32_t* d_out, int n, void* str
     });
 }
 
+// The list of a build whose keys are counted and scanned: fused, the counting pass
+// has listed the runs; else they are listed here, or placed in their cells'
+// segments (kListRunsMax gives the rule).  head: zero where nothing is listed yet.
+static void insert_items(const int* key, const int* offset, int* head, int2* link, int n,
+                         bool fused, bool placed, const int* item_of, int* list,
+                         hipStream_t st) {
+    if (placed)
+        hip_check(launch_place_runs(key, offset, head, n, link, st), "place runs");
+    else if (!fused)
+        hip_check(launch_link_runs(key, n, head, link, st), "link runs");
+    hip_check(launch_stable_reorder(key, offset, placed ? nullptr : head, link, n, item_of, list,
+                                    nullptr, nullptr, nullptr, nullptr, st),
+              "stable insert");
+}
+
 int cwa_grid_build(const float* d_pos4, int n, const float grid_min[3], float cell_size,
                    const int32_t dims[3], int32_t* d_key, int32_t* d_count, int32_t* d_offset,
                    int32_t* d_list, void* stream) {
@@ -1114,10 +1129,8 @@ int cwa_grid_build(const float* d_pos4, int n, const float grid_min[3], float ce
                                     st),
                   "hash");
         hip_check(launch_scan(d_count, d_offset, nc, ws.get(), st), "scan");
-        if (!fuse) hip_check(launch_link_runs(d_key, n, head.get(), link.get(), st), "link runs");
-        hip_check(launch_stable_reorder(d_key, d_offset, head.get(), link.get(), n, nullptr,
-                                        d_list, nullptr, nullptr, nullptr, nullptr, st),
-                  "stable insert");
+        insert_items(d_key, d_offset, head.get(), link.get(), n, fuse, n > kListRunsMax, nullptr,
+                     d_list, st);
         hip_check(hipStreamSynchronize(st), "grid sync");
     });
 }
@@ -1157,10 +1170,7 @@ int cwa_grid_build_static(const float* d_pos4, int n, const float grid_min[3], f
                                     st),
                   "hash");
         hip_check(launch_scan(d_count, d_offset, nc, ws, st), "scan");
-        if (!fuse) hip_check(launch_link_runs(d_key, n, head, link, st), "link runs");
-        hip_check(launch_stable_reorder(d_key, d_offset, head, link, n, nullptr, d_list, nullptr,
-                                        nullptr, nullptr, nullptr, st),
-                  "stable insert");
+        insert_items(d_key, d_offset, head, link, n, fuse, n > kListRunsMax, nullptr, d_list, st);
     });
 }
 
@@ -1207,7 +1217,8 @@ int cwa_grid_build_boxes(const float* d_centre4, const float* d_halfw4, int n,
         const size_t np = (size_t)std::max(npairs, 1);
         DeviceBuffer<int> pkey(np), pbox(np), head(nc);
         DeviceBuffer<int2> link(np);
-        const CellRuns runs{d_count, head.get(), link.get()};
+        const bool fuse = npairs <= kListPairsMax;
+        const CellRuns runs{d_count, fuse ? head.get() : nullptr, link.get()};
         hip_check(launch_box_pairs(x, hw, n, grid_min, cell_size, dims, first.get(), pkey.get(),
                                    pbox.get(), st),
                   "pairs");
@@ -1215,10 +1226,8 @@ int cwa_grid_build_boxes(const float* d_centre4, const float* d_halfw4, int n,
                   "clear");
         hip_check(launch_key_count(pkey.get(), npairs, runs, st), "count");
         hip_check(launch_scan(d_count, d_offset, nc, ws.get(), st), "scan");
-        hip_check(launch_stable_reorder(pkey.get(), d_offset, head.get(), link.get(), npairs,
-                                        pbox.get(), d_list, nullptr, nullptr, nullptr, nullptr,
-                                        st),
-                  "stable insert");
+        insert_items(pkey.get(), d_offset, head.get(), link.get(), npairs, fuse, !fuse, pbox.get(),
+                     d_list, st);
         hip_check(hipStreamSynchronize(st), "box grid sync");
     });
 }

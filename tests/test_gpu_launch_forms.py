@@ -298,3 +298,68 @@ def test_runs_listed_beside_the_scan(gpu, cwa, n, coarse):
     assert np.array_equal(g["list"], np.argsort(g["key"], kind="stable"))
     assert np.array_equal(g["count"], np.bincount(g["key"], minlength=g["count"].size))
     assert np.array_equal(g["offset"], np.concatenate([[0], np.cumsum(g["count"])]))
+
+
+@pytest.mark.parametrize("n", [262_144, 262_145, 786_432, 786_433, 1_000_003])
+@pytest.mark.parametrize("order", ["random", "nearly", "one cell"])
+@pytest.mark.parametrize("static", [False, True])
+def test_grid_builds_in_any_order(gpu, cwa, n, order, static):
+    """Builds of up to 2^18 points list their runs where the keys are counted, up to
+    3 * 2^18 in a pass of their own, larger ones place them in the cells' segments:
+    the stable order of the keys on each."""
+    import ctypes as C
+
+    import torch
+    from coupledwateranimation_amd import _lib
+
+    print(f"grid build n={n} {order} static={static}", flush=True)
+    cells = 20
+    rng = np.random.default_rng(n)
+    pos = np.ones((n, 4), np.float32)
+    pos[:, :3] = rng.random((n, 3)) * (0.9 / cells if order == "one cell" else 1.0)
+    if order == "nearly":
+        c = np.minimum((pos[:, :3] * cells).astype(np.int64), cells - 1)
+        near = (c[:, 2] * cells + c[:, 0]) * cells + c[:, 1] + rng.integers(-2, 3, n)
+        pos = pos[np.argsort(near, kind="stable")]
+    d = torch.tensor(pos, device=gpu)
+    key, cnt, off, lst = [torch.full((k,), -1, dtype=torch.int32, device=gpu)
+                          for k in (n, cells ** 3, cells ** 3 + 1, n)]
+    fn = cwa.lib().cwa_grid_build_static if static else cwa.lib().cwa_grid_build
+    _lib.check(fn(d.data_ptr(), n, (C.c_float * 3)(0, 0, 0), 1.0 / cells,
+                  (C.c_int32 * 3)(cells, cells, cells), key.data_ptr(), cnt.data_ptr(),
+                  off.data_ptr(), lst.data_ptr(), None))
+    torch.cuda.synchronize()
+    k = key.cpu().numpy()
+    count = np.bincount(k, minlength=cells ** 3)
+    assert np.array_equal(lst.cpu().numpy(), np.argsort(k, kind="stable"))
+    assert np.array_equal(cnt.cpu().numpy(), count)
+    assert np.array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(count)]))
+
+
+@pytest.mark.parametrize("n,listed", [(350_000, True), (370_000, False)])
+def test_box_grids_of_many_pairs(gpu, cwa, oracle, n, listed):
+    """The same with boxes over about six cells each: fewer and more pairs than
+    2^21, against the oracle."""
+    import ctypes as C
+
+    import torch
+    from coupledwateranimation_amd import _lib
+
+    cells = 20
+    rng = np.random.default_rng(n)
+    x, h = np.ones((n, 4), np.float32), np.full((n, 4), 0.02, np.float32)
+    x[:, :3] = 0.1 + 0.8 * rng.random((n, 3))
+    ref = oracle.grid_build_boxes(x, h, (0.0,) * 3, (1.0 / cells,) * 3, (cells,) * 3)
+    print(f"box grid n={n} pairs={ref['total']}", flush=True)
+    assert (ref["total"] <= 1 << 21) == listed
+    cap, total = ref["total"], C.c_int64()
+    dx, dh = torch.tensor(x, device=gpu), torch.tensor(h, device=gpu)
+    got = {k: torch.full((m,), -1, dtype=torch.int32, device=gpu)
+           for k, m in (("count", cells ** 3), ("offset", cells ** 3 + 1), ("list", cap))}
+    _lib.check(cwa.lib().cwa_grid_build_boxes(
+        dx.data_ptr(), dh.data_ptr(), n, (C.c_float * 3)(0, 0, 0),
+        (C.c_float * 3)(*[1.0 / cells] * 3), (C.c_int32 * 3)(cells, cells, cells),
+        *[got[k].data_ptr() for k in ("count", "offset", "list")], cap, C.byref(total), None))
+    assert total.value == cap
+    for k, v in got.items():
+        assert np.array_equal(v.cpu().numpy(), ref[k]), k
