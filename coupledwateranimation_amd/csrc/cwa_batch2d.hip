@@ -1287,10 +1287,16 @@ class Batch2D {
             return std::tie(keyed, next, steps) < std::tie(o.keyed, o.next, o.steps);
         }
     };
-    static constexpr int kGraphSteps = 8;
+    // Steps a graph holds: what a capture costs the first call grows with its
+    // launches, what a longer run saves does not (a call of 6 steps of 32 substeps,
+    // captures included: 7.1 ms from graphs of one step, 11.1 of six).
+    static constexpr int kGraphSteps = 8, kGraphLaunches = 176;
+    int graph_steps() const {
+        return std::min(std::max(kGraphLaunches / (5 * dev_.nsph + 1), 1), kGraphSteps);
+    }
 
-    // Graphs of up to kGraphSteps steps, captured when first needed: a call of that
-    // many is one of them, a longer one a first step, runs of kGraphSteps and the
+    // Graphs of up to graph_steps() steps, captured when first needed: a call of that
+    // many is one of them, a longer one a first step, runs of that many and the
     // rest.  Every replay between two steps costs the host a launch and the GPU
     // a gap (MI355X, three batches in flight, a graph a step -> these: 6 steps of 19
     // scenes of 6 601 particles 203 -> 122 us a call, 60 steps 1 260 -> 766, 10 steps of
@@ -1299,10 +1305,11 @@ class Batch2D {
     void StepGraph(float dt, int steps) {
         if (graph_dt_ != dt) InvalidateGraph();
         graph_dt_ = dt;
+        const int most = graph_steps();
         const auto each_run = [&](auto&& f) {
             for (int done = 0; done < steps;) {
                 const int left = steps - done;
-                const int n = left <= kGraphSteps ? left : done == 0 ? 1 : kGraphSteps;
+                const int n = left <= most ? left : done == 0 ? 1 : most;
                 f(GraphForm{done > 0, left > n, n});
                 done += n;
             }

@@ -5,6 +5,7 @@
 //
 //   host_sequence step_fails N     the N-th launch of step(3) fails, then step(1)
 //   host_sequence graph_fails N    the N-th instantiation of step_graph(20) fails, then again
+//   host_sequence graph_first N    step_graph(6) with N SPH substeps
 //   host_sequence tuning           the wave pass before and after settings are written back
 //   host_sequence tune             the tuner
 #include <cxxabi.h>
@@ -171,6 +172,7 @@ hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
     return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) {
+    say("captured " + std::to_string(captured.size()));
     *g = new ihipGraph{captured};
     capturing = nullptr;
     return hipSuccess;
@@ -203,6 +205,7 @@ int main(int argc, char** argv) {
     const int nth = argc > 2 ? std::atoi(argv[2]) : 0;
     cwa2d_params p;
     cwa2d_params_reference(&p);
+    if (what == "graph_first") p.sph_substeps = nth;
     std::vector<cwa2d_scene> sc(2);
     std::vector<float> xv;
     for (auto& s : sc) {
@@ -231,6 +234,8 @@ int main(int argc, char** argv) {
         instantiations_left = nth;
         done(cwa2d_batch_step_graph(b, 1e-3f, 20));
         done(cwa2d_batch_step_graph(b, 1e-3f, 20));
+    } else if (what == "graph_first") {
+        done(cwa2d_batch_step_graph(b, 1e-3f, 6));
     } else if (what == "tuning") {
         cwa2d_tuning t;
         done(cwa2d_batch_get_tuning(b, &t));

@@ -84,3 +84,19 @@ def test_the_tuner_times_replays_alone(run):
     timed = lines[first + 1:last]
     assert _launches(timed, "k2_wave") == 3
     assert "replay" in timed and "capture" not in timed
+
+
+@pytest.mark.parametrize("substeps", [1, 2, 4, 5, 8, 16, 32, 64])
+def test_the_first_call_from_graphs_captures_little(run, substeps):
+    """Graphs of several steps are for steps of few launches: a call captures no more
+    than 200 launches a graph, or three steps (a first one, one of the middle
+    and a last one)."""
+    ((rc, lines),) = run("graph_first", substeps)
+    launches = sum(x.startswith("launch ") for x in lines)
+    captured = [int(x.split()[1]) for x in lines if x.startswith("captured ")]
+    assert rc == 0 and _launches(lines, "k2_wave") == 6
+    per_step = launches / 6
+    assert max(captured) <= max(200, per_step + 1)
+    assert sum(captured) <= max(launches, 3 * per_step + 1)
+    if substeps >= 32:
+        assert sum(captured) <= 3 * per_step + 1
