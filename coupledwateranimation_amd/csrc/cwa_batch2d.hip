@@ -83,6 +83,13 @@ constexpr int kForceBatch2D = 4;
 // 50 287 97.5 -> 68.5, 64 of 68 236 54.8 -> 51.7, 4 of 120 000 149 -> 158, 40 of 141 448
 // 73 -> 74, 10 of 254 690 189 -> 239, 160 of 700 520 150 -> 208.
 constexpr int kQuadMax2D = 80000;
+// Batches with more cells than this per particle clear the run lists of the cells that
+// hold particles, in a launch of its own; others clear all of them beside the
+// density pass.  MI355X, us a call of 6 steps, all -> the particles' cells: 64 scenes
+// of 100 particles with 1 600 cells a particle 476 -> 450, with 10 000 1 945 -> 1 595, with
+// 40 000 6 246 -> 5 334 (5 827 before builds had lists); one of 500 with 2 000 301 -> 286.
+// With few cells a particle the launch costs more than it saves.
+constexpr int kSparseCells = 1024;
 constexpr int kReadPast2D = 8;  // points a batch may load past the end of an array
 static_assert(kDensityBatch2D % 2 == 0 && kForceBatch2D % 2 == 0, "points are loaded in pairs");
 static_assert(kDensityBatch2D <= kReadPast2D && kForceBatch2D <= kReadPast2D, "padding");
@@ -345,6 +352,12 @@ __global__ void __launch_bounds__(256)
     idfB[d] = idfA[s];
 }
 
+// Empties the run lists of the cells that hold particles, for the next build.
+__global__ void __launch_bounds__(256) k2_clear_lists(Keys2D in, int ntot) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < ntot) in.runs.head[in.key[i]] = 0;
+}
+
 // ---------------------------------------------------------------------------
 // tiles
 // ---------------------------------------------------------------------------
@@ -502,7 +515,7 @@ struct DensityArgs {
     int* idfA;
     float* flux;
     int* head;  // run lists of the grid, cleared for the next build
-    int ncells;
+    int ncells;  // (0: k2_clear_lists does)
 };
 
 template <int BS, Form kForm>
@@ -1253,8 +1266,12 @@ class Batch2D {
 
             DensityArgs da{sc_.get(), {td.tiles.get(), td.ntiles, nq, queue_.get(), td.len.get()}, xy_.get(), vel_.get(), rp_[1].get(), idf_[1].get(), offset_.get(),
                            h0_.get(), h1_.get(), qxy_.get(), qva_.get(), rp_[0].get(), idf_[0].get(), flux_.get(),
-                           head_.get(), ncells_};
+                           head_.get(), sparse() ? 0 : ncells_};
             mark(B_DENSITY, first ? 0 : 2);
+            if (sparse()) {
+                k2_clear_lists<<<blocks_for(ntot_, 256), 256, 0, st_>>>(keys, ntot_);
+                hip_check(hipGetLastError(), "clear lists");
+            }
             LaunchDensity(da, dt);
             mark(B_DENSITY, first ? 1 : 3);
             ForceArgs fa{sc_.get(), {tf.tiles.get(), tf.ntiles, nq, queue_.get() + kNumXcd, tf.len.get()}, qxy_.get(), qva_.get(), idf_[0].get(), offset_.get(), h0_.get(), h1_.get(),
@@ -1622,6 +1639,7 @@ class Batch2D {
     // One block per tile, or g persistent blocks when those are fewer.
     // kQuadMax2D's rule; persistent blocks are a tuning choice
     bool quads() const { return ntot_ <= kQuadMax2D; }
+    bool sparse() const { return ncells_ / kSparseCells > ntot_; }
     void ZeroLists() {
         hip_check(hipMemset(count_.get(), 0, sizeof(int) * (ncells_ + 1)), "count zero");
         hip_check(hipMemset(head_.get(), 0, sizeof(int) * (ncells_ + 1)), "list zero");

@@ -275,6 +275,30 @@ def test_batched_keys_from_the_step_before(gpu, cwa, counts, substeps):
             assert np.array_equal(v, other[k], equal_nan=v.dtype.kind == "f"), k
 
 
+@pytest.mark.parametrize("h", [0.02, 0.01, 0.004])
+@pytest.mark.parametrize("counts", [(1,), (5, 63, 64, 65), (700,)])
+def test_batched_keys_in_sparse_grids(gpu, cwa, counts, h):
+    """The same with 14 to 250 000 cells a particle: run lists cleared cell by cell
+    or, with more than 1 024, particle by particle."""
+    from coupledwateranimation_amd import batch2d
+
+    print(f"batched sparse {counts} h={h}", flush=True)
+    spec = batch2d.dam_break_batch(counts, [33] * len(counts), seed=4, dt=1e-4,
+                                   params=batch2d.unit_square_params(h=h))
+    rng = np.random.default_rng(sum(counts))
+    spec.xv[:, 2:] = rng.normal(0.0, 20.0, (spec.n_total, 2))
+    got = []
+    for calls, graph in (([1] * 9, False), ([9], False), ([9], True)):
+        b = spec.make()
+        for c in calls:
+            b.step(spec.dt, c, graph=graph)
+        got.append(b.readback())
+        b.close()
+    for other in got[1:]:
+        for k, v in got[0].items():
+            assert np.array_equal(v, other[k], equal_nan=v.dtype.kind == "f"), k
+
+
 @pytest.mark.parametrize("n", [262_144, 262_145, 270_011])
 @pytest.mark.parametrize("coarse", [1, 2])
 def test_runs_listed_beside_the_scan(gpu, cwa, n, coarse):
