@@ -1464,6 +1464,9 @@ __global__ void __launch_bounds__(256) k_force_integrate(
             }
         }
     }
+    // a particle without neighbours that loaded for its partner: its own record
+    // has no weight, but may hold an infinity or NaN
+    if (nw <= 0) a = PairAcc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     int cell = -1;
     if (valid) {
         if (nw < 0)

@@ -128,6 +128,32 @@ def test_force_with_four_lanes(gpu, cwa, n, shape):
     assert np.array_equal(g["count"], np.bincount(g["key"], minlength=g["count"].size))
 
 
+@pytest.mark.parametrize("which", ["pos", "vel"])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_force_of_a_particle_that_left_the_numbers(gpu, cwa, which, value):
+    """A particle without neighbours adds nothing, whatever its own record holds and
+    however many neighbours the particle has that shares its loads: one lane per
+    particle gives the finite numbers that four lanes give."""
+    from coupledwateranimation_amd import configs
+
+    print(f"force {which} {value}", flush=True)
+    spec = configs.dam_break_diff(2048, 96, 7)
+    n = 2000
+    rng = np.random.default_rng(3)
+    pos, vel = spec.pos[:n].copy(), np.zeros((n, 4), np.float32)
+    vel[:, :3] = rng.normal(0.0, 0.3, (n, 3))
+    odd = rng.permutation(n)[:40]
+    if which == "vel":  # apart from the others, each alone
+        pos[odd, :3] = 0.35 + 0.6 * rng.random((40, 3))
+        pos[odd, 1] = 0.02 * np.arange(40) + 0.1
+    (pos if which == "pos" else vel)[odd, rng.integers(0, 3, 40)] = value
+    (a, _), (b, _) = [_scene_state(cwa, spec, pos, vel, None, k, 1) for k in (-1, 0)]
+    for k in ("force", "vel", "pos"):
+        assert np.array_equal(np.isfinite(a[k]), np.isfinite(b[k])), k
+        both = np.isfinite(a[k])
+        assert np.abs(a[k] - b[k])[both].max() <= 512 * 2.0 ** -24 * np.abs(b[k][both]).max(), k
+
+
 @pytest.mark.parametrize("shape", ["1", "20", "21", "32", "33", "64", "65", "300", "columns",
                                    "lattice", "far"])
 def test_density_by_packed_points(gpu, cwa, oracle, shape):
