@@ -104,7 +104,7 @@ KERNEL_KEYS = [
     ("cwa::b2d::k2_wave(", "batched", "wave"),
     ("cwa::k_density(", "plain", "density"), ("cwa::k_force_integrate<", "plain", "force_integrate"),
     ("cwa::k_hash_count<", "plain", "hash"), ("cwa::k_link_runs(", "plain", "scatter"),
-    ("cwa::k_stable_reorder(", "plain", "reorder"), ("cwa::k_wave4(", "plain", "wave"),
+    ("cwa::k_stable_reorder<", "plain", "reorder"), ("cwa::k_wave4(", "plain", "wave"),
 ]
 
 

@@ -176,8 +176,9 @@ __device__ __forceinline__ void pack_test(uint32_t a, uint32_t b, int bias, uint
 // |y - py| < sqrt(h^2 - d^2) with d the horizontal distance to the
 // footprint; both bounds are widened by grid_eps (well above the rounding
 // of the float bounds), so every neighbour stays inside and the exact
-// per-candidate test decides.  Density, force and the adjoint call this with
-// the same positions, so their candidate ranges (and mask bits) agree.
+// per-candidate test decides.  The four-lane density pass and the re-search of
+// a particle without words go by it.  k_density takes the rows within h of the
+// particle in every column: other ranges, the same neighbours in the same order.
 __device__ __forceinline__ void column_range(const DevParams& P, const int* __restrict__ offset,
                                              float px, float py, float pz, int ix, int iz, int c,
                                              int& b, int& e) {
@@ -207,8 +208,10 @@ __device__ __forceinline__ void column_range(const DevParams& P, const int* __re
 // density pass, for the passes that visit it again (force, adjoint).  For
 // each candidate column in order, each 32-candidate chunk of the column that
 // holds a neighbour of particle i (other than i itself) gives one word
-// (bits, base): bit k set when slot base + k is a neighbour.  The words of
-// particle i are packed, in candidate order:
+// (bits, base): bit k set when slot base + k is a neighbour.  Chunks start where
+// the pass's range of the column does, so words of the two density passes may
+// differ, while the neighbours and their order do not.  The words of particle
+// i are packed, in candidate order:
 //   nbw[k*n + i]                 word k, k < count
 //   nb_count(nbw, n)[i]          count, or -1: the particle has more words
 //                                than kNbEntries (in the four-lane density

@@ -402,8 +402,10 @@ hipError_t launch_scan(const int* in, int* out, int n, int* ws, hipStream_t st,
 //            its own; the lanes of the run take that rank plus their
 //            distance to the head.  The particle positions and ids move to
 //            their sorted slots in the same pass.
-// The wave layout (blocks of 256 over the same item range) is identical in
-// both item passes, so both see the same runs.  The lists need no offsets, so
+// The rank is right because a listed run that starts before a run's head also
+// ends before it.  Runs end where the key changes and at the ends of the listing
+// wave's items: 64, in step with the reorder's waves, or the 16 of k_force_split,
+// whose finer runs still end with the reorder's.  The lists need no offsets, so
 // whoever counts the keys can also list the runs; builds of up to
 // kFuseLinksMax particles do.  In larger ones k_link_runs lists them, and in large
 // builds outside a scene k_place_runs puts them side by side in their cell's
@@ -793,8 +795,8 @@ __global__ void __launch_bounds__(256) k_density(
 // consecutive lanes per particle, each testing every kDensitySplit-th
 // candidate of each column, so a scene of some ten thousand particles still
 // keeps several waves per SIMD busy.  The group's neighbour bits are OR-ed
-// together (the words equal k_density's), its partial sums added in a fixed
-// tree, and the group's first lane finishes the particle.
+// together (k_density's neighbours, in its order), its partial sums added in a
+// fixed tree, and the group's first lane finishes the particle.
 //
 // At these sizes the pass is one dependent chain per wave, not throughput: nine
 // columns, each an offset load, then candidate loads a few at a time.  So the

@@ -200,13 +200,14 @@ const char* cwa_kernel_name(int k);
 
 /* Lanes per particle (no reference counterpart: a tuning knob of this
  * implementation, also used by tests to reach both kernel forms on small
- * scenes).  Scenes of up to max_n particles run the density pass with four
- * lanes per particle and the pair adjoint of a tape created afterwards with
- * four; larger scenes one lane each.  Default 262144 (2^18); max_n < 0
- * restores it.  Process-wide; taken at each density launch (a step graph
- * keeps the form it was captured with) and at tape creation.  *previous
- * (optional) receives the limit before the call.  Both forms find the same
- * neighbour words; the density sums differ in summation order only. */
+ * scenes).  Scenes of up to max_n particles run the density pass and the pair
+ * adjoint of a tape created afterwards with four lanes per particle, those of
+ * up to the smaller of max_n and 32768 the force pass too; larger scenes one
+ * lane each.  Default 262144 (2^18); max_n < 0 restores it.  Process-wide;
+ * taken at each step (a step graph keeps the form it was captured with) and at
+ * tape creation.  *previous (optional) receives the limit before the call.
+ * Both forms visit the same neighbours in the same order; the density and
+ * force sums differ in summation order only. */
 int cwa_set_lane_split_limit(long long max_n, long long* previous);
 
 /* Reference defaults (Main.cpp:184-204 and the shader #defines) for a grid

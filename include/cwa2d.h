@@ -88,11 +88,14 @@ typedef struct cwa2d_scene {
 typedef struct cwa2d_tuning {
     int32_t block_density; /* threads per block = particles per tile: 64..1024  */
     int32_t block_force;
-    int32_t grid_density;  /* persistent blocks; 0: one block per tile          */
+    int32_t grid_density;  /* persistent blocks; 0 (or no fewer than tiles): one
+                              block per tile, in batches of up to 80000 particles
+                              four, with four lanes per particle                */
     int32_t grid_force;
     int32_t xcd_queues;    /* 1: scenes bound to XCD-local tile queues (with
                               stealing); 0: one global queue                    */
-    int32_t wave_block;    /* threads per scene in the wave pass: 64..1024      */
+    int32_t wave_block;    /* threads per scene in the wave pass: 64..1024
+                              (1024 until set)                                  */
     float ms_per_step;     /* tuner: measured time of this setting              */
 } cwa2d_tuning;
 
@@ -156,8 +159,10 @@ int cwa2d_batch_get_params(cwa2d_batch* b, cwa2d_params* p);
 /* `steps` coupled steps of SPH time step dt (each: sph_substeps SPH
  * substeps, then every scene's wave_substeps wave substeps). */
 int cwa2d_batch_step(cwa2d_batch* b, float dt, int32_t steps);
-/* The same, replayed from a hipGraph of one step (captured on first use
- * and after any change of dt, parameters or tuning). */
+/* The same, replayed from hipGraphs of up to eight steps (fewer where a step
+ * has many substeps).  A call captures the graphs it needs that no call
+ * before it has, all of them before the first one runs; a change of dt,
+ * parameters or tuning drops them. */
 int cwa2d_batch_step_graph(cwa2d_batch* b, float dt, int32_t steps);
 /* One step with a HIP event pair around every kernel. */
 int cwa2d_batch_step_profiled(cwa2d_batch* b, float dt, cwa2d_kernel_times* t);
