@@ -106,9 +106,10 @@ def test_fit_graph_reads_updated_parameters(gpu, cwa):
         sc.close()
 
 
-@pytest.mark.parametrize("cells,wave,factors", [
-    (20, 64, (0.25, 1.0, 2.0)), (20, 61, (0.3,)), (100, 512, (1 / 16, 1 / 64, 1 / 1024))])
-def test_fit_graph_follows_the_wave_scale(gpu, cwa, cells, wave, factors):
+@pytest.mark.parametrize("n,cells,wave,factors", [
+    (3000, 20, 64, (0.25, 1.0, 2.0)), (3000, 20, 61, (0.3,)),
+    (3000, 100, 512, (1 / 16, 1 / 64, 1 / 1024)), (33_000, 100, 512, (1 / 16,))])
+def test_fit_graph_follows_the_wave_scale(gpu, cwa, n, cells, wave, factors):
     """The heightfield spread over more of the grid, or less, than when the fit
     was captured: a tile's texels then sample more columns than the tile was
     chosen for (at 0.25 all 20 x 20, with 100 x 100 more than one tile can hold)."""
@@ -116,7 +117,7 @@ def test_fit_graph_follows_the_wave_scale(gpu, cwa, cells, wave, factors):
     from coupledwateranimation_amd.fit import FitBatch
     from coupledwateranimation_amd.scene import Scene
 
-    spec = configs.dam_break_diff(3000, wave, 9)
+    spec = configs.dam_break_diff(n, wave, 9)
     p = spec.params
     p.mass *= (1.0 / cells / p.h) ** 3
     p.h = 1.0 / cells
@@ -127,7 +128,7 @@ def test_fit_graph_follows_the_wave_scale(gpu, cwa, cells, wave, factors):
     with Scene(p, spec.pos, spec.vel, None, spec.wave_size, spec.height0, spec.height1) as sc:
         fb = FitBatch([sc], [target], steps, 3, spec.dt)
         for f in factors:
-            _say(f"wave scale {cells} cells {wave}^2 x {f}")
+            _say(f"wave scale n={n} {cells} cells {wave}^2 x {f}")
             q = p.copy()
             q.wave_uv_scale[:] = [f * v for v in p.wave_uv_scale]
             sc.set_params(q)
